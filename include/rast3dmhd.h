@@ -189,8 +189,9 @@ int mhd_flux_profiles(mhd_t *h, double *ttm, double *rom, double *fconm, double 
 /* Measurement hook (no counterpart in the reference): runs n steps like
  * mhd_steps with HIP events around every launch on the handle's stream and
  * returns the mean duration in milliseconds of one step, one RK stage
- * kernel launch (averaged over the three stages), one CFL reduction and one
- * boundary-plane launch.  Any output pointer may be NULL. */
+ * kernel launch (averaged over the three stages) and one CFL reduction.
+ * ms_bcon is 0: the boundary planes are part of the stage launches.  Any
+ * output pointer may be NULL. */
 int mhd_time_steps(mhd_t *h, int n, double *ms_step, double *ms_stage, double *ms_cfl,
                    double *ms_bcon);
 

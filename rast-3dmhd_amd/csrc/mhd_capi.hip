@@ -52,6 +52,7 @@ struct mhd_ctx {
     Metrics m{};
     std::vector<double> dzzdz, d2zzdz2, ddz, rkapa, dkapa;  // host copies for the background
     DevScalars *sc = nullptr;
+    CflSlots *cs = nullptr;             // CFL reduction slots
     // closure-corrected step (mixed form)
     mhd_net_t *net = nullptr;
     float *force = nullptr;    // [7][fsize]
@@ -111,9 +112,9 @@ static void free_all(mhd_t *h) {
     if (!h) return;
     (void)hipSetDevice(h->dev);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
-    void *bufs[25] = {h->q[0], h->q[1], h->z, h->hq[0], h->hq[1], h->dr, h->rr, h->bgd, h->bgf, h->bgp,
+    void *bufs[26] = {h->q[0], h->q[1], h->z, h->hq[0], h->hq[1], h->dr, h->rr, h->bgd, h->bgf, h->bgp,
                       h->f, h->stage, h->met, h->sc, h->force, h->force_on, h->cx, h->nrm,
-                      h->optmem, h->rs, h->ftacc, h->bgd2, h->bgf2, h->bgp2, h->prof};
+                      h->optmem, h->rs, h->ftacc, h->bgd2, h->bgf2, h->bgp2, h->prof, h->cs};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -200,6 +201,7 @@ extern "C" int mhd_create(const mhd_desc *d, mhd_t **out) {
     if (e == hipSuccess) e = hipMalloc(&h->stage, pbytes);
     if (e == hipSuccess) e = hipMalloc(&h->met, sizeof(double) * (3 * (d->npx + 2) + 3 * (d->npy + 2) + 5 * (d->npz + 2)));
     if (e == hipSuccess) e = hipMalloc(&h->sc, sizeof(DevScalars));
+    if (e == hipSuccess) e = hipMalloc(&h->cs, sizeof(CflSlots));
     if (e != hipSuccess) {
         rc = fail(nullptr, MHD_ERR_HIP, "mhd_create: device allocation failed: %s", hipGetErrorString(e));
         free_all(h);
@@ -215,6 +217,7 @@ extern "C" int mhd_create(const mhd_desc *d, mhd_t **out) {
     }
     const DevScalars s0 = initial_scalars();
     e = hipMemcpy(h->sc, &s0, sizeof(s0), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = launch_cfl_arm(h->cs, 1, h->stream);
     if (e != hipSuccess) {
         rc = fail(nullptr, MHD_ERR_HIP, "mhd_create: %s", hipGetErrorString(e));
         free_all(h);
@@ -465,11 +468,14 @@ extern "C" int mhd_download(mhd_t *h, double *ru, double *rv, double *rw, double
     return MHD_OK;
 }
 
-// The launches of one STEP, optionally bracketed by events (ev[0..13]:
-// CFL, then stage/BCON pairs of the three stages).  The CFL limits of the
-// state a step starts from are reduced by the previous step's stage-3 and
-// boundary kernels; only the first step after an upload runs the
-// stand-alone reduction.
+// Events of one STEP: CFL (and closure), then the three stages.
+constexpr int STEP_EVENTS = 8;
+
+// The launches of one STEP, optionally bracketed by events (ev[0..7]: pairs
+// around CFL and the three stages).  The stage launches apply the boundary
+// conditions, and the third closes the step: the CFL limits of the state a
+// step starts from are reduced by the previous step's third stage.  Only the
+// first step after an upload runs the stand-alone reduction.
 static hipError_t launches(mhd_t *h, hipEvent_t *ev) {
     const Params &p = h->p;
     hipError_t e = time_factors(h);
@@ -477,10 +483,9 @@ static hipError_t launches(mhd_t *h, hipEvent_t *ev) {
         if (ev && e == hipSuccess) e = hipEventRecord(ev[i], h->stream);
     };
     rec(0);
-    if (!h->cfl_valid) {
-        if (!h->mixed) e = launch_cfl(p, h->m, h->q[h->cur], h->sc, h->stream);
-        else e = launch_cfl_mixed(p, h->m, h->bg, h->hq[h->cur], h->rr, h->sc, h->stream);
-        if (e == hipSuccess) e = launch_cfl_final(p, h->sc, false, h->stream);
+    if (!h->cfl_valid && e == hipSuccess) {
+        if (!h->mixed) e = launch_cfl(p, h->m, h->q[h->cur], h->sc, h->cs, h->stream);
+        else e = launch_cfl_mixed(p, h->m, h->bg, h->hq[h->cur], h->rr, h->sc, h->cs, h->stream);
     }
     if (e == hipSuccess && h->closure) {
         // subgrid forcing from the network on the state at the start of the step
@@ -492,23 +497,16 @@ static hipError_t launches(mhd_t *h, hipEvent_t *ev) {
     rec(1);
     int a = h->cur, b = 1 - h->cur;
     for (int st = 1; st <= 3 && e == hipSuccess; ++st) {
-        rec(2 + 4 * (st - 1));
+        rec(2 * st);
         if (h->means) e = launch_opt_means(p, h->m, h->q[a], h->ob, h->sc, h->stream);
         if (e != hipSuccess) break;
-        if (!h->mixed) e = launch_stage(st, p, h->m, h->q[a], h->q[b], h->z, nullptr, h->sc, h->stream);
-        else e = launch_stage_mixed(st, p, h->m, h->bg, h->hq[a], h->hq[b], h->dr, h->rr, h->sc, h->stream);
-        rec(3 + 4 * (st - 1));
-        rec(4 + 4 * (st - 1));
-        if (e == hipSuccess) {
-            if (!h->mixed) e = launch_bcon(p, h->m, h->q[a], h->q[b], h->sc, st == 3, h->stream);
-            else e = launch_bcon_mixed(p, h->m, h->bg, h->hq[b], h->dr, h->rr, h->sc, st == 3, h->stream);
-        }
-        rec(5 + 4 * (st - 1));
+        if (!h->mixed) e = launch_stage(st, p, h->m, h->q[a], h->q[b], h->z, nullptr, h->sc, h->cs, h->stream);
+        else e = launch_stage_mixed(st, p, h->m, h->bg, h->hq[a], h->hq[b], h->dr, h->rr, h->sc, h->cs, h->stream);
+        rec(2 * st + 1);
         const int t = a;
         a = b;
         b = t;
     }
-    if (e == hipSuccess) e = launch_cfl_final(p, h->sc, true, h->stream);
     if (e == hipSuccess) {
         h->cur = 1 - h->cur;
         h->cfl_valid = true;
@@ -543,7 +541,7 @@ static hipError_t rhs_eval(mhd_t *h) {
     if (!h->f) e = hipMalloc(&h->f, (size_t)h->p.fsize * sizeof(double) * nfields(h));
     if (e == hipSuccess) e = time_factors(h);
     if (e == hipSuccess && h->means) e = launch_opt_means(h->p, h->m, h->q[h->cur], h->ob, h->sc, h->stream);
-    if (e == hipSuccess) e = launch_stage(0, h->p, h->m, h->q[h->cur], nullptr, nullptr, h->f, h->sc, h->stream);
+    if (e == hipSuccess) e = launch_stage(0, h->p, h->m, h->q[h->cur], nullptr, nullptr, h->f, h->sc, h->cs, h->stream);
     return e;
 }
 
@@ -585,7 +583,7 @@ extern "C" int mhd_time_steps(mhd_t *h, int n, double *ms_step, double *ms_stage
     if (rc) return rc;
     if (n < 1) return fail(h, MHD_ERR_ARG, "mhd_time_steps: n=%d", n);
     HIPCHK(h, hipSetDevice(h->dev));
-    constexpr int PER = 14;
+    constexpr int PER = STEP_EVENTS;
     std::vector<hipEvent_t> ev((size_t)PER * n + 2);
     size_t made = 0;
     hipError_t e = hipSuccess;
@@ -598,18 +596,16 @@ extern "C" int mhd_time_steps(mhd_t *h, int n, double *ms_step, double *ms_stage
     for (int s = 0; s < n && e == hipSuccess; ++s) e = launches(h, &ev[2 + (size_t)PER * s]);
     if (e == hipSuccess) e = hipEventRecord(ev[1], h->stream);
     if (e == hipSuccess) e = hipEventSynchronize(ev[1]);
-    double tstage = 0, tcfl = 0, tbcon = 0;
+    double tstage = 0, tcfl = 0;
     float ms = 0, total = 0;
     if (e == hipSuccess) {
         for (int s = 0; s < n; ++s) {
             hipEvent_t *x = &ev[2 + (size_t)PER * s];
             (void)hipEventElapsedTime(&ms, x[0], x[1]);
             tcfl += ms;
-            for (int st = 0; st < 3; ++st) {
-                (void)hipEventElapsedTime(&ms, x[2 + 4 * st], x[3 + 4 * st]);
+            for (int st = 1; st <= 3; ++st) {
+                (void)hipEventElapsedTime(&ms, x[2 * st], x[2 * st + 1]);
                 tstage += ms;
-                (void)hipEventElapsedTime(&ms, x[4 + 4 * st], x[5 + 4 * st]);
-                tbcon += ms;
             }
         }
         (void)hipEventElapsedTime(&total, ev[0], ev[1]);
@@ -619,7 +615,7 @@ extern "C" int mhd_time_steps(mhd_t *h, int n, double *ms_step, double *ms_stage
     if (ms_step) *ms_step = total / n;
     if (ms_stage) *ms_stage = tstage / (3.0 * n);
     if (ms_cfl) *ms_cfl = tcfl / n;
-    if (ms_bcon) *ms_bcon = tbcon / (3.0 * n);
+    if (ms_bcon) *ms_bcon = 0.0;  // no launch of its own: part of the stages
     return finish(h, nullptr, nullptr);
 }
 

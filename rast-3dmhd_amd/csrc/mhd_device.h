@@ -19,6 +19,25 @@ __device__ __forceinline__ int xcd_remap(int bid, int nb) {
     const int q = nb >> 3, r = nb & 7;
     return x * q + (x < r ? x : r) + local;
 }
+// Tile and z chunk of workgroup bid of a stage launch over ntiles tiles and
+// nch chunks.  Where the tiles divide by the 8 XCDs, each XCD gets a
+// contiguous run of tiles in every chunk, chunk after chunk: tiles that share
+// halo rows share an L2, and the chunks with the boundary planes, which do
+// more work, are spread over all XCDs (as one contiguous run over all chunks,
+// the two boundary chunks of 512x512x256 fell to two XCDs: FP64 stage 2 took
+// 3.67 ms).  Other counts take the contiguous run.
+struct TileChunk {
+    int tile, chunk;
+};
+__device__ __forceinline__ TileChunk tile_of(int bid, int ntiles, int nch) {
+    if (ntiles % 8 == 0) {
+        const int per = ntiles / 8, local = bid >> 3;
+        const int c = local / per;
+        return TileChunk{(bid & 7) * per + local - c * per, c};
+    }
+    const int id = xcd_remap(bid, ntiles * nch);
+    return TileChunk{id % ntiles, id / ntiles};
+}
 
 // Entry i of a read-only per-plane table (grid metrics, background
 // profiles) at a workgroup-uniform index: read through the constant
@@ -49,6 +68,116 @@ __device__ __forceinline__ X after(X x, Y y) {
 template <class X>
 __device__ __forceinline__ void settle(X x) {
     asm volatile("" ::"v"(x));
+}
+
+// A box's arguments for the code after a march (boundary conditions, CFL
+// reduction), read anew from memory: the empty asm hides where the pointer
+// comes from, so that the values are not loaded before the march and held in
+// scalar registers through it (which spilled 50-60 more of them).
+typedef const __attribute__((address_space(4))) BoxArgs *ArgPtr;
+__device__ __forceinline__ const BoxArgs &late_args(ArgPtr a) {
+    asm volatile("" : "+s"(a));
+    return *(const BoxArgs *)a;
+}
+// Entry b of the ensemble's box table, read through the constant address
+// space (it is written by host copies between launches only): its members
+// arrive by scalar loads also after the stores of an earlier work item.
+__device__ __forceinline__ const BoxDev &box_at(const BoxDev *boxes, int b) {
+    return *(const BoxDev *)((const __attribute__((address_space(4))) BoxDev *)boxes + b);
+}
+// The kernel's first argument in the kernel-argument segment.
+__device__ __forceinline__ ArgPtr kernel_args() { return (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr(); }
+
+// Value of key slot n between reductions (the neutral element of its min).
+__host__ __device__ inline unsigned long long cfl_key_init(int n) { return n == 0 ? ~dkey(0.0) : dkey(INFINITY); }
+
+__device__ __forceinline__ void cfl_arm(CflSlots *cs, int lane) {
+    const int n = lane / CFL_REP, r = lane % CFL_REP;
+    unsigned long long *const w = n < CFL_KEYS ? &cs->key[n][r].v : n == CFL_KEYS ? &cs->count[r].v : &cs->done.v;
+    if (lane <= (CFL_KEYS + 1) * CFL_REP)
+        __hip_atomic_store(w, n < CFL_KEYS ? cfl_key_init(n) : 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// End of a reduction: DT = SF*MIN(...), UMACH = SQRT(MAX(...)) (sub:761,
+// 868-872).  A positive fixed_dt replaces the CFL DT.  With clock set this
+// also closes the step that just ran: NIT, TIMC, TIMT (sub:1171-1173) with
+// the DT it used, which is kept as dt_used / umach_used.
+__device__ __forceinline__ void cfl_final(DevScalars *sc, const unsigned long long *k, double sf, int lmag, int clock) {
+    if (clock) {
+        sc->nit = sc->nit + 1;
+        sc->timc = sc->timc + sc->dt;
+        sc->timt = sc->timi + sc->timc;
+        sc->dt_used = sc->dt;
+        sc->umach_used = sc->umach;
+    }
+    const double mach = dunkey(~k[0]);
+    double mn = INFINITY;
+    bool bad = !(mach == mach);
+    for (int n = 0; n < 4; ++n) {
+        const double w = dunkey(k[n + 1]);
+        sc->cflmin[n] = w;
+        if (n < 3 || lmag) {
+            mn = fmin(mn, w);
+            bad = bad || !(w == w);
+        }
+    }
+    sc->umach = sqrt(mach);
+    const double dcfl = sf * mn;
+    sc->dt = sc->fixed_dt > 0.0 ? sc->fixed_dt : dcfl;
+    if (bad || dcfl == INFINITY) sc->nonfinite |= 1;
+}
+
+// A workgroup's part of a CFL reduction, called by its first wavefront (all
+// 64 lanes); k[0..4] of lane 0 are its keys (the complement of the Mach key,
+// then the four limits).  Workgroup seq of total adds them to copy seq %
+// CFL_REP of the slots and counts itself in; the last of the copy counts the
+// copy in, and the last copy's workgroup combines the copies, re-arms the
+// slots and closes the reduction, so that no launch of its own is needed
+// (a one-thread launch takes 4.8 us in a step that may be 50 us long).
+// Atomics and key reads are at device scope (coherent across the XCDs' L2s).
+// The counter is raised after this wavefront's key updates have returned,
+// so the last workgroup reads every key complete.  Until it is re-armed a
+// key only falls: a workgroup whose value cannot move it skips the atomic,
+// and a stale read there can only cost one that was not needed.
+__device__ __forceinline__ void cfl_publish(const unsigned long long *k, DevScalars *sc, CflSlots *cs, double sf,
+                                            int lmag, int clock, int seq, int total) {
+    const int lane = threadIdx.x & 63, rep = seq % CFL_REP;
+    unsigned long long v = 0;
+#pragma unroll
+    for (int n = 0; n < CFL_KEYS; ++n) {
+        const unsigned long long x = __shfl(k[n], 0, 64);
+        if (lane == n) v = x;
+    }
+    unsigned long long old = 0;
+    if (lane < (lmag ? CFL_KEYS : CFL_KEYS - 1)) {
+        unsigned long long *const w = &cs->key[lane][rep].v;
+        if (v < __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            old = __hip_atomic_fetch_min(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    // the key updates have been performed: their results are here
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(old)::"memory");
+    int last = 0;
+    if (lane == 0) {
+        const unsigned long long in_copy = (unsigned long long)((total - rep + CFL_REP - 1) / CFL_REP);
+        const unsigned long long copies = total < CFL_REP ? total : CFL_REP;
+        if (__hip_atomic_fetch_add(&cs->count[rep].v, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == in_copy)
+            last = __hip_atomic_fetch_add(&cs->done.v, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == copies;
+    }
+    if (!__shfl(last, 0, 64)) return;
+    asm volatile("" ::: "memory");
+    unsigned long long x = ~0ull;
+    if (lane < CFL_KEYS * CFL_REP)
+        x = __hip_atomic_load(&cs->key[lane / CFL_REP][lane % CFL_REP].v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int off = CFL_REP / 2; off > 0; off >>= 1) {
+        const unsigned long long y = __shfl_xor(x, off, 64);
+        x = y < x ? y : x;
+    }
+    unsigned long long kk[CFL_KEYS];
+#pragma unroll
+    for (int n = 0; n < CFL_KEYS; ++n) kk[n] = __shfl(x, n * CFL_REP, 64);
+    cfl_arm(cs, lane);
+    if (lane == 0) cfl_final(sc, kk, sf, lmag, clock);
 }
 
 // Stored values of the mixed form (mhd_mixed.hip) as other kernels read them.

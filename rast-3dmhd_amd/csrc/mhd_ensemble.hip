@@ -4,13 +4,13 @@
 // ping-pong, or FP32 h ping-pong) and the third register (FP64 Z, or FP32
 // D), then the metric blocks, the mixed form's background blocks and one
 // DevScalars per box.  The device table of BoxDev entries points every
-// batched kernel at its box.  A step is: 3 x (persistent stage launch over
-// the StageItem table of all boxes, boundary-plane launch over the
-// ColumnItem table), then one per-box DT/clock update.  Steps are replayed
-// from captured HIP graphs (one graph per register parity for a pair of
-// steps and for a single step); the launches carry no host-side state that
-// changes between steps (DT lives in device memory), so a replay is the
-// same work as direct launches.
+// batched kernel at its box.  A step is three stage launches over the
+// StageItem table of all boxes: the items that hold a boundary plane apply
+// the boundary conditions, and the last item of a box in the third launch
+// updates the box's DT and clock.  Steps are replayed from captured HIP
+// graphs (one graph per register parity for a pair of steps and for a single
+// step); the launches carry no host-side state that changes between steps (DT
+// lives in device memory), so a replay is the same work as direct launches.
 
 #include <hip/hip_runtime.h>
 
@@ -56,14 +56,13 @@ struct mhd_ens {
     float *bgf = nullptr;            // mixed: FP32 background blocks
     PlaneM *bgp = nullptr;           // mixed: per-plane records of the stage kernel, per box
     DevScalars *sc = nullptr;
+    CflSlots *cs = nullptr;          // CFL reduction slots per box
     double *stage = nullptr;         // one padded field of the largest box
     size_t stage_bytes = 0;
     // tiling
     int tile_x = 64, tile_y = 4, kdepth = 16, grid = 0;
     StageItem *ditems = nullptr;
     int nitems = 0;
-    ColumnItem *dcols = nullptr;
-    int ncols = 0;
     // graphs [single=0 / pair=1][register parity]
     hipGraphExec_t gexec[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
     int cur = 0;
@@ -102,7 +101,7 @@ static void free_ens(mhd_ens_t *e) {
     (void)hipSetDevice(e->dev);
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     drop_graphs(e);
-    void *bufs[10] = {e->dbox, e->pool, e->met, e->bgd, e->bgf, e->bgp, e->sc, e->stage, e->ditems, e->dcols};
+    void *bufs[10] = {e->dbox, e->pool, e->met, e->bgd, e->bgf, e->bgp, e->sc, e->cs, e->stage, e->ditems};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (e->stream) (void)hipStreamDestroy(e->stream);
@@ -114,39 +113,37 @@ static int check_box(mhd_ens_t *e, int b, const char *who) {
     return MHD_OK;
 }
 
-// Work tables for the current tiling: StageItems (tile_x x tile_y tiles)
-// box-major (z chunk, row, x tile), ColumnItems 256 columns each.
+// Work table for the current tiling: StageItems (tile_x x tile_y tiles)
+// box-major (z chunk, row, x tile).  A box's planes are split evenly into
+// chunks of at most kdepth planes, and at least three (chunk_begin).
 static int build_tables(mhd_ens_t *e) {
     std::vector<StageItem> items;
-    std::vector<ColumnItem> cols;
     for (int b = 0; b < e->nbox; ++b) {
         const Params &p = e->box[b].p;
-        const int kd = e->kdepth > 0 ? e->kdepth : p.npz;
+        int nc = e->kdepth > 0 ? (p.npz + e->kdepth - 1) / e->kdepth : 1;
+        if (nc > max_chunks(p.npz)) nc = max_chunks(p.npz);
         const int ntx = (p.npx + e->tile_x - 1) / e->tile_x, nty = (p.npy + e->tile_y - 1) / e->tile_y;
-        for (int k0 = 1; k0 <= p.npz; k0 += kd)
+        int seq = 0;
+        for (int c = 0; c < nc; ++c)
             for (int ty = 0; ty < nty; ++ty)
                 for (int tx = 0; tx < ntx; ++tx) {
                     StageItem it;
                     it.box = b;
                     it.i0 = tx * e->tile_x;
                     it.j0 = ty * e->tile_y;
-                    it.kbeg = k0;
-                    it.kend = k0 + kd - 1 < p.npz ? k0 + kd - 1 : p.npz;
+                    it.kbeg = chunk_begin(p.npz, nc, c);
+                    it.kend = chunk_begin(p.npz, nc, c + 1) - 1;
+                    it.seq = seq++;
+                    it.total = nc * ntx * nty;
                     items.push_back(it);
                 }
-        for (long long c = 0; c < p.plane; c += 256) cols.push_back(ColumnItem{b, (int)c});
     }
     drop_graphs(e);
     if (e->ditems) EHIP(e, hipFree(e->ditems));
-    if (e->dcols) EHIP(e, hipFree(e->dcols));
     e->ditems = nullptr;
-    e->dcols = nullptr;
     EHIP(e, hipMalloc(&e->ditems, items.size() * sizeof(StageItem)));
-    EHIP(e, hipMalloc(&e->dcols, cols.size() * sizeof(ColumnItem)));
     EHIP(e, hipMemcpy(e->ditems, items.data(), items.size() * sizeof(StageItem), hipMemcpyHostToDevice));
-    EHIP(e, hipMemcpy(e->dcols, cols.data(), cols.size() * sizeof(ColumnItem), hipMemcpyHostToDevice));
     e->nitems = (int)items.size();
-    e->ncols = (int)cols.size();
     return MHD_OK;
 }
 
@@ -196,6 +193,7 @@ extern "C" int mhd_ens_create(const mhd_desc *descs, int nbox, mhd_ens_t **out) 
     if (r == hipSuccess && e->mixed) r = hipMalloc(&e->bgf, BG_FLT * nzsum * sizeof(float));
     if (r == hipSuccess && e->mixed) r = hipMalloc(&e->bgp, nzsum * sizeof(PlaneM));
     if (r == hipSuccess) r = hipMalloc(&e->sc, nbox * sizeof(DevScalars));
+    if (r == hipSuccess) r = hipMalloc(&e->cs, nbox * sizeof(CflSlots));
     if (r == hipSuccess) r = hipMalloc(&e->stage, e->stage_bytes);
     if (r == hipSuccess) r = hipMalloc(&e->dbox, nbox * sizeof(BoxDev));
     if (r != hipSuccess) {
@@ -208,9 +206,9 @@ extern "C" int mhd_ens_create(const mhd_desc *descs, int nbox, mhd_ens_t **out) 
     for (int b = 0; b < nbox; ++b) {
         EnsBox &B = e->box[b];
         BoxDev &D = e->hbox[b];
-        D.p = B.p;
+        D.a.p = B.p;
         size_t len[11];
-        D.m = metric_table(B.p, e->met + met_off[b], len);
+        D.a.m = metric_table(B.p, e->met + met_off[b], len);
         char *base = e->pool + reg_off[b];
         const size_t rb = align_up(B.reg_elems * esz);
         if (e->mixed) {
@@ -220,16 +218,18 @@ extern "C" int mhd_ens_create(const mhd_desc *descs, int nbox, mhd_ens_t **out) 
             D.rr = reinterpret_cast<unsigned *>(base + 3 * rb);
             const size_t o = bg_off[b];
             // BG_DBL FP64 and BG_FLT FP32 tables of npz+2 entries, laid out per box
-            D.bg = background_view(B.p.npz, e->bgd + BG_DBL * o, e->bgf + BG_FLT * o);
-            D.bg.planes = e->bgp + o;
+            D.a.bg = background_view(B.p.npz, e->bgd + BG_DBL * o, e->bgf + BG_FLT * o);
+            D.a.bg.planes = e->bgp + o;
         } else {
             D.q[0] = reinterpret_cast<double *>(base);
             D.q[1] = reinterpret_cast<double *>(base + rb);
             D.z = reinterpret_cast<double *>(base + 2 * rb);
         }
         D.sc = e->sc + b;
+        D.cs = e->cs + b;
     }
     r = hipMemcpy(e->sc, s0.data(), nbox * sizeof(DevScalars), hipMemcpyHostToDevice);
+    if (r == hipSuccess) r = launch_cfl_arm(e->cs, nbox, e->stream);
     if (r == hipSuccess) r = hipMemcpy(e->dbox, e->hbox.data(), nbox * sizeof(BoxDev), hipMemcpyHostToDevice);
     int rc = r == hipSuccess ? MHD_OK : efail(nullptr, MHD_ERR_HIP, "mhd_ens_create: %s", hipGetErrorString(r));
     if (!rc) {
@@ -255,9 +255,9 @@ extern "C" int mhd_ens_set_metrics(mhd_ens_t *e, int b, const double *dxxdx, con
     const double *src[11] = {dxxdx, d2xxdx2, ddx, dyydy, d2yydy2, ddy, dzzdz, d2zzdz2, ddz, rkapa, dkapa};
     size_t len[11];
     metric_lengths(B.p, len);
-    const double *dst[11] = {e->hbox[b].m.dxxdx, e->hbox[b].m.d2xxdx2, e->hbox[b].m.ddx, e->hbox[b].m.dyydy,
-                             e->hbox[b].m.d2yydy2, e->hbox[b].m.ddy, e->hbox[b].m.dzzdz, e->hbox[b].m.d2zzdz2,
-                             e->hbox[b].m.ddz, e->hbox[b].m.rkapa, e->hbox[b].m.dkapa};
+    const double *dst[11] = {e->hbox[b].a.m.dxxdx, e->hbox[b].a.m.d2xxdx2, e->hbox[b].a.m.ddx, e->hbox[b].a.m.dyydy,
+                             e->hbox[b].a.m.d2yydy2, e->hbox[b].a.m.ddy, e->hbox[b].a.m.dzzdz, e->hbox[b].a.m.d2zzdz2,
+                             e->hbox[b].a.m.ddz, e->hbox[b].a.m.rkapa, e->hbox[b].a.m.dkapa};
     EHIP(e, hipSetDevice(e->dev));
     for (int n = 0; n < 11; ++n) {
         if (!src[n]) return efail(e, MHD_ERR_ARG, "mhd_ens_set_metrics: array %d is null", n);
@@ -293,11 +293,11 @@ extern "C" int mhd_ens_set_background(mhd_ens_t *e, int b, const double *ro0, co
                                       B.dkapa.data(), ro0, tt0, d, f, pl);
     if (bad >= 0) return efail(e, MHD_ERR_ARG, "mhd_ens_set_background: box %d: rho0[%d] <= 0", b, bad);
     EHIP(e, hipSetDevice(e->dev));
-    EHIP(e, hipMemcpyAsync(const_cast<double *>(e->hbox[b].bg.ro), d.data(), d.size() * sizeof(double),
+    EHIP(e, hipMemcpyAsync(const_cast<double *>(e->hbox[b].a.bg.ro), d.data(), d.size() * sizeof(double),
                            hipMemcpyHostToDevice, e->stream));
-    EHIP(e, hipMemcpyAsync(const_cast<float *>(e->hbox[b].bg.ro32), f.data(), f.size() * sizeof(float),
+    EHIP(e, hipMemcpyAsync(const_cast<float *>(e->hbox[b].a.bg.ro32), f.data(), f.size() * sizeof(float),
                            hipMemcpyHostToDevice, e->stream));
-    EHIP(e, hipMemcpyAsync(const_cast<PlaneM *>(e->hbox[b].bg.planes), pl.data(), pl.size() * sizeof(PlaneM),
+    EHIP(e, hipMemcpyAsync(const_cast<PlaneM *>(e->hbox[b].a.bg.planes), pl.data(), pl.size() * sizeof(PlaneM),
                            hipMemcpyHostToDevice, e->stream));
     EHIP(e, hipStreamSynchronize(e->stream));
     B.have_bg = true;
@@ -325,8 +325,8 @@ extern "C" int mhd_ens_upload(mhd_ens_t *e, int b, const double *ru, const doubl
             EHIP(e, launch_pack(B.p, e->stage, D.q[0] + off, e->stream));
             EHIP(e, launch_pack(B.p, e->stage, D.q[1] + off, e->stream));
         } else {
-            EHIP(e, launch_pack_mixed(B.p, e->stage, f, D.bg, D.h[1], D.rr, e->stream));
-            EHIP(e, launch_pack_mixed(B.p, e->stage, f, D.bg, D.h[0], D.rr, e->stream));
+            EHIP(e, launch_pack_mixed(B.p, e->stage, f, D.a.bg, D.h[1], D.rr, e->stream));
+            EHIP(e, launch_pack_mixed(B.p, e->stage, f, D.a.bg, D.h[0], D.rr, e->stream));
         }
     }
     EHIP(e, hipStreamSynchronize(e->stream));
@@ -350,7 +350,7 @@ extern "C" int mhd_ens_download(mhd_ens_t *e, int b, double *ru, double *rv, dou
         if (!dst[f]) continue;
         const size_t off = (size_t)f * B.p.fsize;
         if (!e->mixed) EHIP(e, launch_unpack(B.p, D.q[e->cur] + off, e->stage, 1, e->stream));
-        else EHIP(e, launch_unpack_mixed(B.p, D.h[e->cur], D.rr, f, D.bg, e->stage, e->stream));
+        else EHIP(e, launch_unpack_mixed(B.p, D.h[e->cur], D.rr, f, D.a.bg, e->stage, e->stream));
         EHIP(e, hipMemcpyAsync(dst[f], e->stage, pbytes, hipMemcpyDeviceToHost, e->stream));
         EHIP(e, hipStreamSynchronize(e->stream));
     }
@@ -407,18 +407,13 @@ static hipError_t enqueue_step(mhd_ens_t *e, int a) {
     hipError_t r = hipSuccess;
     const int grid = e->grid > 0 && e->grid < e->nitems ? e->grid : e->nitems;
     for (int st = 1; st <= 3 && r == hipSuccess; ++st) {
-        if (!e->mixed) {
+        if (!e->mixed)
             r = launch_stage_batch(st, e->tile_y, e->lmag, e->dbox, e->ditems, e->nitems, grid, a, e->stream);
-            if (r == hipSuccess) r = launch_bcon_batch(e->lmag, e->dbox, e->dcols, e->ncols, a, st == 3, e->stream);
-        } else {
+        else
             r = launch_stage_batch_mixed(st, e->tile_x, e->tile_y, e->lmag, e->dbox, e->ditems, e->nitems, grid, a,
                                          e->stream);
-            if (r == hipSuccess)
-                r = launch_bcon_batch_mixed(e->lmag, e->dbox, e->dcols, e->ncols, a, st == 3, e->stream);
-        }
         a = 1 - a;
     }
-    if (r == hipSuccess) r = launch_cfl_final_batch(e->dbox, e->nbox, true, e->stream);
     return r;
 }
 
@@ -430,9 +425,8 @@ static int prime_cfl(mhd_ens_t *e) {
             return efail(e, MHD_ERR_STATE, "box %d: metrics and state must be set before stepping", b);
         if (B.cfl_valid) continue;
         const BoxDev &D = e->hbox[b];
-        if (!e->mixed) EHIP(e, launch_cfl(B.p, D.m, D.q[e->cur], D.sc, e->stream));
-        else EHIP(e, launch_cfl_mixed(B.p, D.m, D.bg, D.h[e->cur], D.rr, D.sc, e->stream));
-        EHIP(e, launch_cfl_final(B.p, D.sc, false, e->stream));
+        if (!e->mixed) EHIP(e, launch_cfl(B.p, D.a.m, D.q[e->cur], D.sc, D.cs, e->stream));
+        else EHIP(e, launch_cfl_mixed(B.p, D.a.m, D.a.bg, D.h[e->cur], D.rr, D.sc, D.cs, e->stream));
         B.cfl_valid = true;
     }
     return MHD_OK;

@@ -72,6 +72,35 @@ inline int check_desc(const mhd_desc *d, char *msg, size_t len) {
     return MHD_OK;
 }
 
+// z chunks of a box's stage launches.  A launch is a number of rounds in
+// which every CU holds `occ` workgroups, and a last round with fewer; a
+// workgroup's time is its planes plus about 1.5 planes of warm-up, times the
+// time of a plane, which grows with the workgroups that share the CU (FP64:
+// 3.3 us alone, 5.7 us with two; mixed: 2.6, 3.5, 4.4 us).  The count with
+// the least sum wins: small boxes split until the chip is about full (64x64x32
+// FP64: 11 chunks of 3 planes, a stage of 20 us against 38 with 4 chunks on 64
+// of 256 CUs), larger ones take whole rounds (256x256x128 mixed: 6 chunks, two
+// full rounds, 230 us against 254 with 16 chunks of 5.3 rounds).  Chunks are
+// at most 32 planes: over a longer march the tiles that share halo rows drift
+// apart and re-read them from HBM (512x512x256 FP64, 128 planes: 14% more
+// bytes fetched).
+inline int z_chunks(int npz, int ntiles, int occ, double alone, double more) {
+    constexpr int CUS = 256;
+    int best = 1;
+    double tbest = 0.0;
+    for (int nc = (npz + 31) / 32; nc <= max_chunks(npz) || nc == 1; ++nc) {
+        const long long n = (long long)ntiles * nc, slots = (long long)CUS * occ;
+        const long long rest = (n % slots + CUS - 1) / CUS;
+        const double round = alone + (occ - 1) * more, last = rest ? alone + (rest - 1) * more : 0.0;
+        const double t = ((npz + nc - 1) / nc + 1.5) * ((double)(n / slots) * round + last);
+        if (tbest == 0.0 || t < tbest) {
+            tbest = t;
+            best = nc;
+        }
+    }
+    return best;
+}
+
 // Kernel parameters of a box.  The products the reference forms once per
 // FLUXES / STEP call are formed here with the same association.
 inline Params params_from_desc(const mhd_desc *d) {
@@ -81,6 +110,13 @@ inline Params params_from_desc(const mhd_desc *d) {
     p.izc = d->izcon; p.itc = d->itcon; p.ibc = d->ibcon;
     p.tile_y = 4;
     if (const char *ty = getenv("RAST3DMHD_TILE_Y")) p.tile_y = atoi(ty) == 8 ? 8 : 4;
+    {
+        // workgroups per CU by LDS and registers (64x8 tiles: half)
+        const bool mixed = d->precision == MHD_MIXED;
+        const int occ = (mixed ? (d->lmag ? 3 : 4) : 2) / (p.tile_y == 8 ? 2 : 1);
+        const int ntiles = ((d->npx + 63) / 64) * ((d->npy + p.tile_y - 1) / p.tile_y);
+        p.nchunks = z_chunks(d->npz, ntiles, occ, mixed ? 2.6 : 3.3, mixed ? 0.9 : 2.4);
+    }
     p.plane = (long long)d->npx * d->npy;
     p.fsize = p.plane * (d->npz + 2) + FIELD_PAD;
     p.hx = d->hx; p.h2x = d->h2x; p.hy = d->hy; p.h2y = d->h2y; p.hz = d->hz; p.h2z = d->h2z;
@@ -106,11 +142,9 @@ inline Params params_from_desc(const mhd_desc *d) {
     return p;
 }
 
-// Initial device scalars: reduction keys armed, clocks zero.
+// Initial device scalars: clocks zero.
 inline DevScalars initial_scalars() {
     DevScalars s{};
-    s.key_mach = dkey(0.0);
-    for (int n = 0; n < 4; ++n) s.key_min[n] = dkey(INFINITY);
     s.dd2min = INFINITY;
     return s;
 }

@@ -41,6 +41,7 @@ struct Params {
     int npx, npy, npz;          // interior sizes
     int lmag, lrot, izc, itc, ibc;
     int tile_y;                 // rows per stage-kernel tile (4 or 8)
+    int nchunks;                // z chunks of a stage launch (z_chunks)
     long long plane;            // npx*npy
     long long fsize;            // field stride: plane*(npz+2) values incl. z ghost planes, + FIELD_PAD
     double hx, h2x, hy, h2y, hz, h2z, c13, c23, c43;
@@ -76,19 +77,34 @@ struct Metrics {
     const double *rkcfl;        // conductivity of the CFL limit: RKAPA, or 1+RKAPA with LREM (sub:844-852)
 };
 
-// Per-step device scalars.  The reductions keep order-preserving integer
-// keys of the doubles so that min/max can use 64-bit integer atomics.
+// Per-step device scalars.
 struct DevScalars {
     double dt, umach;                 // for the next step (from the last reduction)
     double dt_used, umach_used;       // of the step that last completed
     double cflmin[4];
     double timc, timi, timt;
-    unsigned long long key_mach;      // max of OGAMMA*UU/TT
-    unsigned long long key_min[4];    // mins of the CFL limits
     double fixed_dt;                  // > 0: step with this dt instead of the CFL dt
     double dd2min;                    // min over all points of min(DDX,DDY,DDZ)^2 (metric only)
     int nit;
     int nonfinite;
+};
+
+// Reduction slots of the CFL limits of one box: order-preserving integer keys
+// of the doubles (dkey), so that min/max are exact and independent of their
+// order, and the arrival counters by which the last workgroup of a reduction
+// closes it (cfl_publish).  key[0] holds the complement of the Mach key, so
+// that all five are minima.  Each slot has a cache line of its own, in
+// CFL_REP copies: the workgroups of a launch end close together, and atomics
+// on one line queue (512 workgroups with five keys in one line: 23 us for a
+// reduction whose arithmetic takes 4).
+constexpr int CFL_REP = 8, CFL_KEYS = 5;
+struct alignas(128) CflSlot {
+    unsigned long long v;
+};
+struct CflSlots {
+    CflSlot key[CFL_KEYS][CFL_REP];
+    CflSlot count[CFL_REP];
+    CflSlot done;
 };
 
 // Hydrostatic background of the mixed form, per plane k = 0..npz+1:
@@ -121,50 +137,46 @@ struct Background {
     const int *force_on;
 };
 
+// A box's parameters and tables, as kernel arguments and in BoxDev.
+struct BoxArgs {
+    Params p;
+    Metrics m;
+    Background bg;  // mixed form
+};
+
 // One box of an ensemble as the batched kernels see it (device memory).
 // FP64 boxes use q/z, mixed boxes h/dr/rr and bg.
 struct BoxDev {
-    Params p;
-    Metrics m;
-    Background bg;
+    BoxArgs a;
     double *q[2];
     double *z;
     float *h[2];
     float *dr;
     unsigned *rr;
     DevScalars *sc;
+    CflSlots *cs;
 };
 
 // Bytes of the mixed form's residual register R for nf fields.
 inline size_t resid_bytes(int nf, long long fsize) { return (size_t)((nf + 1) / 2) * (size_t)fsize * 4; }
 
-// Work item of a batched stage launch: one tile column chunk of one box.
+// Work item of a batched stage launch: one tile column chunk of one box,
+// number seq of the box's total items.
 struct StageItem {
-    int box, i0, j0, kbeg, kend;
+    int box, i0, j0, kbeg, kend, seq, total;
 };
 
-// Work item of a batched boundary-plane launch: 256 columns of one box.
-struct ColumnItem {
-    int box, col0;
-};
+// Planes 1..npz of a box split into nc chunks of sizes that differ by at most
+// one: chunk c covers planes chunk_begin(npz, nc, c) .. chunk_begin(npz, nc,
+// c + 1) - 1.  A chunk with a boundary plane also applies the boundary
+// conditions there, which read the two planes next to it, so a chunk has at
+// least three planes: nc <= max_chunks(npz).
+__host__ __device__ inline int chunk_begin(int npz, int nc, int c) { return 1 + (int)((long long)c * npz / nc); }
+__host__ __device__ inline int max_chunks(int npz) { return npz / 3 > 0 ? npz / 3 : 1; }
 
 __host__ __device__ inline unsigned long long dkey(double v) {
     unsigned long long b = __builtin_bit_cast(unsigned long long, v);
     return (b >> 63) ? ~b : (b | 0x8000000000000000ull);
-}
-// Updates of a reduction key.  Between its reset (by an earlier launch or
-// the host) and its read (by a later launch) a key only moves one way, so
-// a workgroup whose value cannot move it, by a read of the key at device
-// scope (coherent across the XCDs' L2 caches), skips the atomic: a stale
-// read can only cost an atomic that was not needed, never skip one that
-// was.  Without the check every workgroup of a launch queues an atomic on
-// the same cache line; for the 1024 short workgroups of a boundary-plane
-// launch that queue was three quarters of the launch.
-__device__ inline void key_raise(unsigned long long *k, unsigned long long v) {
-    if (v > __hip_atomic_load(k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(k, v);
-}
-__device__ inline void key_lower(unsigned long long *k, unsigned long long v) {
-    if (v < __hip_atomic_load(k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(k, v);
 }
 __host__ __device__ inline double dunkey(unsigned long long k) {
     unsigned long long b = (k >> 63) ? (k & 0x7fffffffffffffffull) : ~k;
@@ -196,13 +208,15 @@ inline size_t opt_work_len(const Params &p) { return 3 * (size_t)(p.npz + 2) + p
 hipError_t launch_opt_means(const Params &p, const Metrics &m, const double *q, const OptBuffers &o,
                             DevScalars *sc, hipStream_t s);
 
-// Launchers (mhd_kernels.hip).
+// Launchers (mhd_kernels.hip).  launch_stage with mode 1..3 also applies the
+// boundary conditions to qout; mode 3 closes the step (DT of the next step,
+// clock).  launch_cfl is the stand-alone reduction after an upload.
 hipError_t launch_stage(int mode, const Params &p, const Metrics &m, const double *qin, double *qout,
-                        double *z, double *fout, DevScalars *sc, hipStream_t s);
-hipError_t launch_bcon(const Params &p, const Metrics &m, const double *qin, double *qout, DevScalars *sc,
-                       bool cfl, hipStream_t s);
-hipError_t launch_cfl(const Params &p, const Metrics &m, const double *q, DevScalars *sc, hipStream_t s);
-hipError_t launch_cfl_final(const Params &p, DevScalars *sc, bool clock, hipStream_t s);
+                        double *z, double *fout, DevScalars *sc, CflSlots *cs, hipStream_t s);
+hipError_t launch_cfl(const Params &p, const Metrics &m, const double *q, DevScalars *sc, CflSlots *cs,
+                      hipStream_t s);
+// Arms the CFL reduction slots of n boxes.
+hipError_t launch_cfl_arm(CflSlots *cs, int n, hipStream_t s);
 hipError_t launch_pack(const Params &p, const double *padded, double *field, hipStream_t s);
 hipError_t launch_unpack(const Params &p, const double *field, double *padded, int mode, hipStream_t s);
 
@@ -210,9 +224,6 @@ hipError_t launch_unpack(const Params &p, const double *field, double *padded, i
 // a of every box is the stage input.  grid is the persistent grid size.
 hipError_t launch_stage_batch(int mode, int tile_y, int lmag, const BoxDev *boxes, const StageItem *items,
                               int nitems, int grid, int a, hipStream_t s);
-hipError_t launch_bcon_batch(int lmag, const BoxDev *boxes, const ColumnItem *items, int nitems, int a, bool cfl,
-                             hipStream_t s);
-hipError_t launch_cfl_final_batch(const BoxDev *boxes, int nbox, bool clock, hipStream_t s);
 hipError_t launch_box_filter(const Params &p, const double *q, int nf, int factor, int zmode, int nxc, int nyc, int nzc,
                              double *out, hipStream_t s);
 
@@ -238,11 +249,9 @@ hipError_t launch_flux_profiles_mixed(const Params &p, const float *h, const uns
 // fields per 32-bit word: (nf+1)/2 words per point, written by stage 3 and
 // the upload, read by stage 1).
 hipError_t launch_stage_mixed(int mode, const Params &p, const Metrics &m, const Background &bg, const float *hin,
-                              float *hout, float *dr, unsigned *rr, DevScalars *sc, hipStream_t s);
-hipError_t launch_bcon_mixed(const Params &p, const Metrics &m, const Background &bg, float *h, float *dr,
-                             unsigned *rr, DevScalars *sc, bool last, hipStream_t s);
+                              float *hout, float *dr, unsigned *rr, DevScalars *sc, CflSlots *cs, hipStream_t s);
 hipError_t launch_cfl_mixed(const Params &p, const Metrics &m, const Background &bg, const float *h,
-                            const unsigned *rr, DevScalars *sc, hipStream_t s);
+                            const unsigned *rr, DevScalars *sc, CflSlots *cs, hipStream_t s);
 // Conversion of field `field` between a padded FP64 array and the stored
 // values / resting residuals of the registers hreg, rreg (base pointers, all
 // fields).  Pack rho (field 3) before T (field 4).
@@ -257,8 +266,6 @@ hipError_t launch_rebase_mixed(const Params &p, const Background &ob, const Back
 
 hipError_t launch_stage_batch_mixed(int mode, int tile_x, int tile_y, int lmag, const BoxDev *boxes,
                                     const StageItem *items, int nitems, int grid, int a, hipStream_t s);
-hipError_t launch_bcon_batch_mixed(int lmag, const BoxDev *boxes, const ColumnItem *items, int nitems, int a,
-                                   bool last, hipStream_t s);
 
 // Network entry points used by the closure-corrected step (mhd_net.hip).
 int net_shape(const mhd_net *n, int *cin, int *cout);

@@ -2,10 +2,10 @@
 //
 // K2 k_stage : right-hand side of FLUXES (3dmhdsub.f:1178-2637) fused with one
 //              Wray RK3 stage update of STEP (3dmhdsub.f:926-969, 977-1067,
-//              1075-1165), one launch per stage.  Stage 3 also reduces the
-//              CFL limits of the new state for the next step (sub:741-873).
-// K3 k_bcon  : boundary planes of BCON (3dmhdsub.f:2751-2958); after stage 3
-//              it adds the boundary planes' CFL contributions.
+//              1075-1165), one launch per stage, with the boundary planes of
+//              BCON (3dmhdsub.f:2751-2958).  Stage 3 also reduces the CFL
+//              limits of the new state for the next step (sub:741-873), and
+//              its last workgroup closes the step (DT, clock).
 // K1 k_cfl   : stand-alone CFL / Mach reduction for the first step after an
 //              upload (sub:741-873).
 // K4 k_pack / k_unpack : conversion between the reference's padded arrays
@@ -25,7 +25,12 @@
 // is computed, and the Z register of the RK3 scheme is prefetched the same
 // way, so each global load has a whole plane of arithmetic to hide behind.
 // Outputs are written with non-temporal stores so that L2 keeps the halo
-// rows that neighbouring tiles re-read.
+// rows that neighbouring tiles re-read.  What bounds it: at 512x512x256 HBM
+// (2.86 / 3.59 / 3.13 ms for 12.9 / 17.2 / 12.9 GB of algorithmic bytes); on
+// small boxes the latency of a plane's march (3.3 us with one workgroup on a
+// CU) and of the launch, hence few planes per chunk (z_chunks) and three
+// launches per step (64x64x32: 72 us per step, 132 with boundary, CFL and
+// 8-plane launches of their own; 16x16x12 by single steps: 88 against 210).
 //
 // Arithmetic: every expression keeps the reference's left-to-right
 // association and the file is compiled with -ffp-contract=off, so results
@@ -90,12 +95,12 @@ __device__ __forceinline__ void cfl_point(const Params &p, const double *q, doub
     if (MAG) w4 = fmin(w4, 0.5 * dd * dd * p.rm);
 }
 
-// Workgroup reduction of the CFL accumulators and one set of 64-bit atomics
-// on order-preserving keys (min/max are exact, so the order is irrelevant).
-// NaN keys sort above +Inf: they win the max and, through the key of -NaN
-// (below -Inf), the min, so a non-finite state cannot go unnoticed.
-__device__ void cfl_reduce(double mach, double w1, double w2, double w3, double w4, int lmag,
-                           DevScalars *__restrict__ sc) {
+// Workgroup reduction of the CFL accumulators, published as order-preserving
+// keys (min/max are exact, so the order is irrelevant); workgroup seq of
+// total.  NaN keys sort above +Inf: they win the max and, through the key of
+// -NaN (below -Inf), the min, so a non-finite state cannot go unnoticed.
+__device__ void cfl_reduce(double mach, double w1, double w2, double w3, double w4, double sf, int lmag,
+                           int clock, DevScalars *__restrict__ sc, CflSlots *__restrict__ cs, int seq, int total) {
     __shared__ unsigned long long red[16][5];
     unsigned long long km = dkey(mach), k1 = dkey(w1), k2 = dkey(w2), k3 = dkey(w3), k4 = dkey(w4);
     // a NaN limit becomes -NaN for the min reduction
@@ -123,11 +128,99 @@ __device__ void cfl_reduce(double mach, double w1, double w2, double w3, double 
             k3 = red[v][3] < k3 ? red[v][3] : k3;
             k4 = red[v][4] < k4 ? red[v][4] : k4;
         }
-        key_raise(&sc->key_mach, km);
-        key_lower(&sc->key_min[0], k1);
-        key_lower(&sc->key_min[1], k2);
-        key_lower(&sc->key_min[2], k3);
-        if (lmag) key_lower(&sc->key_min[3], k4);
+    }
+    if (threadIdx.x < 64) {
+        const unsigned long long k[CFL_KEYS] = {~km, k1, k2, k3, k4};
+        cfl_publish(k, sc, cs, sf, lmag, clock, seq, total);
+    }
+}
+
+// BCON on the boundary planes (top: plane 1, bot: plane npz) of one column of
+// the freshly written register q, and the in-place 1/rho of the untouched z
+// ghost planes that FLUXES performs (sub:1390) so that the resident ghosts
+// follow the reference exactly.  A stage's workgroup calls it for the columns
+// it owns when its chunk holds a boundary plane and so, with at least three
+// planes, everything BCON reads: the conditions then need no launch of their
+// own (5, 5 and 10 us of a 130 us step at 64x64x32, 8, 8 and 23 us of 1280
+// at 256x256x128).  With CFL set (stage 3), the boundary planes' CFL limits
+// of the final state are added to the accumulators.
+template <bool MAG, bool CFL>
+__device__ __forceinline__ void bcon_column(const Params &p, const Metrics &m, const double *__restrict__ qin,
+                                            double *q, const DevScalars *sc, int i, int j, bool top, bool bot,
+                                            double &c_mach, double &c_w1, double &c_w2, double &c_w3, double &c_w4) {
+    const long long fs = p.fsize, pl = p.plane, idx = (long long)j * p.npx + i;
+    const int nz = p.npz;
+    const double C13 = p.c13, C23 = p.c23, C43 = p.c43;
+    double *RU = q, *RV = q + fs, *RW = q + 2 * fs, *RO = q + 3 * fs, *TT = q + 4 * fs, *BZ = q + 7 * fs;
+    const double *ROi = qin + 3 * fs;
+    // shear boundaries: RRT = 1, RRB = -1, RPP = 0 (sub:2751-2756)
+    const double shear = p.lshr ? cos(0.0 * sc->timt) : 0.0;
+    auto limits = [&](int k) __attribute__((always_inline)) {
+        const long long o = (long long)k * pl + idx;
+        double v[8];
+#pragma unroll
+        for (int f = 0; f < (MAG ? 8 : 5); ++f) v[f] = q[f * fs + o];
+        cfl_point<MAG>(p, v, m.ddx[i + 1], m.ddy[j + 1], m.ddz[k], m.rkcfl[k], c_mach, c_w1, c_w2, c_w3, c_w4);
+    };
+    if (top) {  // sub:2771-2868
+        const long long a = pl + idx, b = 2 * pl + idx, c = 3 * pl + idx;
+        if (p.lshr) {
+            RU[a] = 0.0;
+            RV[a] = 1.0 * shear * RO[a];
+        } else {
+            RU[a] = RO[a] * (C43 * RU[b] / RO[b] - C13 * RU[c] / RO[c]);
+            RV[a] = RO[a] * (C43 * RV[b] / RO[b] - C13 * RV[c] / RO[c]);
+        }
+        RW[a] = 0.0;
+        if (p.tp != 0.0 && (p.itc == 0 || p.itc == 1)) {
+            // Gaussian top temperature or flux (sub:2790-2827)
+            const double HH = p.hh, ex = p.gx[i + 1], ey = p.gy[j + 1];
+            if (p.itc == 0) {
+                TT[a] = 1.0 - (1.0 - p.tpr) * ex / HH * ey / HH;
+            } else {
+                const double dz = p.dzf / m.dzzdz[1];
+                TT[a] = C43 * TT[b] - C13 * TT[c] - C23 * dz * (p.theta - (p.theta - p.tpr) * ex / HH * ey / HH);
+            }
+        } else if (p.itc == 0 || p.itc == 2 || p.itc == 4) {
+            // fixed T; TU with LREM; ITC=4: TP cooler on I <= NX/2 (sub:2828-2850)
+            if (p.lrem) TT[a] = p.tu;
+            else TT[a] = (p.itc == 4 && i + 2 <= (p.npx + 2) / 2) ? 1.0 - p.tp : 1.0;
+        } else if (p.itc == 1) {
+            if (p.lrem) {
+                TT[a] = C43 * TT[b] - C13 * TT[c] + p.dztu;
+            } else {
+                const double dz = p.dzf / m.dzzdz[1];
+                TT[a] = C43 * TT[b] - C13 * TT[c] - C23 * dz * p.theta;
+            }
+        }  // ITC=3: the top temperature is left to the equations
+        if (MAG && p.ibc == 0) BZ[a] = 0.0;
+        // the z ghost plane of RO flips to 1/RO once per FLUXES call; with ID
+        // or LREM it held the mirrored RO of plane 2 (sub:1301-1310)
+        RO[idx] = 1.0 / ROi[(p.mirror ? 2 * pl : 0) + idx];
+        if (CFL) limits(1);
+    }
+    if (bot) {  // sub:2873-2955
+        const long long a = (long long)nz * pl + idx, b = (long long)(nz - 1) * pl + idx,
+                        c = (long long)(nz - 2) * pl + idx;
+        if (p.lshr) {
+            RU[a] = 0.0;
+            RV[a] = -1.0 * shear * RO[a];
+        } else {
+            RU[a] = RO[a] * (C43 * RU[b] / RO[b] - C13 * RU[c] / RO[c]);
+            RV[a] = RO[a] * (C43 * RV[b] / RO[b] - C13 * RV[c] / RO[c]);
+        }
+        RW[a] = 0.0;
+        if (p.izc == 0) {
+            TT[a] = p.tb;
+        } else if (p.lrem) {
+            TT[a] = C43 * TT[b] - C13 * TT[c] + p.dztb;
+        } else {
+            const double dz = p.dzf / m.dzzdz[nz];
+            TT[a] = C43 * TT[b] - C13 * TT[c] + C23 * dz * p.theta / m.rkapa[nz];
+        }
+        if (MAG && p.ibc == 0) BZ[a] = 0.0;
+        RO[(long long)(nz + 1) * pl + idx] = 1.0 / ROi[(long long)(p.mirror ? nz - 1 : nz + 1) * pl + idx];
+        if (CFL) limits(nz);
     }
 }
 
@@ -139,17 +232,20 @@ constexpr int stage_lds_bytes() {
 
 // One tile column chunk of a stage: interior columns i0..i0+TX-1, rows
 // j0..j0+TY-1 (clipped to the box), planes kbeg..kend.  MODE 0 writes the
-// right-hand side F to fout; MODE 1..3 performs RK3 stage s.  The whole
-// workgroup calls it with the same arguments.
+// right-hand side F to fout; MODE 1..3 performs RK3 stage s with the boundary
+// conditions on the boundary planes it holds.  The whole workgroup calls it
+// with the same arguments.
 // OPT instantiates the optional branches of FLUXES (density diffusion,
 // Rempel conduction, shear boundaries, flux relaxation, embedded heat loss;
 // the per-plane tables come from mhd_opt.hip); the main path has none of
 // their code.
 template <int TY, bool MAG, int MODE, bool OPT = false>
-__device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, const double *__restrict__ qin,
+__device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, ArgPtr args,
+                                           const double *__restrict__ qin,
                                            double *__restrict__ qout, double *__restrict__ zr,
-                                           double *__restrict__ fout, DevScalars *__restrict__ sc, int i0, int j0,
-                                           int kbeg, int kend, double *lds) {
+                                           double *__restrict__ fout, DevScalars *__restrict__ sc,
+                                           CflSlots *__restrict__ cs, int i0, int j0, int kbeg, int kend, int seq,
+                                           int total, double *lds) {
     using T = Tile<TY>;
     constexpr int SW = T::SW, SP = T::SP;
     constexpr int NF = MAG ? 8 : 5;
@@ -193,32 +289,39 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, co
         ring(k, 2, pt) = r.v[S_RW] * ri;
     };
 
+    // Warm-up: planes kbeg-1 (own values + ring), kbeg and kbeg+1 (LDS + ring).
+    // Every load is issued before the first is used: a chunk then pays one
+    // memory latency before its march instead of three.
     Raw rm_, rp_o, rp_h;
-    // warm-up: planes kbeg-1 (own values + ring), kbeg and kbeg+1 (LDS + ring)
-    load_raw<MAG>(qin, fs, (long long)(kbeg - 1) * pl + ooff, rm_);
-    if (OPT && p.mirror && kbeg == 1) {
-        // ghost plane 0 holds RO of plane 2 while FLUXES runs (sub:1303-1304)
-        rm_.v[S_RO] = qin[3 * fs + 2 * pl + ooff];
-    }
-    put_ring(kbeg - 1, opt, rm_);
-    if (has_h) {
-        load_raw<MAG>(qin, fs, (long long)(kbeg - 1) * pl + hoff, rp_h);
-        if (OPT && p.mirror && kbeg == 1) rp_h.v[S_RO] = qin[3 * fs + 2 * pl + hoff];
-        put_ring(kbeg - 1, hpt, rp_h);
-    }
-#pragma unroll 1
-    for (int kk = kbeg; kk <= kbeg + 1; ++kk) {
-        // ghost plane npz+1 holds RO of plane npz-1 (sub:1306-1307)
-        const bool mir = OPT && p.mirror && kk == npz + 1;
-        load_raw<MAG>(qin, fs, (long long)kk * pl + ooff, rp_o);
-        if (mir) rp_o.v[S_RO] = qin[3 * fs + (long long)(npz - 1) * pl + ooff];
-        put_cur(kk, opt, rp_o);
-        put_ring(kk, opt, rp_o);
+    {
+        Raw ro_[2], rh_[3];
+        // with ID or LREM the ghost planes 0 and npz+1 hold RO of planes 2 and
+        // npz-1 while FLUXES runs (sub:1303-1307)
+        auto get = [&](int kk, long long off, Raw &r) __attribute__((always_inline)) {
+            load_raw<MAG>(qin, fs, (long long)kk * pl + off, r);
+            if (OPT && p.mirror && (kk == 0 || kk == npz + 1))
+                r.v[S_RO] = qin[3 * fs + (long long)(kk == 0 ? 2 : npz - 1) * pl + off];
+        };
+        get(kbeg - 1, ooff, rm_);
+        get(kbeg, ooff, ro_[0]);
+        get(kbeg + 1, ooff, ro_[1]);
         if (has_h) {
-            load_raw<MAG>(qin, fs, (long long)kk * pl + hoff, rp_h);
-            if (mir) rp_h.v[S_RO] = qin[3 * fs + (long long)(npz - 1) * pl + hoff];
-            put_cur(kk, hpt, rp_h);
-            put_ring(kk, hpt, rp_h);
+#pragma unroll
+            for (int n = 0; n < 3; ++n) get(kbeg - 1 + n, hoff, rh_[n]);
+        }
+        put_ring(kbeg - 1, opt, rm_);
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            put_cur(kbeg + n, opt, ro_[n]);
+            put_ring(kbeg + n, opt, ro_[n]);
+        }
+        if (has_h) {
+            put_ring(kbeg - 1, hpt, rh_[0]);
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {
+                put_cur(kbeg + n, hpt, rh_[n + 1]);
+                put_ring(kbeg + n, hpt, rh_[n + 1]);
+            }
         }
     }
 
@@ -613,28 +716,34 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, co
 #pragma unroll 1
     for (int k = k0; k <= k1; ++k) plane(k, std::false_type{});
     if (last_bnd) plane(npz, std::true_type{});
-    if (MODE == 3) cfl_reduce(c_mach, c_w1, c_w2, c_w3, c_w4, p.lmag, sc);
+    if (MODE > 0 && (kbeg == 1 || kend == npz) && valid) {
+        const BoxArgs &l = late_args(args);
+        bcon_column<MAG, MODE == 3>(l.p, l.m, qin, qout, sc, gi, gj, kbeg == 1, kend == npz, c_mach, c_w1, c_w2, c_w3,
+                                    c_w4);
+    }
+    if (MODE == 3) {
+        const BoxArgs &l = late_args(args);
+        cfl_reduce(c_mach, c_w1, c_w2, c_w3, c_w4, l.p.sf, l.p.lmag, 1, sc, cs, seq, total);
+    }
 }
 
 // Single box: workgroup -> (tile, z chunk), XCD-aware.
 template <int TY, bool MAG, int MODE, bool OPT>
-__global__ __launch_bounds__(TX *TY, 2) void k_stage(const Params p, const Metrics m,
+__global__ __launch_bounds__(TX *TY, 2) void k_stage(const BoxArgs b,
                                                   const double *__restrict__ qin,
                                                   double *__restrict__ qout,
                                                   double *__restrict__ zr,
                                                   double *__restrict__ fout,
-                                                  DevScalars *__restrict__ sc,
-                                                  int kchunk) {
+                                                  DevScalars *__restrict__ sc, CflSlots *__restrict__ cs,
+                                                  int nchunks) {
     extern __shared__ double lds[];
+    const Params &p = b.p;
     const int ntx = (p.npx + TX - 1) / TX, nty = (p.npy + TY - 1) / TY;
-    const int bid = xcd_remap(blockIdx.x, gridDim.x);
-    const int tz = bid / (ntx * nty);
-    const int rem = bid - tz * (ntx * nty);
-    const int tyb = rem / ntx, txb = rem - tyb * ntx;
-    const int kbeg = 1 + tz * kchunk;
-    const int kend = min(p.npz, kbeg + kchunk - 1);
-    if (kbeg > p.npz) return;
-    stage_tile<TY, MAG, MODE, OPT>(p, m, qin, qout, zr, fout, sc, txb * TX, tyb * TY, kbeg, kend, lds);
+    const TileChunk tc = tile_of(blockIdx.x, ntx * nty, nchunks);
+    const int tz = tc.chunk, tyb = tc.tile / ntx, txb = tc.tile - tyb * ntx;
+    const int kbeg = chunk_begin(p.npz, nchunks, tz), kend = chunk_begin(p.npz, nchunks, tz + 1) - 1;
+    stage_tile<TY, MAG, MODE, OPT>(p, b.m, kernel_args(), qin, qout, zr, fout, sc, cs, txb * TX, tyb * TY, kbeg, kend,
+                                   blockIdx.x, gridDim.x, lds);
 }
 
 // Ensemble: a persistent grid walks the work-item table of all boxes with a
@@ -647,127 +756,17 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage_batch(const BoxDev *__restr
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
     for (int w = slot; w < nitems; w += gridDim.x) {
         const StageItem it = items[w];
-        const BoxDev &B = boxes[it.box];
+        const BoxDev &B = box_at(boxes, it.box);
         __syncthreads();  // the previous item's last LDS reads are done
-        stage_tile<TY, MAG, MODE>(B.p, B.m, B.q[a], B.q[1 - a], B.z, nullptr, B.sc, it.i0, it.j0, it.kbeg, it.kend,
-                                  lds);
+        stage_tile<TY, MAG, MODE>(B.a.p, B.a.m, (ArgPtr)&B.a, B.q[a], B.q[1 - a], B.z, nullptr, B.sc, B.cs, it.i0, it.j0, it.kbeg,
+                                  it.kend, it.seq, it.total, lds);
     }
-}
-
-// BCON on the two boundary planes of the freshly written register, and the
-// in-place 1/rho of the untouched z ghost planes that FLUXES performs
-// (sub:1390) so that the resident ghosts follow the reference exactly.
-// With CFL set (after stage 3), the boundary planes' CFL limits of the final
-// state are added to the reduction.
-// Column idx of the plane (npx*npy columns); the whole workgroup calls it.
-template <bool MAG, bool CFL>
-__device__ __forceinline__ void bcon_column(const Params &p, const Metrics &m, const double *__restrict__ qin,
-                                            double *__restrict__ q, DevScalars *__restrict__ sc, int idx) {
-    double c_mach = 0.0, c_w1 = INFINITY, c_w2 = INFINITY, c_w3 = INFINITY, c_w4 = INFINITY;
-    if (idx < p.npx * p.npy) {
-        const long long fs = p.fsize, pl = p.plane;
-        const int nz = p.npz;
-        const double C13 = p.c13, C23 = p.c23, C43 = p.c43;
-        const int j = idx / p.npx, i = idx - j * p.npx;
-        double *RU = q, *RV = q + fs, *RW = q + 2 * fs, *RO = q + 3 * fs, *TT = q + 4 * fs, *BZ = q + 7 * fs;
-        // shear boundaries: RRT = 1, RRB = -1, RPP = 0 (sub:2751-2756)
-        const double shear = p.lshr ? cos(0.0 * sc->timt) : 0.0;
-        // top (sub:2771-2868)
-        {
-            const long long a = pl + idx, b = 2 * pl + idx, c = 3 * pl + idx;
-            if (p.lshr) {
-                RU[a] = 0.0;
-                RV[a] = 1.0 * shear * RO[a];
-            } else {
-                RU[a] = RO[a] * (C43 * RU[b] / RO[b] - C13 * RU[c] / RO[c]);
-                RV[a] = RO[a] * (C43 * RV[b] / RO[b] - C13 * RV[c] / RO[c]);
-            }
-            RW[a] = 0.0;
-            if (p.tp != 0.0 && (p.itc == 0 || p.itc == 1)) {
-                // Gaussian top temperature or flux (sub:2790-2827)
-                const double HH = p.hh, ex = p.gx[i + 1], ey = p.gy[j + 1];
-                if (p.itc == 0) {
-                    TT[a] = 1.0 - (1.0 - p.tpr) * ex / HH * ey / HH;
-                } else {
-                    const double dz = p.dzf / m.dzzdz[1];
-                    TT[a] = C43 * TT[b] - C13 * TT[c] - C23 * dz * (p.theta - (p.theta - p.tpr) * ex / HH * ey / HH);
-                }
-            } else if (p.itc == 0 || p.itc == 2 || p.itc == 4) {
-                // fixed T; TU with LREM; ITC=4: TP cooler on I <= NX/2 (sub:2828-2850)
-                if (p.lrem) TT[a] = p.tu;
-                else TT[a] = (p.itc == 4 && i + 2 <= (p.npx + 2) / 2) ? 1.0 - p.tp : 1.0;
-            } else if (p.itc == 1) {
-                if (p.lrem) {
-                    TT[a] = C43 * TT[b] - C13 * TT[c] + p.dztu;
-                } else {
-                    const double dz = p.dzf / m.dzzdz[1];
-                    TT[a] = C43 * TT[b] - C13 * TT[c] - C23 * dz * p.theta;
-                }
-            }  // ITC=3: the top temperature is left to the equations
-            if (MAG && p.ibc == 0) BZ[a] = 0.0;
-        }
-        // bottom (sub:2873-2955)
-        {
-            const long long a = (long long)nz * pl + idx, b = (long long)(nz - 1) * pl + idx,
-                            c = (long long)(nz - 2) * pl + idx;
-            if (p.lshr) {
-                RU[a] = 0.0;
-                RV[a] = -1.0 * shear * RO[a];
-            } else {
-                RU[a] = RO[a] * (C43 * RU[b] / RO[b] - C13 * RU[c] / RO[c]);
-                RV[a] = RO[a] * (C43 * RV[b] / RO[b] - C13 * RV[c] / RO[c]);
-            }
-            RW[a] = 0.0;
-            if (p.izc == 0) {
-                TT[a] = p.tb;
-            } else if (p.lrem) {
-                TT[a] = C43 * TT[b] - C13 * TT[c] + p.dztb;
-            } else {
-                const double dz = p.dzf / m.dzzdz[nz];
-                TT[a] = C43 * TT[b] - C13 * TT[c] + C23 * dz * p.theta / m.rkapa[nz];
-            }
-            if (MAG && p.ibc == 0) BZ[a] = 0.0;
-        }
-        // z ghost planes of RO flip to 1/RO once per FLUXES call; with ID or
-        // LREM they held the mirrored RO of planes 2 and npz-1 (sub:1301-1310)
-        const double *ROi = qin + 3 * fs;
-        RO[idx] = 1.0 / ROi[(p.mirror ? 2 * pl : 0) + idx];
-        RO[(long long)(nz + 1) * pl + idx] = 1.0 / ROi[(long long)(p.mirror ? nz - 1 : nz + 1) * pl + idx];
-        if (CFL) {
-            for (int kb = 0; kb < 2; ++kb) {
-                const int k = kb ? nz : 1;
-                const long long o = (long long)k * pl + idx;
-                double v[8];
-#pragma unroll
-                for (int f = 0; f < (MAG ? 8 : 5); ++f) v[f] = q[f * fs + o];
-                cfl_point<MAG>(p, v, m.ddx[i + 1], m.ddy[j + 1], m.ddz[k], m.rkcfl[k], c_mach, c_w1, c_w2,
-                               c_w3, c_w4);
-            }
-        }
-    }
-    if (CFL) cfl_reduce(c_mach, c_w1, c_w2, c_w3, c_w4, p.lmag, sc);
-}
-
-template <bool MAG, bool CFL>
-__global__ __launch_bounds__(256) void k_bcon(const Params p, const Metrics m, const double *__restrict__ qin,
-                                              double *__restrict__ q, DevScalars *__restrict__ sc) {
-    bcon_column<MAG, CFL>(p, m, qin, q, sc, blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-// Ensemble: one workgroup per (box, run of 256 columns); register a of
-// every box was the stage input, 1-a the freshly written output.
-template <bool MAG, bool CFL>
-__global__ __launch_bounds__(256) void k_bcon_batch(const BoxDev *__restrict__ boxes,
-                                                    const ColumnItem *__restrict__ items, int a) {
-    const ColumnItem it = items[blockIdx.x];
-    const BoxDev &B = boxes[it.box];
-    bcon_column<MAG, CFL>(B.p, B.m, B.q[a], B.q[1 - a], B.sc, it.col0 + threadIdx.x);
 }
 
 // Stand-alone CFL reduction over planes 1..npz (first step after an upload).
 template <bool MAG>
 __global__ __launch_bounds__(256) void k_cfl(const Params p, const Metrics m, const double *__restrict__ q,
-                                             DevScalars *__restrict__ sc) {
+                                             DevScalars *__restrict__ sc, CflSlots *__restrict__ cs) {
     const long long fs = p.fsize, pl = p.plane;
     const long long n = (long long)p.npz * pl;
     double mach = 0.0, w1 = INFINITY, w2 = INFINITY, w3 = INFINITY, w4 = INFINITY;
@@ -782,46 +781,11 @@ __global__ __launch_bounds__(256) void k_cfl(const Params p, const Metrics m, co
         for (int f = 0; f < (MAG ? 8 : 5); ++f) v[f] = q[f * fs + o];
         cfl_point<MAG>(p, v, m.ddx[i + 1], m.ddy[j + 1], m.ddz[k], m.rkcfl[k], mach, w1, w2, w3, w4);
     }
-    cfl_reduce(mach, w1, w2, w3, w4, p.lmag, sc);
+    cfl_reduce(mach, w1, w2, w3, w4, p.sf, p.lmag, 0, sc, cs, blockIdx.x, gridDim.x);
 }
 
-// End of a reduction: DT = SF*MIN(...), UMACH = SQRT(MAX(...)) (sub:761,
-// 868-872), then re-arm the keys.  A positive fixed_dt replaces the CFL DT.  With clock set this also closes the step
-// that just ran: NIT, TIMC, TIMT (sub:1171-1173) with the DT it used, which
-// is kept as dt_used / umach_used.
-__device__ __forceinline__ void cfl_final(DevScalars *sc, double sf, int lmag, int clock) {
-    if (clock) {
-        sc->nit = sc->nit + 1;
-        sc->timc = sc->timc + sc->dt;
-        sc->timt = sc->timi + sc->timc;
-        sc->dt_used = sc->dt;
-        sc->umach_used = sc->umach;
-    }
-    const double mach = dunkey(sc->key_mach);
-    double mn = INFINITY;
-    bool bad = !(mach == mach);
-    for (int n = 0; n < 4; ++n) {
-        sc->cflmin[n] = dunkey(sc->key_min[n]);
-        if (n < 3 || lmag) {
-            mn = fmin(mn, sc->cflmin[n]);
-            bad = bad || !(sc->cflmin[n] == sc->cflmin[n]);
-        }
-    }
-    sc->umach = sqrt(mach);
-    const double dcfl = sf * mn;
-    sc->dt = sc->fixed_dt > 0.0 ? sc->fixed_dt : dcfl;
-    if (bad || dcfl == INFINITY) sc->nonfinite |= 1;
-    sc->key_mach = dkey(0.0);
-    for (int n = 0; n < 4; ++n) sc->key_min[n] = dkey(INFINITY);
-}
-
-__global__ void k_cfl_final(DevScalars *sc, double sf, int lmag, int clock) { cfl_final(sc, sf, lmag, clock); }
-
-// Ensemble: one thread per box.
-__global__ void k_cfl_final_batch(const BoxDev *__restrict__ boxes, int nbox, int clock) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < nbox) cfl_final(boxes[b].sc, boxes[b].p.sf, boxes[b].p.lmag, clock);
-}
+// Arms the reduction slots of one box per workgroup (a new handle).
+__global__ __launch_bounds__(64) void k_cfl_arm(CflSlots *cs) { cfl_arm(cs + blockIdx.x, threadIdx.x); }
 
 // padded Fortran (npx+2, npy+2, npz+2) -> resident field (x/y ghosts dropped)
 __global__ void k_pack(const Params p, const double *__restrict__ padded, double *__restrict__ field) {
@@ -905,72 +869,52 @@ __global__ void k_box_filter(const Params p, const double *__restrict__ q, int n
 // ---------------------------------------------------------------------------
 // launchers
 
-// z chunks of about 32 planes: the tiles a cohort of co-resident workgroups
-// (one XCD) marches stay closer in step over a short march, so more of the
-// halo rows they share are still in L2 when the neighbour reads them
-// (512x512x256: 8 chunks fetch 14% fewer bytes and run 3% faster than 2
-// chunks of 128 planes).  At least 2048 workgroups; at least 8 planes.
-static int chunk_for(const Params &p, int ty, int *nchunks) {
-    const int ntiles = ((p.npx + TX - 1) / TX) * ((p.npy + ty - 1) / ty);
-    int nc = (p.npz + 31) / 32;
-    const int need = (2048 + ntiles - 1) / ntiles;     // workgroups to fill the chip
-    if (nc < need) nc = need;
-    int maxc = p.npz / 8;                              // but keep >= 8 planes per chunk
-    if (maxc < 1) maxc = 1;
-    if (nc > maxc) nc = maxc;
-    if (nc < 1) nc = 1;
-    const int kc = (p.npz + nc - 1) / nc;
-    *nchunks = (p.npz + kc - 1) / kc;
-    return kc;
-}
-
 template <int TY, bool MAG, int MODE, bool OPT>
 static hipError_t launch_stage_o(const Params &p, const Metrics &m, const double *qin, double *qout, double *z,
-                                 double *fout, DevScalars *sc, hipStream_t s) {
+                                 double *fout, DevScalars *sc, CflSlots *cs, hipStream_t s) {
     constexpr int lds = stage_lds_bytes<TY, MAG>();
     static std::atomic<unsigned long long> attr{0};
     {
         hipError_t e = lds_limit_once(attr, reinterpret_cast<const void *>(&k_stage<TY, MAG, MODE, OPT>), lds);
         if (e != hipSuccess) return e;
     }
-    int nch;
-    const int kc = chunk_for(p, TY, &nch);
+    const int nch = p.nchunks;
     const int ntiles = ((p.npx + TX - 1) / TX) * ((p.npy + TY - 1) / TY);
-    hipLaunchKernelGGL((k_stage<TY, MAG, MODE, OPT>), dim3(ntiles * nch), dim3(TX * TY), lds, s, p, m, qin, qout,
-                       z, fout, sc, kc);
+    hipLaunchKernelGGL((k_stage<TY, MAG, MODE, OPT>), dim3(ntiles * nch), dim3(TX * TY), lds, s, BoxArgs{p, m, {}},
+                       qin, qout, z, fout, sc, cs, nch);
     return hipGetLastError();
 }
 
 template <int TY, bool MAG, int MODE>
 static hipError_t launch_stage_t(const Params &p, const Metrics &m, const double *qin, double *qout, double *z,
-                                 double *fout, DevScalars *sc, hipStream_t s) {
-    if (p.opt) return launch_stage_o<TY, MAG, MODE, true>(p, m, qin, qout, z, fout, sc, s);
-    return launch_stage_o<TY, MAG, MODE, false>(p, m, qin, qout, z, fout, sc, s);
+                                 double *fout, DevScalars *sc, CflSlots *cs, hipStream_t s) {
+    if (p.opt) return launch_stage_o<TY, MAG, MODE, true>(p, m, qin, qout, z, fout, sc, cs, s);
+    return launch_stage_o<TY, MAG, MODE, false>(p, m, qin, qout, z, fout, sc, cs, s);
 }
 
 template <int TY>
 static hipError_t launch_stage_ty(int mode, const Params &p, const Metrics &m, const double *qin, double *qout,
-                                  double *z, double *fout, DevScalars *sc, hipStream_t s) {
+                                  double *z, double *fout, DevScalars *sc, CflSlots *cs, hipStream_t s) {
     if (p.lmag) {
         switch (mode) {
-            case 0: return launch_stage_t<TY, true, 0>(p, m, qin, qout, z, fout, sc, s);
-            case 1: return launch_stage_t<TY, true, 1>(p, m, qin, qout, z, fout, sc, s);
-            case 2: return launch_stage_t<TY, true, 2>(p, m, qin, qout, z, fout, sc, s);
-            default: return launch_stage_t<TY, true, 3>(p, m, qin, qout, z, fout, sc, s);
+            case 0: return launch_stage_t<TY, true, 0>(p, m, qin, qout, z, fout, sc, cs, s);
+            case 1: return launch_stage_t<TY, true, 1>(p, m, qin, qout, z, fout, sc, cs, s);
+            case 2: return launch_stage_t<TY, true, 2>(p, m, qin, qout, z, fout, sc, cs, s);
+            default: return launch_stage_t<TY, true, 3>(p, m, qin, qout, z, fout, sc, cs, s);
         }
     }
     switch (mode) {
-        case 0: return launch_stage_t<TY, false, 0>(p, m, qin, qout, z, fout, sc, s);
-        case 1: return launch_stage_t<TY, false, 1>(p, m, qin, qout, z, fout, sc, s);
-        case 2: return launch_stage_t<TY, false, 2>(p, m, qin, qout, z, fout, sc, s);
-        default: return launch_stage_t<TY, false, 3>(p, m, qin, qout, z, fout, sc, s);
+        case 0: return launch_stage_t<TY, false, 0>(p, m, qin, qout, z, fout, sc, cs, s);
+        case 1: return launch_stage_t<TY, false, 1>(p, m, qin, qout, z, fout, sc, cs, s);
+        case 2: return launch_stage_t<TY, false, 2>(p, m, qin, qout, z, fout, sc, cs, s);
+        default: return launch_stage_t<TY, false, 3>(p, m, qin, qout, z, fout, sc, cs, s);
     }
 }
 
 hipError_t launch_stage(int mode, const Params &p, const Metrics &m, const double *qin, double *qout,
-                        double *z, double *fout, DevScalars *sc, hipStream_t s) {
-    if (p.tile_y == 8) return launch_stage_ty<8>(mode, p, m, qin, qout, z, fout, sc, s);
-    return launch_stage_ty<4>(mode, p, m, qin, qout, z, fout, sc, s);
+                        double *z, double *fout, DevScalars *sc, CflSlots *cs, hipStream_t s) {
+    if (p.tile_y == 8) return launch_stage_ty<8>(mode, p, m, qin, qout, z, fout, sc, cs, s);
+    return launch_stage_ty<4>(mode, p, m, qin, qout, z, fout, sc, cs, s);
 }
 
 template <int TY, bool MAG, int MODE>
@@ -1005,50 +949,19 @@ hipError_t launch_stage_batch(int mode, int tile_y, int lmag, const BoxDev *boxe
     return launch_batch_ty<4>(mode, lmag, boxes, items, nitems, grid, a, s);
 }
 
-hipError_t launch_bcon_batch(int lmag, const BoxDev *boxes, const ColumnItem *items, int nitems, int a, bool cfl,
-                             hipStream_t s) {
-    dim3 grid(nitems), block(256);
-    if (lmag) {
-        if (cfl) hipLaunchKernelGGL((k_bcon_batch<true, true>), grid, block, 0, s, boxes, items, a);
-        else hipLaunchKernelGGL((k_bcon_batch<true, false>), grid, block, 0, s, boxes, items, a);
-    } else {
-        if (cfl) hipLaunchKernelGGL((k_bcon_batch<false, true>), grid, block, 0, s, boxes, items, a);
-        else hipLaunchKernelGGL((k_bcon_batch<false, false>), grid, block, 0, s, boxes, items, a);
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_cfl_final_batch(const BoxDev *boxes, int nbox, bool clock, hipStream_t s) {
-    hipLaunchKernelGGL(k_cfl_final_batch, dim3((nbox + 63) / 64), dim3(64), 0, s, boxes, nbox, clock ? 1 : 0);
-    return hipGetLastError();
-}
-
-hipError_t launch_bcon(const Params &p, const Metrics &m, const double *qin, double *qout, DevScalars *sc,
-                       bool cfl, hipStream_t s) {
-    const int n = p.npx * p.npy;
-    dim3 grid((n + 255) / 256), block(256);
-    if (p.lmag) {
-        if (cfl) hipLaunchKernelGGL((k_bcon<true, true>), grid, block, 0, s, p, m, qin, qout, sc);
-        else hipLaunchKernelGGL((k_bcon<true, false>), grid, block, 0, s, p, m, qin, qout, sc);
-    } else {
-        if (cfl) hipLaunchKernelGGL((k_bcon<false, true>), grid, block, 0, s, p, m, qin, qout, sc);
-        else hipLaunchKernelGGL((k_bcon<false, false>), grid, block, 0, s, p, m, qin, qout, sc);
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_cfl(const Params &p, const Metrics &m, const double *q, DevScalars *sc, hipStream_t s) {
+hipError_t launch_cfl(const Params &p, const Metrics &m, const double *q, DevScalars *sc, CflSlots *cs,
+                      hipStream_t s) {
     const long long n = (long long)p.npz * p.plane;
     long long nb = (n + 255) / 256;
-    if (nb > 4096) nb = 4096;
+    if (nb > 2048) nb = 2048;
     dim3 grid((unsigned)nb), block(256);
-    if (p.lmag) hipLaunchKernelGGL(k_cfl<true>, grid, block, 0, s, p, m, q, sc);
-    else hipLaunchKernelGGL(k_cfl<false>, grid, block, 0, s, p, m, q, sc);
+    if (p.lmag) hipLaunchKernelGGL(k_cfl<true>, grid, block, 0, s, p, m, q, sc, cs);
+    else hipLaunchKernelGGL(k_cfl<false>, grid, block, 0, s, p, m, q, sc, cs);
     return hipGetLastError();
 }
 
-hipError_t launch_cfl_final(const Params &p, DevScalars *sc, bool clock, hipStream_t s) {
-    hipLaunchKernelGGL(k_cfl_final, dim3(1), dim3(1), 0, s, sc, p.sf, p.lmag, clock ? 1 : 0);
+hipError_t launch_cfl_arm(CflSlots *cs, int n, hipStream_t s) {
+    hipLaunchKernelGGL(k_cfl_arm, dim3(n), dim3(64), 0, s, cs);
     return hipGetLastError();
 }
 

@@ -81,7 +81,7 @@ __host__ __device__ __forceinline__ double pprime(double r0, double t0, double r
 //   min 0.375 dd^2 RE rho        = 0.375 RE min(rho dd^2)
 //   min 0.5 dd^2 RM              = 0.5 RM min(dd^2)
 // (U the fast-mode speed squared of sub:750-856).  The workgroup converts
-// back once and updates the same keys as cfl_reduce.  NaN sticks.
+// back once and publishes the same keys as cfl_reduce.  NaN sticks.
 struct CflFast {
     double mach, q1, s2, s3, d2;
 };
@@ -120,7 +120,8 @@ __device__ __forceinline__ DdPair ddpair(double ddx, double ddy, double ddz) {
 
 // d2extra: a min(dd^2) contribution computed elsewhere (the grid-only term
 // of the stage kernel, which does not reduce it per point).
-__device__ void cflf_reduce(const Params &p, CflFast c, DevScalars *__restrict__ sc, double d2extra = INFINITY) {
+__device__ void cflf_reduce(const Params &p, CflFast c, int clock, DevScalars *__restrict__ sc,
+                            CflSlots *__restrict__ cs, int seq, int total, double d2extra = INFINITY) {
     __shared__ double red[16][5];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -135,7 +136,7 @@ __device__ void cflf_reduce(const Params &p, CflFast c, DevScalars *__restrict__
         red[wv][0] = c.mach; red[wv][1] = c.q1; red[wv][2] = c.s2; red[wv][3] = c.s3; red[wv][4] = c.d2;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (threadIdx.x < 64) {
         for (int v = 1; v < nw; ++v) {
             c.mach = nmax(c.mach, red[v][0]);
             c.q1 = nmax(c.q1, red[v][1]);
@@ -145,12 +146,11 @@ __device__ void cflf_reduce(const Params &p, CflFast c, DevScalars *__restrict__
         }
         c.d2 = nmin(c.d2, d2extra);
         const double w[4] = {1.0 / sqrt(c.q1), 0.5 * p.repr * p.cv * c.s2, 0.375 * p.re * c.s3, 0.5 * p.rm * c.d2};
-        key_raise(&sc->key_mach, dkey(c.mach));
-        for (int n = 0; n < 4; ++n) {
-            if (n == 3 && !p.lmag) break;
-            // a NaN limit becomes -NaN for the min reduction
-            key_lower(&sc->key_min[n], (w[n] == w[n]) ? dkey(w[n]) : 0ull);
-        }
+        unsigned long long k[CFL_KEYS];
+        k[0] = ~dkey(c.mach);
+        // a NaN limit becomes -NaN for the min reduction
+        for (int n = 0; n < 4; ++n) k[n + 1] = (w[n] == w[n]) ? dkey(w[n]) : 0ull;
+        cfl_publish(k, sc, cs, p.sf, p.lmag, clock, seq, total);
     }
 }
 
@@ -164,6 +164,78 @@ __device__ __forceinline__ void load_rawf(const float *__restrict__ q, long long
     for (int f = 0; f < (MAG ? 8 : 5); ++f) r.v[f] = q[f * fs + off];
 }
 
+// BCON of the mixed form on the boundary planes (top: plane 1, bot: plane
+// npz) of one column, in FP64 on the full state bg + value (+ R after the
+// last stage, where R holds the rounding residual); called by the stage
+// workgroup that owns the column and the planes (see bcon_column of the FP64
+// form).  New boundary values are split again into stored values and the
+// residual (D after stages 1-2, R after stage 3); a new boundary temperature
+// is stored as the P' of the plane's stored rho'.  LAST also accumulates the
+// boundary planes' CFL limits.
+template <bool MAG, bool LAST>
+__device__ __forceinline__ void bcon_column_m(const Params &p, const Metrics &m, const Background &bg, float *h,
+                                              float *dr, unsigned *rr, int i, int j, bool top, bool bot,
+                                              CflFast &cfl) {
+    const long long fs = p.fsize, pl = p.plane, idx = (long long)j * p.npx + i;
+    const int nz = p.npz;
+    const double C13 = p.c13, C23 = p.c23, C43 = p.c43;
+    auto full = [&](int f, int k) -> double {
+        const long long o = f * fs + (long long)k * pl + idx;
+        double v = f == 4 ? (double)trep(bg.ro32[k], bg.tt32[k], h[o - fs], h[o]) : (double)h[o];
+        if (LAST) v += (double)r_get(rr, fs, f, (long long)k * pl + idx);
+        if (f == 3) v += bg.ro[k];
+        if (f == 4) v += bg.tt[k];
+        return v;
+    };
+    auto residual = [&](int f, int k, double r) {
+        if (LAST) r_put(rr, fs, f, (long long)k * pl + idx, (float)r);
+        else dr[f * fs + (long long)k * pl + idx] = (float)r;
+    };
+    auto put = [&](int f, int k, double v) {
+        const long long o = f * fs + (long long)k * pl + idx;
+        if (f == 4) {
+            const double tp = v - bg.tt[k];
+            const float rh = h[o - fs];
+            const double rhx = LAST ? (double)rh + (double)r_get(rr, fs, 3, (long long)k * pl + idx) : (double)rh;
+            const float hp = (float)pprime(bg.ro[k], bg.tt[k], rhx, tp);
+            h[o] = hp;
+            residual(4, k, tp - (double)trep(bg.ro32[k], bg.tt32[k], rh, hp));
+            return;
+        }
+        if (f == 3) v -= bg.ro[k];
+        const float hn = (float)v;
+        h[o] = hn;
+        residual(f, k, v - (double)hn);
+    };
+#pragma unroll 1
+    for (int side = 0; side < 2; ++side) {
+        if (side ? !bot : !top) continue;
+        const int a = side ? nz : 1, b = side ? nz - 1 : 2, c = side ? nz - 2 : 3;
+        const double roa = full(3, a), rob = full(3, b), roc = full(3, c);
+        put(0, a, roa * (C43 * full(0, b) / rob - C13 * full(0, c) / roc));
+        put(1, a, roa * (C43 * full(1, b) / rob - C13 * full(1, c) / roc));
+        put(2, a, 0.0);
+        const int code = side ? p.izc : p.itc;
+        double tnew;
+        if (code == 0) {
+            tnew = side ? p.tb : 1.0;
+        } else {
+            const double dz = p.dzf / m.dzzdz[a];
+            tnew = side ? C43 * full(4, b) - C13 * full(4, c) + C23 * dz * p.theta / m.rkapa[a]
+                        : C43 * full(4, b) - C13 * full(4, c) - C23 * dz * p.theta;
+        }
+        put(4, a, tnew);
+        if (MAG && p.ibc == 0) put(7, a, 0.0);
+        if (LAST) {
+            double v[8];
+#pragma unroll
+            for (int f = 0; f < (MAG ? 8 : 5); ++f) v[f] = full(f, a);
+            const DdPair d = ddpair(m.ddx[i + 1], m.ddy[j + 1], m.ddz[a]);
+            cflf_point<MAG>(p, v, d.dd2, d.idd2, 1.0 / m.rkapa[a], cfl);
+        }
+    }
+}
+
 // One tile column chunk of mixed stage s = MODE (1..3); see stage_tile of
 // the FP64 form for the tile organisation.
 // Per-plane values (z metrics, background, coefficients) from the
@@ -173,11 +245,11 @@ __device__ __forceinline__ void load_rawf(const float *__restrict__ q, long long
 #define PLP(F, K) uload(&bg.planes[K].F, 0)
 
 template <int TY, bool MAG, int MODE, int TXW = MTX>
-__device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, const Background &bg,
+__device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, const Background &bg, ArgPtr args,
                                              const float *__restrict__ hin, float *__restrict__ hout,
                                              float *__restrict__ dr, unsigned *__restrict__ rr,
-                                             DevScalars *__restrict__ sc, int i0, int j0, int kbeg, int kend,
-                                             float *ldsf) {
+                                             DevScalars *__restrict__ sc, CflSlots *__restrict__ cs, int i0, int j0,
+                                             int kbeg, int kend, int seq, int total, float *ldsf) {
     using T = MTile<TXW, TY>;
     constexpr int SW = T::SW, SP = T::SP;
     constexpr int NF = MAG ? 8 : 5;
@@ -220,22 +292,30 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
         ring(k, 3, pt) = trep(PLB(ro32, k), PLB(tt32, k), r.v[3], r.v[4]);  // temperature perturbation
     };
 
+    // warm-up: planes kbeg-1 .. kbeg+1, every load issued before the first is
+    // used (lanes without a halo point re-read their own)
     RawF rm_, rp_o, rp_h;
-    load_rawf<MAG>(hin, fs, (long long)(kbeg - 1) * pl + ooff, rm_);
-    put_ring(kbeg - 1, opt, rm_);
-    if (has_h) {
-        load_rawf<MAG>(hin, fs, (long long)(kbeg - 1) * pl + hoff, rp_h);
-        put_ring(kbeg - 1, hpt, rp_h);
-    }
-#pragma unroll 1
-    for (int kk = kbeg; kk <= kbeg + 1; ++kk) {
-        load_rawf<MAG>(hin, fs, (long long)kk * pl + ooff, rp_o);
-        put_cur(kk, opt, rp_o);
-        put_ring(kk, opt, rp_o);
+    {
+        RawF ro_[2], rh_[3];
+        const long long ho = has_h ? hoff : ooff;
+        load_rawf<MAG>(hin, fs, (long long)(kbeg - 1) * pl + ooff, rm_);
+#pragma unroll
+        for (int n = 0; n < 2; ++n) load_rawf<MAG>(hin, fs, (long long)(kbeg + n) * pl + ooff, ro_[n]);
+#pragma unroll
+        for (int n = 0; n < 3; ++n) load_rawf<MAG>(hin, fs, (long long)(kbeg - 1 + n) * pl + ho, rh_[n]);
+        put_ring(kbeg - 1, opt, rm_);
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            put_cur(kbeg + n, opt, ro_[n]);
+            put_ring(kbeg + n, opt, ro_[n]);
+        }
         if (has_h) {
-            load_rawf<MAG>(hin, fs, (long long)kk * pl + hoff, rp_h);
-            put_cur(kk, hpt, rp_h);
-            put_ring(kk, hpt, rp_h);
+            put_ring(kbeg - 1, hpt, rh_[0]);
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {
+                put_cur(kbeg + n, hpt, rh_[n + 1]);
+                put_ring(kbeg + n, hpt, rh_[n + 1]);
+            }
         }
     }
 
@@ -540,29 +620,32 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
         if (k == 1 || k == npz) plane(k, std::true_type{});
         else plane(k, std::false_type{});
     }
+    if ((kbeg == 1 || kend == npz) && valid) {
+        const BoxArgs &l = late_args(args);
+        bcon_column_m<MAG, MODE == 3>(l.p, l.m, l.bg, hout, dr, rr, gi, gj, kbeg == 1, kend == npz, cfl_acc);
+    }
     if (MODE == 3) {
         // min(dd^2) depends on the grid only: its minimum over all points
         // comes with the metrics
-        cflf_reduce(p, CflFast{cfl_acc.mach, cfl_acc.q1, cfl_acc.s2, cfl_acc.s3, INFINITY}, sc,
+        cflf_reduce(late_args(args).p, CflFast{cfl_acc.mach, cfl_acc.q1, cfl_acc.s2, cfl_acc.s3, INFINITY}, 1, sc, cs, seq, total,
                     MAG ? sc->dd2min : INFINITY);
     }
 }
 
 template <int TY, bool MAG, int MODE>
-__global__ __launch_bounds__(MTX *TY, 3) void k_stage_m(const Params p, const Metrics m, const Background bg,
+__global__ __launch_bounds__(MTX *TY, 3) void k_stage_m(const BoxArgs b,
                                                      const float *__restrict__ hin, float *__restrict__ hout,
                                                      float *__restrict__ dr, unsigned *__restrict__ rr,
-                                                     DevScalars *__restrict__ sc, int kchunk) {
+                                                     DevScalars *__restrict__ sc, CflSlots *__restrict__ cs,
+                                                     int nchunks) {
     extern __shared__ float ldsf[];
+    const Params &p = b.p;
     const int ntx = (p.npx + MTX - 1) / MTX, nty = (p.npy + TY - 1) / TY;
-    const int bid = xcd_remap(blockIdx.x, gridDim.x);
-    const int tz = bid / (ntx * nty);
-    const int rem = bid - tz * (ntx * nty);
-    const int tyb = rem / ntx, txb = rem - tyb * ntx;
-    const int kbeg = 1 + tz * kchunk;
-    const int kend = min(p.npz, kbeg + kchunk - 1);
-    if (kbeg > p.npz) return;
-    stage_tile_m<TY, MAG, MODE>(p, m, bg, hin, hout, dr, rr, sc, txb * MTX, tyb * TY, kbeg, kend, ldsf);
+    const TileChunk tc = tile_of(blockIdx.x, ntx * nty, nchunks);
+    const int tz = tc.chunk, tyb = tc.tile / ntx, txb = tc.tile - tyb * ntx;
+    const int kbeg = chunk_begin(p.npz, nchunks, tz), kend = chunk_begin(p.npz, nchunks, tz + 1) - 1;
+    stage_tile_m<TY, MAG, MODE>(p, b.m, b.bg, kernel_args(), hin, hout, dr, rr, sc, cs, txb * MTX, tyb * TY, kbeg, kend,
+                                blockIdx.x, gridDim.x, ldsf);
 }
 
 // Ensemble: persistent grid over the work items of all boxes (static stride);
@@ -574,109 +657,18 @@ __global__ __launch_bounds__(TXW *TY, 3) void k_stage_m_batch(const BoxDev *__re
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
     for (int w = slot; w < nitems; w += gridDim.x) {
         const StageItem it = items[w];
-        const BoxDev &B = boxes[it.box];
+        const BoxDev &B = box_at(boxes, it.box);
         __syncthreads();  // the previous item's last LDS reads are done
-        stage_tile_m<TY, MAG, MODE, TXW>(B.p, B.m, B.bg, B.h[a], B.h[1 - a], B.dr, B.rr, B.sc, it.i0, it.j0, it.kbeg,
-                                    it.kend, ldsf);
+        stage_tile_m<TY, MAG, MODE, TXW>(B.a.p, B.a.m, B.a.bg, (ArgPtr)&B.a, B.h[a], B.h[1 - a], B.dr, B.rr, B.sc, B.cs, it.i0, it.j0,
+                                         it.kbeg, it.kend, it.seq, it.total, ldsf);
     }
-}
-
-// BCON of the mixed form, in FP64 on the full state bg + value (+ R after
-// the last stage, where R holds the rounding residual).  New boundary
-// values are split again into stored values and the residual (D after
-// stages 1-2, R after stage 3); a new boundary temperature is stored as the
-// P' of the plane's stored rho'.
-template <bool MAG, bool LAST>
-__device__ __forceinline__ void bcon_column_m(const Params &p, const Metrics &m, const Background &bg,
-                                              float *__restrict__ h, float *__restrict__ dr,
-                                              unsigned *__restrict__ rr, DevScalars *__restrict__ sc,
-                                              int idx) {
-    CflFast cfl = cflf_init();
-    if (idx < p.npx * p.npy) {
-        const long long fs = p.fsize, pl = p.plane;
-        const int nz = p.npz;
-        const double C13 = p.c13, C23 = p.c23, C43 = p.c43;
-        auto full = [&](int f, int k) -> double {
-            const long long o = f * fs + (long long)k * pl + idx;
-            double v = f == 4 ? (double)trep(bg.ro32[k], bg.tt32[k], h[o - fs], h[o]) : (double)h[o];
-            if (LAST) v += (double)r_get(rr, fs, f, (long long)k * pl + idx);
-            if (f == 3) v += bg.ro[k];
-            if (f == 4) v += bg.tt[k];
-            return v;
-        };
-        auto residual = [&](int f, int k, double r) {
-            if (LAST) r_put(rr, fs, f, (long long)k * pl + idx, (float)r);
-            else dr[f * fs + (long long)k * pl + idx] = (float)r;
-        };
-        auto put = [&](int f, int k, double v) {
-            const long long o = f * fs + (long long)k * pl + idx;
-            if (f == 4) {
-                const double tp = v - bg.tt[k];
-                const float rh = h[o - fs];
-                const double rhx = LAST ? (double)rh + (double)r_get(rr, fs, 3, (long long)k * pl + idx) : (double)rh;
-                const float hp = (float)pprime(bg.ro[k], bg.tt[k], rhx, tp);
-                h[o] = hp;
-                residual(4, k, tp - (double)trep(bg.ro32[k], bg.tt32[k], rh, hp));
-                return;
-            }
-            if (f == 3) v -= bg.ro[k];
-            const float hn = (float)v;
-            h[o] = hn;
-            residual(f, k, v - (double)hn);
-        };
-        for (int side = 0; side < 2; ++side) {
-            const int a = side ? nz : 1, b = side ? nz - 1 : 2, c = side ? nz - 2 : 3;
-            const double roa = full(3, a), rob = full(3, b), roc = full(3, c);
-            put(0, a, roa * (C43 * full(0, b) / rob - C13 * full(0, c) / roc));
-            put(1, a, roa * (C43 * full(1, b) / rob - C13 * full(1, c) / roc));
-            put(2, a, 0.0);
-            const int code = side ? p.izc : p.itc;
-            double tnew;
-            if (code == 0) {
-                tnew = side ? p.tb : 1.0;
-            } else {
-                const double dz = p.dzf / m.dzzdz[a];
-                tnew = side ? C43 * full(4, b) - C13 * full(4, c) + C23 * dz * p.theta / m.rkapa[a]
-                            : C43 * full(4, b) - C13 * full(4, c) - C23 * dz * p.theta;
-            }
-            put(4, a, tnew);
-            if (MAG && p.ibc == 0) put(7, a, 0.0);
-        }
-        if (LAST) {
-            const int j = idx / p.npx, i = idx - j * p.npx;
-            for (int side = 0; side < 2; ++side) {
-                const int k = side ? nz : 1;
-                double v[8];
-                for (int f = 0; f < (MAG ? 8 : 5); ++f) v[f] = full(f, k);
-                const DdPair d = ddpair(m.ddx[i + 1], m.ddy[j + 1], m.ddz[k]);
-                cflf_point<MAG>(p, v, d.dd2, d.idd2, 1.0 / m.rkapa[k], cfl);
-            }
-        }
-    }
-    if (LAST) cflf_reduce(p, cfl, sc);
-}
-
-template <bool MAG, bool LAST>
-__global__ __launch_bounds__(256) void k_bcon_m(const Params p, const Metrics m, const Background bg,
-                                                float *__restrict__ h, float *__restrict__ dr,
-                                                unsigned *__restrict__ rr, DevScalars *__restrict__ sc) {
-    bcon_column_m<MAG, LAST>(p, m, bg, h, dr, rr, sc, blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-// Ensemble: one workgroup per (box, run of 256 columns) of register 1-a.
-template <bool MAG, bool LAST>
-__global__ __launch_bounds__(256) void k_bcon_m_batch(const BoxDev *__restrict__ boxes,
-                                                      const ColumnItem *__restrict__ items, int a) {
-    const ColumnItem it = items[blockIdx.x];
-    const BoxDev &B = boxes[it.box];
-    bcon_column_m<MAG, LAST>(B.p, B.m, B.bg, B.h[1 - a], B.dr, B.rr, B.sc, it.col0 + threadIdx.x);
 }
 
 // Stand-alone CFL of the mixed state (first step after an upload).
 template <bool MAG>
 __global__ __launch_bounds__(256) void k_cfl_m(const Params p, const Metrics m, const Background bg,
                                                const float *__restrict__ h, const unsigned *__restrict__ rr,
-                                               DevScalars *__restrict__ sc) {
+                                               DevScalars *__restrict__ sc, CflSlots *__restrict__ cs) {
     const long long fs = p.fsize, pl = p.plane;
     const long long n = (long long)p.npz * pl;
     CflFast cfl = cflf_init();
@@ -696,7 +688,7 @@ __global__ __launch_bounds__(256) void k_cfl_m(const Params p, const Metrics m, 
         const DdPair d = ddpair(m.ddx[i + 1], m.ddy[j + 1], m.ddz[k]);
         cflf_point<MAG>(p, v, d.dd2, d.idd2, 1.0 / m.rkapa[k], cfl);
     }
-    cflf_reduce(p, cfl, sc);
+    cflf_reduce(p, cfl, 0, sc, cs, blockIdx.x, gridDim.x);
 }
 
 // padded FP64 field f -> (stored value, R = rounding residual) in the
@@ -822,80 +814,48 @@ __global__ void k_closure_forcing(const Params p, const float *__restrict__ y, c
 
 // ---------------------------------------------------------------------------
 
-// z chunks of about 32 planes (the tiles of a co-resident cohort stay closer
-// in step over a short march: 512x512x256, 8 chunks 1% faster than 4), at
-// least 4096 workgroups, at least 8 planes.
-static int chunk_m(const Params &p, int ty, int *nchunks) {
-    const int ntiles = ((p.npx + MTX - 1) / MTX) * ((p.npy + ty - 1) / ty);
-    int nc = (p.npz + 31) / 32;
-    const int need = (4096 + ntiles - 1) / ntiles;
-    if (nc < need) nc = need;
-    int maxc = p.npz / 8;
-    if (maxc < 1) maxc = 1;
-    if (nc > maxc) nc = maxc;
-    if (nc < 1) nc = 1;
-    const int kc = (p.npz + nc - 1) / nc;
-    *nchunks = (p.npz + kc - 1) / kc;
-    return kc;
-}
-
 template <int TY, bool MAG, int MODE>
 static hipError_t launch_m(const Params &p, const Metrics &m, const Background &bg, const float *hin, float *hout,
-                           float *dr, unsigned *rr, DevScalars *sc, hipStream_t s) {
+                           float *dr, unsigned *rr, DevScalars *sc, CflSlots *cs, hipStream_t s) {
     constexpr int lds = mixed_lds_bytes<TY, MAG, MODE>();
     static std::atomic<unsigned long long> attr{0};
     {
         hipError_t e = lds_limit_once(attr, reinterpret_cast<const void *>(&k_stage_m<TY, MAG, MODE>), lds);
         if (e != hipSuccess) return e;
     }
-    int nch;
-    const int kc = chunk_m(p, TY, &nch);
+    const int nch = p.nchunks;
     const int ntiles = ((p.npx + MTX - 1) / MTX) * ((p.npy + TY - 1) / TY);
-    hipLaunchKernelGGL((k_stage_m<TY, MAG, MODE>), dim3(ntiles * nch), dim3(MTX * TY), lds, s, p, m, bg, hin, hout,
-                       dr, rr, sc, kc);
+    hipLaunchKernelGGL((k_stage_m<TY, MAG, MODE>), dim3(ntiles * nch), dim3(MTX * TY), lds, s, BoxArgs{p, m, bg}, hin, hout,
+                       dr, rr, sc, cs, nch);
     return hipGetLastError();
 }
 
 template <int TY>
 static hipError_t launch_m_ty(int mode, const Params &p, const Metrics &m, const Background &bg, const float *hin,
-                              float *hout, float *dr, unsigned *rr, DevScalars *sc, hipStream_t s) {
+                              float *hout, float *dr, unsigned *rr, DevScalars *sc, CflSlots *cs, hipStream_t s) {
     if (p.lmag) {
-        if (mode == 1) return launch_m<TY, true, 1>(p, m, bg, hin, hout, dr, rr, sc, s);
-        if (mode == 2) return launch_m<TY, true, 2>(p, m, bg, hin, hout, dr, rr, sc, s);
-        return launch_m<TY, true, 3>(p, m, bg, hin, hout, dr, rr, sc, s);
+        if (mode == 1) return launch_m<TY, true, 1>(p, m, bg, hin, hout, dr, rr, sc, cs, s);
+        if (mode == 2) return launch_m<TY, true, 2>(p, m, bg, hin, hout, dr, rr, sc, cs, s);
+        return launch_m<TY, true, 3>(p, m, bg, hin, hout, dr, rr, sc, cs, s);
     }
-    if (mode == 1) return launch_m<TY, false, 1>(p, m, bg, hin, hout, dr, rr, sc, s);
-    if (mode == 2) return launch_m<TY, false, 2>(p, m, bg, hin, hout, dr, rr, sc, s);
-    return launch_m<TY, false, 3>(p, m, bg, hin, hout, dr, rr, sc, s);
+    if (mode == 1) return launch_m<TY, false, 1>(p, m, bg, hin, hout, dr, rr, sc, cs, s);
+    if (mode == 2) return launch_m<TY, false, 2>(p, m, bg, hin, hout, dr, rr, sc, cs, s);
+    return launch_m<TY, false, 3>(p, m, bg, hin, hout, dr, rr, sc, cs, s);
 }
 
 hipError_t launch_stage_mixed(int mode, const Params &p, const Metrics &m, const Background &bg, const float *hin,
-                              float *hout, float *dr, unsigned *rr, DevScalars *sc, hipStream_t s) {
-    if (p.tile_y == 8) return launch_m_ty<8>(mode, p, m, bg, hin, hout, dr, rr, sc, s);
-    return launch_m_ty<4>(mode, p, m, bg, hin, hout, dr, rr, sc, s);
-}
-
-hipError_t launch_bcon_mixed(const Params &p, const Metrics &m, const Background &bg, float *h, float *dr,
-                             unsigned *rr, DevScalars *sc, bool last, hipStream_t s) {
-    const int n = p.npx * p.npy;
-    dim3 grid((n + 255) / 256), block(256);
-    if (p.lmag) {
-        if (last) hipLaunchKernelGGL((k_bcon_m<true, true>), grid, block, 0, s, p, m, bg, h, dr, rr, sc);
-        else hipLaunchKernelGGL((k_bcon_m<true, false>), grid, block, 0, s, p, m, bg, h, dr, rr, sc);
-    } else {
-        if (last) hipLaunchKernelGGL((k_bcon_m<false, true>), grid, block, 0, s, p, m, bg, h, dr, rr, sc);
-        else hipLaunchKernelGGL((k_bcon_m<false, false>), grid, block, 0, s, p, m, bg, h, dr, rr, sc);
-    }
-    return hipGetLastError();
+                              float *hout, float *dr, unsigned *rr, DevScalars *sc, CflSlots *cs, hipStream_t s) {
+    if (p.tile_y == 8) return launch_m_ty<8>(mode, p, m, bg, hin, hout, dr, rr, sc, cs, s);
+    return launch_m_ty<4>(mode, p, m, bg, hin, hout, dr, rr, sc, cs, s);
 }
 
 hipError_t launch_cfl_mixed(const Params &p, const Metrics &m, const Background &bg, const float *h,
-                            const unsigned *rr, DevScalars *sc, hipStream_t s) {
+                            const unsigned *rr, DevScalars *sc, CflSlots *cs, hipStream_t s) {
     const long long n = (long long)p.npz * p.plane;
     long long nb = (n + 255) / 256;
-    if (nb > 4096) nb = 4096;
-    if (p.lmag) hipLaunchKernelGGL(k_cfl_m<true>, dim3((unsigned)nb), dim3(256), 0, s, p, m, bg, h, rr, sc);
-    else hipLaunchKernelGGL(k_cfl_m<false>, dim3((unsigned)nb), dim3(256), 0, s, p, m, bg, h, rr, sc);
+    if (nb > 2048) nb = 2048;
+    if (p.lmag) hipLaunchKernelGGL(k_cfl_m<true>, dim3((unsigned)nb), dim3(256), 0, s, p, m, bg, h, rr, sc, cs);
+    else hipLaunchKernelGGL(k_cfl_m<false>, dim3((unsigned)nb), dim3(256), 0, s, p, m, bg, h, rr, sc, cs);
     return hipGetLastError();
 }
 
@@ -960,19 +920,6 @@ hipError_t launch_stage_batch_mixed(int mode, int tile_x, int tile_y, int lmag, 
     if (tile_x == 32) return launch_mb_ty<8, 32>(mode, lmag, boxes, items, nitems, grid, a, s);
     if (tile_y == 8) return launch_mb_ty<8, MTX>(mode, lmag, boxes, items, nitems, grid, a, s);
     return launch_mb_ty<4, MTX>(mode, lmag, boxes, items, nitems, grid, a, s);
-}
-
-hipError_t launch_bcon_batch_mixed(int lmag, const BoxDev *boxes, const ColumnItem *items, int nitems, int a,
-                                   bool last, hipStream_t s) {
-    dim3 grid(nitems), block(256);
-    if (lmag) {
-        if (last) hipLaunchKernelGGL((k_bcon_m_batch<true, true>), grid, block, 0, s, boxes, items, a);
-        else hipLaunchKernelGGL((k_bcon_m_batch<true, false>), grid, block, 0, s, boxes, items, a);
-    } else {
-        if (last) hipLaunchKernelGGL((k_bcon_m_batch<false, true>), grid, block, 0, s, boxes, items, a);
-        else hipLaunchKernelGGL((k_bcon_m_batch<false, false>), grid, block, 0, s, boxes, items, a);
-    }
-    return hipGetLastError();
 }
 
 hipError_t launch_closure_inputs(const Params &p, const Background &bg, const float *h, const unsigned *rr,

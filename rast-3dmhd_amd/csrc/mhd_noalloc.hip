@@ -6,14 +6,16 @@
 // mhd_create).  Here they live in one file-scope device array, `scratch`,
 // of NOALLOC_BYTES per GPU:
 //
-//   [0, 256)             DevScalars (reduction keys, DT, clock)
+//   [0, 256)             DevScalars (DT, clock)
 //   [256, 256 + 3*R)     q[0], q[1], Z; R = nf * fsize doubles each (fsize
 //                        the field stride of Params, padding included)
+//
+// The CFL reduction slots are a second small array, `slots`.
 //
 // On the host the name `scratch` stands for no device address: its address
 // on each device is looked up once per device with hipGetSymbolAddress and
 // only that pointer is passed to kernels.  Every call re-initialises the
-// scalars with a one-thread kernel and overwrites the registers completely
+// scalars and slots with a one-wavefront kernel and overwrites the registers completely
 // (pack of every field, z ghost planes included), so no content of an
 // earlier call is read.  Calls that overlap on one GPU share the array and
 // race.
@@ -28,6 +30,7 @@
 #include <mutex>
 
 #include "../../include/rast3dmhd.h"
+#include "mhd_device.h"
 #include "mhd_host.h"
 
 using namespace rmhd;
@@ -39,25 +42,31 @@ constexpr size_t SCALARS_BYTES = 256;
 static_assert(sizeof(DevScalars) <= SCALARS_BYTES, "DevScalars fits its 256-byte slot");
 
 __device__ __align__(256) unsigned char scratch[NOALLOC_BYTES];
+__device__ CflSlots slots;
 
 constexpr int MAX_DEV = 64;
 std::mutex g_mu;
-void *g_scratch[MAX_DEV];  // device address of `scratch` per device (null: not looked up yet)
+// device addresses of `scratch` and `slots` per device (null: not looked up yet)
+void *g_scratch[MAX_DEV], *g_slots[MAX_DEV];
 
-__global__ void k_noalloc_init(DevScalars *sc, DevScalars s0) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *sc = s0;
+__global__ __launch_bounds__(64) void k_noalloc_init(DevScalars *sc, DevScalars s0, CflSlots *cs) {
+    if (threadIdx.x == 0) *sc = s0;
+    cfl_arm(cs, threadIdx.x);
 }
 
-// Device address of this device's scratch array (dev is current).
-hipError_t scratch_ptr(int dev, unsigned char **out) {
+// Device addresses of this device's scratch array and slots (dev is current).
+hipError_t scratch_ptr(int dev, unsigned char **out, CflSlots **cs) {
     std::lock_guard<std::mutex> lock(g_mu);
     if (!g_scratch[dev]) {
-        void *p = nullptr;
-        const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+        void *p = nullptr, *q = nullptr;
+        hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+        if (e == hipSuccess) e = hipGetSymbolAddress(&q, HIP_SYMBOL(slots));
         if (e != hipSuccess) return e;
         g_scratch[dev] = p;
+        g_slots[dev] = q;
     }
     *out = static_cast<unsigned char *>(g_scratch[dev]);
+    *cs = static_cast<CflSlots *>(g_slots[dev]);
     return hipSuccess;
 }
 
@@ -102,7 +111,8 @@ extern "C" int mhd_step_noalloc(const mhd_desc *d, const mhd_dev_metrics *met, d
     NACHK(hipGetDevice(&dev));
     if (dev < 0 || dev >= MAX_DEV) return global_fail(MHD_ERR_HIP, "mhd_step_noalloc: device %d", dev);
     unsigned char *base = nullptr;
-    NACHK(scratch_ptr(dev, &base));
+    CflSlots *cs = nullptr;
+    NACHK(scratch_ptr(dev, &base, &cs));
     DevScalars *sc = reinterpret_cast<DevScalars *>(base);
     double *q[2] = {reinterpret_cast<double *>(base + SCALARS_BYTES),
                     reinterpret_cast<double *>(base + SCALARS_BYTES) + reg};
@@ -116,13 +126,13 @@ extern "C" int mhd_step_noalloc(const mhd_desc *d, const mhd_dev_metrics *met, d
     m.rkapa = met->rkapa; m.dkapa = met->dkapa;
     m.rkcfl = met->rkapa;
 
-    // scalars: keys armed, the caller's clock
+    // scalars (the caller's clock), slots armed
     DevScalars s0 = initial_scalars();
     s0.nit = *nit;
     s0.timc = *timc;
     s0.timi = timi;
     s0.timt = timi + *timc;
-    hipLaunchKernelGGL(k_noalloc_init, dim3(1), dim3(64), 0, s, sc, s0);
+    hipLaunchKernelGGL(k_noalloc_init, dim3(1), dim3(64), 0, s, sc, s0, cs);
     NACHK(hipGetLastError());
     // upload: both registers carry the z ghost planes (as mhd_upload)
     for (int f = 0; f < nf; ++f) {
@@ -130,17 +140,14 @@ extern "C" int mhd_step_noalloc(const mhd_desc *d, const mhd_dev_metrics *met, d
         NACHK(launch_pack(p, state[f], q[1] + (size_t)f * p.fsize, s));
     }
     // step (as mhd_step on a freshly uploaded handle)
-    NACHK(launch_cfl(p, m, q[0], sc, s));
-    NACHK(launch_cfl_final(p, sc, false, s));
+    NACHK(launch_cfl(p, m, q[0], sc, cs, s));
     int a = 0, b = 1;
     for (int st = 1; st <= 3; ++st) {
-        NACHK(launch_stage(st, p, m, q[a], q[b], z, nullptr, sc, s));
-        NACHK(launch_bcon(p, m, q[a], q[b], sc, st == 3, s));
+        NACHK(launch_stage(st, p, m, q[a], q[b], z, nullptr, sc, cs, s));
         const int t = a;
         a = b;
         b = t;
     }
-    NACHK(launch_cfl_final(p, sc, true, s));
     // download into the caller's arrays (as mhd_download), register a holds the result
     for (int f = 0; f < nf; ++f) NACHK(launch_unpack(p, q[a] + (size_t)f * p.fsize, state[f], 1, s));
     DevScalars out;
