@@ -47,12 +47,15 @@ struct mhd_ctx {
     double *prof = nullptr;             // mixed: plane means for mhd_rebase [3][npz]
     int rebase_every = 0, since_rebase = 0;
     double *f = nullptr;                // right-hand side (mhd_fluxes only)
-    double *stage = nullptr;            // one padded field for host transfers
+    double *stage = nullptr;            // padded fields for host transfers
+    int stage_n = 1;                    // how many
+    double *out = nullptr;              // results of box_filter and flux_profiles
+    size_t out_bytes = 0;
     double *met = nullptr;              // 11 metric arrays
     Metrics m{};
     std::vector<double> dzzdz, d2zzdz2, ddz, rkapa, dkapa;  // host copies for the background
     DevScalars *sc = nullptr;
-    CflSlots *cs = nullptr;             // CFL reduction slots
+    CflSlots *cs = nullptr;             // CFL reduction slots (after sc)
     // closure-corrected step (mixed form)
     mhd_net_t *net = nullptr;
     float *force = nullptr;    // [7][fsize]
@@ -114,10 +117,22 @@ static void free_all(mhd_t *h) {
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     void *bufs[26] = {h->q[0], h->q[1], h->z, h->hq[0], h->hq[1], h->dr, h->rr, h->bgd, h->bgf, h->bgp,
                       h->f, h->stage, h->met, h->sc, h->force, h->force_on, h->cx, h->nrm,
-                      h->optmem, h->rs, h->ftacc, h->bgd2, h->bgf2, h->bgp2, h->prof, h->cs};
+                      h->optmem, h->rs, h->ftacc, h->bgd2, h->bgf2, h->bgp2, h->prof, h->out};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (h->stream) (void)hipStreamDestroy(h->stream);
+    copy_release();
+}
+
+// The handle's result buffer with room for bytes (kept; freed with the handle).
+static hipError_t result_buffer(mhd_t *h, size_t bytes) {
+    if (bytes <= h->out_bytes) return hipSuccess;
+    if (h->out) (void)hipFree(h->out);
+    h->out = nullptr;
+    h->out_bytes = 0;
+    const hipError_t e = hipMalloc(&h->out, bytes);
+    if (e == hipSuccess) h->out_bytes = bytes;
+    return e;
 }
 
 // Device buffers of the optional branches: the per-plane and per-axis tables
@@ -179,6 +194,7 @@ extern "C" int mhd_create(const mhd_desc *d, mhd_t **out) {
         delete h;
         return rc;
     }
+    copy_retain();  // given back by free_all
     const int nf = p.lmag ? 8 : 5;
     const size_t pbytes = (size_t)(d->npx + 2) * (d->npy + 2) * (d->npz + 2) * sizeof(double);
     const size_t nzp = (size_t)d->npz + 2;
@@ -198,10 +214,12 @@ extern "C" int mhd_create(const mhd_desc *d, mhd_t **out) {
         if (e == hipSuccess) e = hipMalloc(&h->bgf, BG_FLT * nzp * sizeof(float));
         if (e == hipSuccess) e = hipMalloc(&h->bgp, nzp * sizeof(PlaneM));
     }
-    if (e == hipSuccess) e = hipMalloc(&h->stage, pbytes);
+    h->stage_n = stage_fields(nf, pbytes);
+    if (e == hipSuccess) e = hipMalloc(&h->stage, h->stage_n * pbytes);
     if (e == hipSuccess) e = hipMalloc(&h->met, sizeof(double) * (3 * (d->npx + 2) + 3 * (d->npy + 2) + 5 * (d->npz + 2)));
-    if (e == hipSuccess) e = hipMalloc(&h->sc, sizeof(DevScalars));
-    if (e == hipSuccess) e = hipMalloc(&h->cs, sizeof(CflSlots));
+    static_assert(sizeof(DevScalars) <= 256, "the slots follow the scalars in one allocation");
+    if (e == hipSuccess) e = hipMalloc(&h->sc, 256 + sizeof(CflSlots));
+    if (e == hipSuccess) h->cs = reinterpret_cast<CflSlots *>(reinterpret_cast<char *>(h->sc) + 256);
     if (e != hipSuccess) {
         rc = fail(nullptr, MHD_ERR_HIP, "mhd_create: device allocation failed: %s", hipGetErrorString(e));
         free_all(h);
@@ -457,14 +475,11 @@ extern "C" int mhd_download(mhd_t *h, double *ru, double *rv, double *rw, double
     const int nf = nfields(h);
     const size_t pbytes = (size_t)(h->p.npx + 2) * (h->p.npy + 2) * (h->p.npz + 2) * sizeof(double);
     HIPCHK(h, hipSetDevice(h->dev));
-    for (int f = 0; f < nf; ++f) {
-        if (!dst[f]) continue;
-        const size_t off = (size_t)f * h->p.fsize;
-        if (!h->mixed) HIPCHK(h, launch_unpack(h->p, h->q[h->cur] + off, h->stage, 1, h->stream));
-        else HIPCHK(h, launch_unpack_mixed(h->p, h->hq[h->cur], h->rr, f, h->bg, h->stage, h->stream));
-        HIPCHK(h, hipMemcpyAsync(dst[f], h->stage, pbytes, hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(h, hipStreamSynchronize(h->stream));
-    }
+    auto unpack = [&](const FieldList &l) {
+        return h->mixed ? launch_unpack_mixed(h->p, h->hq[h->cur], h->rr, l, h->bg, h->stream)
+                        : launch_unpack(h->p, h->q[h->cur], l, 1, h->stream);
+    };
+    HIPCHK(h, download_fields(dst, nf, pbytes, h->stage, h->stage_n, unpack, h->stream));
     return MHD_OK;
 }
 
@@ -671,12 +686,8 @@ extern "C" int mhd_fluxes(mhd_t *h, double *fu, double *fv, double *fw, double *
     HIPCHK(h, rhs_eval(h));
     double *dst[8] = {fu, fv, fw, fr, ft, ww1, ww2, ww3};
     const size_t pbytes = (size_t)(h->p.npx + 2) * (h->p.npy + 2) * (h->p.npz + 2) * sizeof(double);
-    for (int f = 0; f < nf; ++f) {
-        if (!dst[f]) continue;
-        HIPCHK(h, launch_unpack(h->p, h->f + (size_t)f * h->p.fsize, h->stage, 0, h->stream));
-        HIPCHK(h, hipMemcpyAsync(dst[f], h->stage, pbytes, hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(h, hipStreamSynchronize(h->stream));
-    }
+    auto unpack = [&](const FieldList &l) { return launch_unpack(h->p, h->f, l, 0, h->stream); };
+    HIPCHK(h, download_fields(dst, nf, pbytes, h->stage, h->stage_n, unpack, h->stream));
     return MHD_OK;
 }
 
@@ -754,12 +765,9 @@ extern "C" int mhd_box_filter(mhd_t *h, int factor, int zmode, int source, doubl
         src = h->f;
     }
     const size_t bytes = (size_t)nf * nzc * nyc * nxc * sizeof(double);
-    double *d = nullptr;
-    HIPCHK(h, hipMalloc(&d, bytes));
-    hipError_t e = launch_box_filter(p, src, nf, factor, zmode, nxc, nyc, nzc, d, h->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(out, d, bytes, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    (void)hipFree(d);
+    HIPCHK(h, result_buffer(h, bytes));
+    hipError_t e = launch_box_filter(p, src, nf, factor, zmode, nxc, nyc, nzc, h->out, h->stream);
+    if (e == hipSuccess) e = download_array(out, h->out, bytes, h->stream);
     if (e != hipSuccess) return fail(h, MHD_ERR_HIP, "mhd_box_filter: %s", hipGetErrorString(e));
     return MHD_OK;
 }
@@ -772,13 +780,11 @@ extern "C" int mhd_flux_profiles(mhd_t *h, double *ttm, double *rom, double *fco
     HIPCHK(h, hipSetDevice(h->dev));
     const int nz = p.npz;
     std::vector<double> prof(3 * (size_t)nz);
-    double *d = nullptr;
-    HIPCHK(h, hipMalloc(&d, prof.size() * sizeof(double)));
-    hipError_t e = h->mixed ? launch_flux_profiles_mixed(p, h->hq[h->cur], h->rr, h->bg, d, h->stream)
-                            : launch_flux_profiles(p, h->q[h->cur], d, h->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(prof.data(), d, prof.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream);
+    HIPCHK(h, result_buffer(h, prof.size() * sizeof(double)));
+    hipError_t e = h->mixed ? launch_flux_profiles_mixed(p, h->hq[h->cur], h->rr, h->bg, h->out, h->stream)
+                            : launch_flux_profiles(p, h->q[h->cur], h->out, h->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(prof.data(), h->out, prof.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    (void)hipFree(d);
     if (e != hipSuccess) return fail(h, MHD_ERR_HIP, "mhd_flux_profiles: %s", hipGetErrorString(e));
     const double *t = prof.data();  // t[k-1]: plane k = 1..nz (reference K = k+1)
     if (ttm) std::copy(t, t + nz, ttm);

@@ -14,6 +14,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstddef>
 #include <cstdio>
@@ -57,7 +58,7 @@ struct mhd_ens {
     PlaneM *bgp = nullptr;           // mixed: per-plane records of the stage kernel, per box
     DevScalars *sc = nullptr;
     CflSlots *cs = nullptr;          // CFL reduction slots per box
-    double *stage = nullptr;         // one padded field of the largest box
+    double *stage = nullptr;         // padded fields for host transfers
     size_t stage_bytes = 0;
     // tiling
     int tile_x = 64, tile_y = 4, kdepth = 16, grid = 0;
@@ -98,6 +99,7 @@ static void drop_graphs(mhd_ens_t *e) {
 }
 
 static void free_ens(mhd_ens_t *e) {
+    copy_release();
     (void)hipSetDevice(e->dev);
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     drop_graphs(e);
@@ -161,6 +163,7 @@ extern "C" int mhd_ens_create(const mhd_desc *descs, int nbox, mhd_ens_t **out) 
     }
     mhd_ens_t *e = new (std::nothrow) mhd_ens();
     if (!e) return efail(nullptr, MHD_ERR_ARG, "mhd_ens_create: out of host memory");
+    copy_retain();  // given back by free_ens
     e->nbox = nbox;
     e->lmag = descs[0].lmag ? 1 : 0;
     e->mixed = descs[0].precision == MHD_MIXED;
@@ -182,7 +185,7 @@ extern "C" int mhd_ens_create(const mhd_desc *descs, int nbox, mhd_ens_t **out) 
         bg_off[b] = nzsum;
         nzsum += align_up((size_t)(B.p.npz + 2) * sizeof(double)) / sizeof(double);
         const size_t pb = (size_t)(B.p.npx + 2) * (B.p.npy + 2) * (B.p.npz + 2) * sizeof(double);
-        if (pb > e->stage_bytes) e->stage_bytes = pb;
+        e->stage_bytes = std::max(e->stage_bytes, stage_fields(nf, pb) * pb);
     }
     hipError_t r = hipGetDevice(&e->dev);
     if (r == hipSuccess) r = hipDeviceGetAttribute(&e->cus, hipDeviceAttributeMultiprocessorCount, e->dev);
@@ -346,14 +349,12 @@ extern "C" int mhd_ens_download(mhd_ens_t *e, int b, double *ru, double *rv, dou
     const int nf = e->lmag ? 8 : 5;
     const size_t pbytes = (size_t)(B.p.npx + 2) * (B.p.npy + 2) * (B.p.npz + 2) * sizeof(double);
     EHIP(e, hipSetDevice(e->dev));
-    for (int f = 0; f < nf; ++f) {
-        if (!dst[f]) continue;
-        const size_t off = (size_t)f * B.p.fsize;
-        if (!e->mixed) EHIP(e, launch_unpack(B.p, D.q[e->cur] + off, e->stage, 1, e->stream));
-        else EHIP(e, launch_unpack_mixed(B.p, D.h[e->cur], D.rr, f, D.a.bg, e->stage, e->stream));
-        EHIP(e, hipMemcpyAsync(dst[f], e->stage, pbytes, hipMemcpyDeviceToHost, e->stream));
-        EHIP(e, hipStreamSynchronize(e->stream));
-    }
+    auto unpack = [&](const FieldList &l) {
+        return e->mixed ? launch_unpack_mixed(B.p, D.h[e->cur], D.rr, l, D.a.bg, e->stream)
+                        : launch_unpack(B.p, D.q[e->cur], l, 1, e->stream);
+    };
+    EHIP(e, download_fields(dst, nf, pbytes, e->stage, (int)std::min<size_t>(nf, e->stage_bytes / pbytes), unpack,
+                            e->stream));
     return MHD_OK;
 }
 

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "../../include/rast3dmhd.h"
+#include "mhd_copy.h"
 #include "mhd_kernels.h"
 
 namespace rmhd {
@@ -268,6 +269,61 @@ inline int background_tables(const Params &p, const double *dzzdz, const double 
         q.omz = (float)p.omz;
     }
     return -1;
+}
+
+// Fields of the device staging buffer of a box (its size in padded fields):
+// as many as fit 16 MiB, and at least one: the download of a small box is then
+// one launch, of a large one a launch per field beside the copy of the last.
+inline int stage_fields(int nf, size_t field_bytes) {
+    const size_t n = ((size_t)16 << 20) / field_bytes;
+    return n < 1 ? 1 : n > (size_t)nf ? nf : (int)n;
+}
+
+// Download of the padded fields f = 0..nf-1 with dst[f] set: unpack(list)
+// queues the launch that writes the listed fields into the staging buffer
+// (room fields of field_bytes).
+template <class Unpack>
+hipError_t download_fields(double *const *dst, int nf, size_t field_bytes, double *stage, int room, Unpack unpack,
+                           hipStream_t s) {
+    struct Ctx {
+        int n = 0, f[NFIELD];
+        double *stage;
+        size_t field_bytes;
+        int room;
+        Unpack *unpack;
+    } c;
+    HostSpan spans[NFIELD];
+    for (int f = 0; f < nf; ++f)
+        if (dst[f]) {
+            spans[c.n] = HostSpan{dst[f], field_bytes};
+            c.f[c.n++] = f;
+        }
+    c.stage = stage;
+    c.field_bytes = field_bytes;
+    c.room = room;
+    c.unpack = &unpack;
+    const FillFn fill = [](void *ctx, int i, const char **src, hipError_t *err) {
+        const Ctx &x = *static_cast<Ctx *>(ctx);
+        FieldList l{};
+        for (l.n = 0; l.n < x.room && i + l.n < x.n; ++l.n) {
+            l.f[l.n] = x.f[i + l.n];
+            l.dst[l.n] = x.stage + (size_t)l.n * (x.field_bytes / sizeof(double));
+        }
+        *src = reinterpret_cast<const char *>(x.stage);
+        *err = (*x.unpack)(l);
+        return *err == hipSuccess ? l.n : 0;
+    };
+    return c.n ? copy_out(spans, c.n, fill, &c, s) : hipSuccess;
+}
+
+// Download of one contiguous device array that work queued on s produces.
+inline hipError_t download_array(void *dst, const void *src, size_t bytes, hipStream_t s) {
+    const HostSpan span{dst, bytes};
+    const FillFn fill = [](void *ctx, int, const char **out, hipError_t *) {
+        *out = static_cast<const char *>(ctx);
+        return 1;
+    };
+    return copy_out(&span, 1, fill, const_cast<void *>(src), s);
 }
 
 // Background table pointers into device blocks laid out as background_tables.

@@ -218,7 +218,14 @@ hipError_t launch_cfl(const Params &p, const Metrics &m, const double *q, DevSca
 // Arms the CFL reduction slots of n boxes.
 hipError_t launch_cfl_arm(CflSlots *cs, int n, hipStream_t s);
 hipError_t launch_pack(const Params &p, const double *padded, double *field, hipStream_t s);
-hipError_t launch_unpack(const Params &p, const double *field, double *padded, int mode, hipStream_t s);
+// n fields f[0..n) of register q into the padded arrays dst[0..n), one launch:
+// mode 1 with periodic ghosts, mode 0 with zero ghosts (right-hand sides).
+struct FieldList {
+    int n;
+    int f[NFIELD];
+    double *dst[NFIELD];
+};
+hipError_t launch_unpack(const Params &p, const double *q, const FieldList &l, int mode, hipStream_t s);
 
 // Ensemble launchers (all boxes share lmag and the tile height).  Register
 // a of every box is the stage input.  grid is the persistent grid size.
@@ -257,8 +264,8 @@ hipError_t launch_cfl_mixed(const Params &p, const Metrics &m, const Background 
 // fields).  Pack rho (field 3) before T (field 4).
 hipError_t launch_pack_mixed(const Params &p, const double *padded, int field, const Background &bg, float *hreg,
                              unsigned *rreg, hipStream_t s);
-hipError_t launch_unpack_mixed(const Params &p, const float *hreg, const unsigned *rreg, int field,
-                               const Background &bg, double *padded, hipStream_t s);
+hipError_t launch_unpack_mixed(const Params &p, const float *hreg, const unsigned *rreg, const FieldList &l,
+                               const Background &bg, hipStream_t s);
 // Re-expresses rho and T of the interior planes about the background nb
 // instead of ob, in place (mhd_rebase).
 hipError_t launch_rebase_mixed(const Params &p, const Background &ob, const Background &nb, float *hreg,

@@ -800,9 +800,12 @@ __global__ void k_pack(const Params p, const double *__restrict__ padded, double
     }
 }
 
-// resident field -> padded Fortran array; periodic ghost fill (mode 1) or
-// zero ghosts and zero z ghost planes (mode 0, for right-hand sides)
-__global__ void k_unpack(const Params p, const double *__restrict__ field, double *__restrict__ padded, int mode) {
+// resident fields -> padded Fortran arrays (one field per blockIdx.y);
+// periodic ghost fill (mode 1) or zero ghosts and zero z ghost planes (mode 0,
+// for right-hand sides)
+__global__ void k_unpack(const Params p, const double *__restrict__ q, const FieldList l, int mode) {
+    const double *__restrict__ const field = q + l.f[blockIdx.y] * p.fsize;
+    double *__restrict__ const padded = l.dst[blockIdx.y];
     const int nxp = p.npx + 2, nyp = p.npy + 2, nzp = p.npz + 2;
     const long long n = (long long)nxp * nyp * nzp;
     for (long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x; idx < n;
@@ -972,11 +975,11 @@ hipError_t launch_pack(const Params &p, const double *padded, double *field, hip
     return hipGetLastError();
 }
 
-hipError_t launch_unpack(const Params &p, const double *field, double *padded, int mode, hipStream_t s) {
+hipError_t launch_unpack(const Params &p, const double *q, const FieldList &l, int mode, hipStream_t s) {
     const long long n = (long long)(p.npx + 2) * (p.npy + 2) * (p.npz + 2);
     long long nb = (n + 255) / 256;
     if (nb > 8192) nb = 8192;
-    hipLaunchKernelGGL(k_unpack, dim3((unsigned)nb), dim3(256), 0, s, p, field, padded, mode);
+    hipLaunchKernelGGL(k_unpack, dim3((unsigned)nb, l.n), dim3(256), 0, s, p, q, l, mode);
     return hipGetLastError();
 }
 

@@ -720,9 +720,12 @@ __global__ void k_pack_m(const Params p, const double *__restrict__ padded, int 
     }
 }
 
-// field f of (stored value, R) -> padded FP64 field with periodic ghosts
+// fields of (stored value, R) -> padded FP64 fields with periodic ghosts (one
+// field per blockIdx.y)
 __global__ void k_unpack_m(const Params p, const float *__restrict__ hreg, const unsigned *__restrict__ rreg,
-                           int field, const Background bg, double *__restrict__ padded) {
+                           const FieldList l, const Background bg) {
+    const int field = l.f[blockIdx.y];
+    double *__restrict__ const padded = l.dst[blockIdx.y];
     const int nxp = p.npx + 2, nyp = p.npy + 2, nzp = p.npz + 2;
     const long long n = (long long)nxp * nyp * nzp, fs = p.fsize;
     for (long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x; idx < n;
@@ -867,12 +870,12 @@ hipError_t launch_pack_mixed(const Params &p, const double *padded, int field, c
     return hipGetLastError();
 }
 
-hipError_t launch_unpack_mixed(const Params &p, const float *hreg, const unsigned *rreg, int field,
-                               const Background &bg, double *padded, hipStream_t s) {
+hipError_t launch_unpack_mixed(const Params &p, const float *hreg, const unsigned *rreg, const FieldList &l,
+                               const Background &bg, hipStream_t s) {
     const long long n = (long long)(p.npx + 2) * (p.npy + 2) * (p.npz + 2);
     long long nb = (n + 255) / 256;
     if (nb > 8192) nb = 8192;
-    hipLaunchKernelGGL(k_unpack_m, dim3((unsigned)nb), dim3(256), 0, s, p, hreg, rreg, field, bg, padded);
+    hipLaunchKernelGGL(k_unpack_m, dim3((unsigned)nb, l.n), dim3(256), 0, s, p, hreg, rreg, l, bg);
     return hipGetLastError();
 }
 

@@ -149,7 +149,12 @@ extern "C" int mhd_step_noalloc(const mhd_desc *d, const mhd_dev_metrics *met, d
         b = t;
     }
     // download into the caller's arrays (as mhd_download), register a holds the result
-    for (int f = 0; f < nf; ++f) NACHK(launch_unpack(p, q[a] + (size_t)f * p.fsize, state[f], 1, s));
+    FieldList l{};
+    for (l.n = 0; l.n < nf; ++l.n) {
+        l.f[l.n] = l.n;
+        l.dst[l.n] = state[l.n];
+    }
+    NACHK(launch_unpack(p, q[a], l, 1, s));
     DevScalars out;
     NACHK(hipMemcpyAsync(&out, sc, sizeof(out), hipMemcpyDeviceToHost, s));
     NACHK(hipStreamSynchronize(s));
