@@ -8,19 +8,29 @@
 // periodic in x and y, zero padding in z.  Master parameters FP32 in the
 // order W1[co][tap][ci], b1, W2, b2, W3, b3 with tap = 9(dz+1)+3(dy+1)+(dx+1).
 //
-// k_conv: implicit GEMM D[voxel][co] = sum_k A[voxel][k] B[k][co] with
+// k_conv: implicit GEMM D[co][voxel] = sum_k W[co][k] A[voxel][k] with
 //   k = tap*CIN + ci, on v_mfma_f32_16x16x32_bf16 (lane l holds
-//   A[l%16][8(l/16)..+7], B[8(l/16)..+7][l%16], D[4(l/16)..+3][l%16]).  A
-//   workgroup (4 wavefronts) owns a 64 x 4 column tile and marches down a z
-//   chunk with a ring of three input planes (halo 1) in LDS; each wavefront
-//   computes one row of 64 voxels (4 M-tiles) for all output channels.  Each
-//   lane holds its B fragments of the whole layer in registers (most in
-//   accumulation registers, which the MFMA reads directly) for the whole
-//   march, so the fully unrolled K loop reads only A from LDS, one K block
-//   ahead of the MFMAs that use it.  The voxel stride in LDS is an odd
-//   number of 16-byte units so the 16 lanes of a fragment read hit distinct
-//   banks.  The epilogue adds the bias and applies GELU (hidden layers), or
-//   multiplies by GELU'(z) (backward).
+//   first[l%16][8(l/16)..+7], second[l%16][8(l/16)..+7],
+//   D[4(l/16)..+3][l%16]).  A workgroup owns a 64 x 4 column
+//   tile and marches down a z chunk with a ring of input planes (halo 1) in
+//   LDS; a wavefront computes 16 columns x 4 rows (4 tiles).
+//   - Weights stay in registers for the march; the only LDS is the input ring.
+//     32 -> 32 channels: 8 wavefronts, each half of the output channels, so
+//     that two share a SIMD and one's GELU (vector unit) runs beside the
+//     other's products; within one wavefront the two add up.
+//   - With 32 input channels a K block is one tap, so the fragment of an input
+//     row serves the three output rows it touches: 54 reads per plane instead
+//     of 108 (at 108 the LDS was as busy as the matrix cores).
+//   - Output channels are the first operand, so that a lane ends with 4 or 8
+//     consecutive channels of one voxel: one 8- or 16-byte store where the
+//     other order needs as many of 2 bytes.
+//   - Loads and stores are buffer accesses whose bounds check replaces the
+//     branches at the volume's edges, and the epilogue of a plane runs in
+//     pieces between the K blocks of the next.
+//   What bounds it: the vector work of the GELU (22 instructions a value, two
+//   of them at quarter rate) about as long as the products, and the LDS reads.
+//   Measured at 128x128x64 (before): 8 -> 32 35 us (60), 32 -> 32 60 us (90),
+//   32 -> 7 32 us (56); forward 127 us (204), 64x64x64 49 us (72).
 //   The backward pass for the input reuses it with the flipped, transposed
 //   kernel.
 // k_dw: weight gradient dW[co][tap][ci] = sum_v G[v][co] X[v+off][ci] as
@@ -35,6 +45,7 @@
 #include <cstdio>
 #include <cstring>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/rast3dmhd_closure.h"
@@ -45,6 +56,8 @@ namespace {
 typedef __bf16 bf16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int CTX = 64, CTY = 4;          // conv output tile per plane
 constexpr int LW = CTX + 2, LH = CTY + 2; // LDS plane with halo
@@ -52,8 +65,26 @@ constexpr int DSEG = 64;                  // dW: voxels per segment (two K block
 constexpr int GS = DSEG + 8;              // dW: LDS row stride of G (odd number of 16-B units)
 constexpr int XS = LW + 7;                // dW: LDS row stride of X (73, odd)
 
+// Shape of a convolution's workgroup.  32 -> 32 channels: 8 wavefronts, each
+// half of the output channels, so that two share a SIMD (the weights of all 32
+// are 216 registers a lane); 32 -> 8: three ring slots, so that two workgroups
+// fit a CU's LDS.
+template <int CIN, int NT>
+struct ConvShape {
+    static constexpr int HALVES = CIN == 32 && NT == 2 ? 2 : 1;
+    static constexpr int NTW = NT / HALVES;  // 16-channel tiles of a wavefront
+    static constexpr int THREADS = 256 * HALVES;
+    static constexpr int SLOTS = CIN == 32 && NT == 1 ? 3 : 4;
+    static constexpr int LDS = SLOTS * LW * LH * CIN * 2;  // bytes
+};
+
+// 16-byte unit of an LDS voxel that holds channel group u of column col.  The
+// 16 lanes that the LDS serves together read one group of 16 consecutive
+// columns, or two groups of 8 columns each, and so hit distinct banks.
 template <int CIN>
-constexpr int cstride() { return ((CIN / 8) % 2 == 0) ? CIN + 8 : CIN; }
+__device__ __forceinline__ int unit_of(int u, int col) {
+    return CIN == 32 ? u ^ ((0x78 >> (2 * ((col >> 2) & 3))) & 3) : u;
+}
 
 __device__ __forceinline__ int wrapn(int x, int n) {
     int r = x % n;
@@ -83,21 +114,23 @@ __device__ __forceinline__ float gelu_grad(float x) {
 // EPI 4: out16 = gelu(acc + bias) (inference: the pre-activation, which only
 // the backward pass reads, is not stored).
 template <int CIN, int NT, int EPI>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+__global__ __launch_bounds__((ConvShape<CIN, NT>::THREADS)) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_conv(const bf16 *__restrict__ x, const bf16 *__restrict__ wt, int kp,
                                               const float *__restrict__ bias, const float *__restrict__ zprev,
                                               bf16 *__restrict__ out16, float *__restrict__ out32,
                                               float *__restrict__ zout, int cout, int ostride, int nx, int ny,
                                               int nz, int kchunk) {
-    constexpr int CS = cstride<CIN>();
-    constexpr int PLANE = LW * LH * CS;
-    constexpr int NCH = CIN / 8;
-    constexpr int NLOAD = (LW * LH * NCH + 255) / 256;
+    using S = ConvShape<CIN, NT>;
+    constexpr int PLANE = LW * LH * CIN;
+    constexpr int NCH = CIN / 8, NTHR = S::THREADS, NTW = S::NTW;
+    constexpr int NLOAD = (LW * LH * NCH + NTHR - 1) / NTHR;
     constexpr int KTOT = 27 * CIN, KB = (KTOT + 31) / 32;
+    constexpr bool BIAS = EPI == 0 || EPI == 1 || EPI == 4;
+    constexpr int NCL = 4 * NTW;  // channels of a lane, consecutive
     extern __shared__ uint4 lds_raw[];
     bf16 *const lds = reinterpret_cast<bf16 *>(lds_raw);
 
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, lr = lane & 15, lg = lane >> 4;
+    const int t = threadIdx.x, lane = t & 63, wv = (t >> 6) & 3, half = t >> 8, lr = lane & 15, lg = lane >> 4;
     const int ntx = (nx + CTX - 1) / CTX, nty = (ny + CTY - 1) / CTY;
     const int bid = blockIdx.x;
     const int tz = bid / (ntx * nty);
@@ -106,134 +139,237 @@ void k_conv(const bf16 *__restrict__ x, const bf16 *__restrict__ wt, int kp,
     const int zb = tz * kchunk, ze = min(nz, zb + kchunk);
     if (zb >= nz) return;
 
-    // this thread's 16-byte pieces of an input plane with halo: offsets in a
-    // plane of x (-1: no piece) and in an LDS plane, computed once
-    int goff[NLOAD], loff[NLOAD];
+    constexpr unsigned NREC = 0xfffffff0u, OUT = 0xffffffffu;  // bytes of a buffer, an offset past them
+    // this thread's 16-byte pieces of an input plane with halo: byte offsets in
+    // a plane of x (OUT: no piece) and offsets in an LDS plane, computed once
+    unsigned goff[NLOAD];
+    int loff[NLOAD];
 #pragma unroll
     for (int i = 0; i < NLOAD; ++i) {
-        const int c = t + 256 * i;
-        goff[i] = -1;
+        const int c = t + NTHR * i;
+        goff[i] = OUT;
         loff[i] = 0;
         if (c < LW * LH * NCH) {
             const int vox = c / NCH, part = c - vox * NCH;
             const int row = vox / LW, col = vox - row * LW;
             const int gy = wrapn(y0 + row - 1, ny), gx = wrapn(x0 + col - 1, nx);
-            goff[i] = (gy * nx + gx) * CIN + part * 8;
-            loff[i] = vox * CS + part * 8;
+            goff[i] = ((unsigned)(gy * nx + gx) * CIN + part * 8) * (unsigned)sizeof(bf16);
+            loff[i] = vox * CIN + unit_of<CIN>(part, col) * 8;
         }
     }
     const long long pstride = (long long)nx * ny * CIN;
-    uint4 pre[NLOAD];
-    auto fetch = [&](int zz) {
+    typedef u32x4 Piece[NLOAD];
+    auto fetch = [&](int zz, Piece &pre) __attribute__((always_inline)) {
+        // a plane outside the volume, like a lane without a piece, reads past
+        // the buffer's end: zeros
         const bool in = zz >= 0 && zz < nz;
-        const bf16 *xz = x + (in ? zz : 0) * pstride;
-#pragma unroll
-        for (int i = 0; i < NLOAD; ++i) {
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (in && goff[i] >= 0) v = *reinterpret_cast<const uint4 *>(xz + goff[i]);
-            pre[i] = v;
-        }
-    };
-    auto slot = [](int zz) { return ((zz % 3) + 3) % 3; };
-    auto store = [&](int zz) {
-        bf16 *pl = lds + slot(zz) * PLANE;
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16 *>(x + (in ? zz : 0) * pstride), 0,
+                                                          in ? NREC : 0u, 0x00020000);
 #pragma unroll
         for (int i = 0; i < NLOAD; ++i)
-            if (goff[i] >= 0) *reinterpret_cast<uint4 *>(pl + loff[i]) = pre[i];
+            pre[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, goff[i], 0, 0);
     };
-    // the layer's B fragments (weights) of this lane, held in registers
-    // for the whole march: every plane uses all of them
-    bf16x8 wb[KB][NT];
+    auto store = [&](int sl, const Piece &pre) __attribute__((always_inline)) {
+        bf16 *pl = lds + sl * PLANE;
+#pragma unroll
+        for (int i = 0; i < NLOAD; ++i)  // (only the last piece is missing in some lanes)
+            if (i + 1 < NLOAD || goff[i] != OUT) *reinterpret_cast<u32x4 *>(pl + loff[i]) = pre[i];
+    };
+    // planes zb-1, zb, zb+1 into slots 0, 1, 2, their loads issued together (the
+    // first plane of the march waits for one memory latency, not for three)
+    {
+        Piece first[3];
+#pragma unroll
+        for (int n = 0; n < 3; ++n) fetch(zb - 1 + n, first[n]);
+#pragma unroll
+        for (int n = 0; n < 3; ++n) store(n, first[n]);
+    }
+    // the layer's weights of this lane, held in registers for the whole march.
+    // Row m of tile nt is channel 8 (m/4) + 4 nt + m%4 with two tiles, m (plus 16
+    // in the second half) with one.
+    bf16x8 wb[KB][NTW];
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-            wb[kb][nt] = *reinterpret_cast<const bf16x8 *>(wt + (long long)(16 * nt + lr) * kp + kb * 32 + lg * 8);
-    for (int zz = zb - 1; zz <= zb + 1; ++zz) {
-        fetch(zz);
-        store(zz);
+        for (int nt = 0; nt < NTW; ++nt) {
+            const int row = NTW == 2 ? 8 * (lr >> 2) + 4 * nt + (lr & 3) : 16 * half + lr;
+            wb[kb][nt] = *reinterpret_cast<const bf16x8 *>(wt + (long long)row * kp + kb * 32 + lg * 8);
+        }
+    const int co0 = 16 * half + NCL * lg;  // this lane's channels co0 .. co0 + NCL - 1
+    float bco[NCL];
+#pragma unroll
+    for (int c = 0; c < NCL; ++c) bco[c] = BIAS && co0 + c < cout ? bias[co0 + c] : 0.f;
+    const int gx = x0 + 16 * wv + lr;
+    const bool vx = gx < nx && co0 < ostride;
+    // this lane's column in an LDS row for dx = 0, 1, 2 (CIN = 32: its channels)
+    int vcol[3];
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx) {
+        const int col = 16 * wv + lr + dx;
+        vcol[dx] = CIN == 32 ? col * CIN + unit_of<CIN>(lg, col) * 8 : col * CIN;
     }
-    __syncthreads();
-
-    for (int z = zb; z < ze; ++z) {
-        const bool more = z + 1 < ze;
-        if (more) fetch(z + 2);
-        f32x4 acc[4][NT];
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        // the A fragments of K block kb: 4 M tiles of this wavefront's row
-        auto frag = [&](int kb, bf16x8 *a) __attribute__((always_inline)) {
-            const int k0 = kb * 32 + lg * 8;
-            if (k0 < KTOT) {
-                const int tap = k0 / CIN, ci0 = k0 - tap * CIN;
-                const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-                const bf16 *pl = lds + slot(z + dz) * PLANE + ((wv + 1 + dy) * LW + 1 + dx) * CS + ci0;
-#pragma unroll
-                for (int mt = 0; mt < 4; ++mt) a[mt] = *reinterpret_cast<const bf16x8 *>(pl + (16 * mt + lr) * CS);
-            } else {
-#pragma unroll
-                for (int mt = 0; mt < 4; ++mt) a[mt] = bf16x8{};
-            }
-        };
-        // K loop, software-pipelined: the LDS reads of block kb + 1 are
-        // issued before the MFMAs of block kb, which cover their latency
-        // (one wavefront per SIMD: nothing else would)
-        bf16x8 fa[2][4];
-        frag(0, fa[0]);
+    // CIN = 8: a K block holds four taps, one per lane group; the lane's offset
+    // of each block within a plane and its plane
+    int toff[CIN == 8 ? KB : 1], tdz[CIN == 8 ? KB : 1];
+    if (CIN == 8) {
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb) {
-            const int c = kb & 1;
-            if (kb + 1 < KB) frag(kb + 1, fa[c ^ 1]);
-#pragma unroll
-            for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
-                    acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[c][mt], wb[kb][nt], acc[mt][nt], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
+            const int tap = min(4 * kb + lg, 26);  // (there is no tap 27: zero)
+            tdz[kb] = tap / 9;
+            toff[kb] = ((tap / 3) % 3 * LW + tap % 3) * CIN;
         }
-        // epilogue: lane (lr, lg) holds voxels x0 + 16 mt + 4 lg + r of this
-        // wavefront's row for channel 16 nt + lr.  The row and channel
-        // checks are per lane; the column check only in a ragged tile.
-        const int gy = y0 + wv;
-        const long long rowo = (((long long)z * ny + gy) * nx + x0) * ostride;
-        auto emit = [&](float v, int co, float bco, long long o) __attribute__((always_inline)) {
-            if (EPI == 0) out32[o] = v + bco;
-            if (EPI == 1 || EPI == 4) {
-                const float zz = v + bco;
-                if (EPI == 1) zout[o] = zz;
-                out16[o] = (bf16)gelu(zz);
-            }
-            if (EPI == 2) out16[o] = (bf16)(v * gelu_grad(zprev[o]));
-            if (EPI == 3) out32[o] = v;
-        };
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const int co = 16 * nt + lr;
-            if (gy < ny && co < cout) {
-                const float bco = (EPI == 0 || EPI == 1 || EPI == 4) ? bias[co] : 0.f;
-                if (x0 + CTX <= nx) {
-#pragma unroll
-                    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            emit(acc[mt][nt][r], co, bco, rowo + (long long)(16 * mt + 4 * lg + r) * ostride + co);
-                } else {
-#pragma unroll
-                    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const int xo = 16 * mt + 4 * lg + r;
-                            if (x0 + xo < nx) emit(acc[mt][nt][r], co, bco, rowo + (long long)xo * ostride + co);
-                        }
-                }
-            }
-        }
-        __syncthreads();
-        if (more) store(z + 2);
-        __syncthreads();
     }
+
+    f32x4 acc[CTY][NTW], prv[CTY][NTW];
+    // Pieces of the epilogue of the plane held in prv: piece e < 4 NT CTY is one
+    // channel of row e / (4 NT); a row's last piece stores it.  Lanes and
+    // rows outside the volume access past the buffer's end, which the hardware
+    // drops: no branch splits the code that the products are mixed with.
+    constexpr int NPIECE = NCL * CTY;
+    auto row_of = [&](const void *base, int size, int zp, int gy) __attribute__((always_inline)) {
+        return __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<char *>(static_cast<const char *>(base)) + ((((long long)zp * ny + gy) * nx + x0) * ostride) * size, 0, NREC,
+            0x00020000);
+    };
+    const unsigned eo = (unsigned)((gx - x0) * ostride + co0);  // element offset of this lane in the tile's row
+    bf16 o16[NCL];
+    float o32[NCL], zrow[NCL];
+    auto piece = [&](int e, int zp) __attribute__((always_inline)) {
+        const int row = e / NCL, c = e % NCL;
+        const int gy = y0 + row;
+        const unsigned o2 = vx && gy < ny ? eo * 2 : OUT, o4 = vx && gy < ny ? eo * 4 : OUT;
+        if (EPI == 2 && c == 0) {
+            const auto rs = row_of(zprev, 4, zp, gy);
+#pragma unroll
+            for (int n = 0; n < NCL; n += 4) {
+                const f32x4 z4 = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, o4, 4 * n, 0));
+#pragma unroll
+                for (int r = 0; r < 4; ++r) zrow[n + r] = z4[r];
+            }
+        }
+        const float v = prv[row][c / 4][c % 4];
+        if (EPI == 2) {
+            o16[c] = (bf16)(v * gelu_grad(zrow[c]));
+        } else {
+            o32[c] = v + bco[c];
+            if (EPI == 1 || EPI == 4) o16[c] = (bf16)gelu(o32[c]);
+        }
+        if (c == NCL - 1) {
+            if (EPI == 0 || EPI == 1 || EPI == 3) {
+                const auto rs = row_of(EPI == 1 ? zout : out32, 4, zp, gy);
+#pragma unroll
+                for (int n = 0; n < NCL; n += 4)
+                    __builtin_amdgcn_raw_buffer_store_b128(
+                        __builtin_bit_cast(u32x4, (f32x4){o32[n], o32[n + 1], o32[n + 2], o32[n + 3]}), rs, o4, 4 * n, 0);
+            }
+            if (EPI == 1 || EPI == 2 || EPI == 4) {
+                typedef __bf16 out_t __attribute__((ext_vector_type(NCL)));
+                out_t w;
+#pragma unroll
+                for (int n = 0; n < NCL; ++n) w[n] = o16[n];
+                const auto rs = row_of(out16, 2, zp, gy);
+                if constexpr (NCL == 8)
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, w), rs, o2, 0, 0);
+                else
+                    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, w), rs, o2, 0, 0);
+            }
+        }
+    };
+
+    // plane z + 2 enters the fourth slot while plane z is computed (with three:
+    // the slot of plane z - 1 after it)
+    __syncthreads();
+    int s0 = 0, s1 = 1, s2 = 2, s3 = S::SLOTS == 4 ? 3 : 0;  // slots of planes z-1 .. z+2
+    auto plane = [&](int z, auto late_) __attribute__((always_inline)) {
+        constexpr bool late = decltype(late_)::value;  // the plane before waits in prv
+        const bool more = z + 1 < ze;
+        Piece next;
+        if (more) fetch(z + 2, next);
+#pragma unroll
+        for (int row = 0; row < CTY; ++row)
+#pragma unroll
+            for (int nt = 0; nt < NTW; ++nt) acc[row][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // K loop, software-pipelined: the LDS reads of the next unit are issued
+        // before the products of this one, which cover their latency (one
+        // wavefront per SIMD: nothing else would)
+        if constexpr (CIN == 32) {
+            // unit u: input row u % 6 of plane u / 6, three fragments (dx)
+            bf16x8 fa[2][3];
+            auto frag = [&](int u, bf16x8 *a) __attribute__((always_inline)) {
+                const int dz = u / 6, yin = u % 6;
+                const bf16 *pl = lds + (dz == 0 ? s0 : dz == 1 ? s1 : s2) * PLANE;
+#pragma unroll
+                for (int dx = 0; dx < 3; ++dx)
+                    a[dx] = *reinterpret_cast<const bf16x8 *>(pl + yin * LW * CIN + vcol[dx]);
+            };
+            frag(0, fa[0]);
+#pragma unroll
+            for (int u = 0; u < 18; ++u) {
+                const int c = u & 1, dz = u / 6, yin = u % 6;
+                if (u + 1 < 18) frag(u + 1, fa[c ^ 1]);
+                if (late && u < NPIECE) piece(u, z - 1);
+#pragma unroll
+                for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                    for (int row = 0; row < CTY; ++row) {
+                        const int dy = yin - row;
+                        if (dy < 0 || dy > 2) continue;
+#pragma unroll
+                        for (int nt = 0; nt < NTW; ++nt)
+                            acc[row][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[dz * 9 + dy * 3 + dx][nt], fa[c][dx],
+                                                                                   acc[row][nt], 0, 0, 0);
+                    }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            // unit u: K block u, the fragments of the four output rows
+            bf16x8 fa[2][CTY];
+            auto frag = [&](int u, bf16x8 *a) __attribute__((always_inline)) {
+                const int p0 = s0, p1 = s1, p2 = s2;
+                const int sl = tdz[u] == 0 ? p0 : tdz[u] == 1 ? p1 : p2;
+                const bf16 *pl = lds + sl * PLANE + toff[u] + vcol[0];
+#pragma unroll
+                for (int row = 0; row < CTY; ++row) {
+                    a[row] = *reinterpret_cast<const bf16x8 *>(pl + row * LW * CIN);
+                    if (u == KB - 1 && lg == 3) a[row] = bf16x8{};  // (no tap 27)
+                }
+            };
+            frag(0, fa[0]);
+#pragma unroll
+            for (int u = 0; u < KB; ++u) {
+                const int c = u & 1;
+                if (u + 1 < KB) frag(u + 1, fa[c ^ 1]);
+                constexpr int PER = (NPIECE + KB - 1) / KB;
+#pragma unroll
+                for (int e = 0; e < PER; ++e)
+                    if (late && u * PER + e < NPIECE) piece(u * PER + e, z - 1);
+#pragma unroll
+                for (int row = 0; row < CTY; ++row)
+#pragma unroll
+                    for (int nt = 0; nt < NTW; ++nt)
+                        acc[row][nt] =
+                            __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[u][nt], fa[c][row], acc[row][nt], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int row = 0; row < CTY; ++row)
+#pragma unroll
+            for (int nt = 0; nt < NTW; ++nt) prv[row][nt] = acc[row][nt];
+        if (S::SLOTS == 3) __syncthreads();  // plane z - 1 is done with
+        if (more) store(s3, next);
+        __syncthreads();
+        const int s = s0;
+        s0 = s1;
+        s1 = s2;
+        s2 = s3;
+        s3 = S::SLOTS == 4 ? s : s0;
+    };
+    plane(zb, std::false_type{});
+#pragma unroll 1
+    for (int z = zb + 1; z < ze; ++z) plane(z, std::true_type{});
+#pragma unroll
+    for (int e = 0; e < NPIECE; ++e) piece(e, ze - 1);
 }
 
 // Weight gradient partials: wave w accumulates taps w, w+4, ...; the
@@ -535,10 +671,12 @@ static int kchunk_for(int nx, int ny, int nz, int target, int *nblocks) {
 template <int CIN, int NT, int EPI>
 static hipError_t conv(hipStream_t s, const bf16 *x, const bf16 *w, int kp, const float *bias, const float *zprev,
                        bf16 *out16, float *out32, float *zout, int cout, int ostride, int nx, int ny, int nz) {
-    const int lds = 3 * LW * LH * cstride<CIN>() * (int)sizeof(bf16);
+    using S = ConvShape<CIN, NT>;
+    constexpr int lds = S::LDS;
     if (kp != 32 * ((27 * CIN + 31) / 32)) return hipErrorInvalidValue;  // the kernel's K blocks
-    if (lds > 160 * 1024) return hipErrorInvalidValue;
-    if ((long long)nx * ny * CIN > 0x7fffffffLL) return hipErrorInvalidValue;  // in-plane offsets are 32-bit
+    if (NT == 2 ? cout != 32 || ostride != 32 : cout > 8 || ostride != 8) return hipErrorInvalidValue;
+    static_assert(lds <= 160 * 1024, "the LDS of a CU");
+    if ((long long)nx * ny * CIN > 0x7fffffffLL) return hipErrorInvalidValue;  // in-plane byte offsets are 32-bit
     static std::atomic<unsigned long long> attr{0};
     hipError_t e = rmhd::lds_limit_once(attr, reinterpret_cast<const void *>(&k_conv<CIN, NT, EPI>), lds);
     if (e != hipSuccess) return e;
@@ -553,7 +691,7 @@ static hipError_t conv(hipStream_t s, const bf16 *x, const bf16 *w, int kp, cons
     if (!res) {
         int per_cu = 0, ncu = 0;
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(&k_conv<CIN, NT, EPI>),
-                                                         256, lds);
+                                                         S::THREADS, lds);
         if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
         if (e != hipSuccess) return e;
         res = std::max(1, per_cu) * std::max(1, ncu);
@@ -561,7 +699,7 @@ static hipError_t conv(hipStream_t s, const bf16 *x, const bf16 *w, int kp, cons
     }
     int nb;
     const int kc = kchunk_for(nx, ny, nz, res, &nb);
-    hipLaunchKernelGGL((k_conv<CIN, NT, EPI>), dim3(nb), dim3(256), lds, s, x, w, kp, bias, zprev, out16, out32, zout,
+    hipLaunchKernelGGL((k_conv<CIN, NT, EPI>), dim3(nb), dim3(S::THREADS), lds, s, x, w, kp, bias, zprev, out16, out32, zout,
                        cout, ostride, nx, ny, nz, kc);
     return hipGetLastError();
 }
