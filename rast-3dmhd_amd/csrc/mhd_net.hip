@@ -34,8 +34,10 @@
 //   The backward pass for the input reuses it with the flipped, transposed
 //   kernel.
 // k_dw: weight gradient dW[co][tap][ci] = sum_v G[v][co] X[v+off][ci] as
-//   D[co][ci] over K = voxels; per-workgroup partials, reduced in a fixed
-//   order (deterministic).
+//   D[co][ci] over K = voxels, and the bias gradient sum_v G[v][co] beside it;
+//   per-workgroup partials, reduced in a fixed order (deterministic) by
+//   k_update, which in training also takes the Adam step and writes the BF16
+//   weight panels.
 
 #include <hip/hip_runtime.h>
 
@@ -62,8 +64,9 @@ typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 constexpr int CTX = 64, CTY = 4;          // conv output tile per plane
 constexpr int LW = CTX + 2, LH = CTY + 2; // LDS plane with halo
 constexpr int DSEG = 64;                  // dW: voxels per segment (two K blocks)
-constexpr int GS = DSEG + 8;              // dW: LDS row stride of G (odd number of 16-B units)
-constexpr int XS = LW + 7;                // dW: LDS row stride of X (73, odd)
+constexpr int DS = DSEG + 8;              // dW: LDS row stride (odd number of 16-byte units)
+constexpr int DRING = 6;                  // dW: ring slots of X rows (4 in use, 2 arriving)
+constexpr int DBLK = 256;                 // dW: workgroups at most (one per CU)
 
 // Shape of a convolution's workgroup.  32 -> 32 channels: 8 wavefronts, each
 // half of the output channels, so that two share a SIMD (the weights of all 32
@@ -372,162 +375,253 @@ void k_conv(const bf16 *__restrict__ x, const bf16 *__restrict__ wt, int kp,
     for (int e = 0; e < NPIECE; ++e) piece(e, ze - 1);
 }
 
-// Weight gradient partials: wave w accumulates taps w, w+4, ...; the
-// workgroup walks segments of DSEG voxels of one (z, y) row.
+// Weight gradient partials.  The operands want 8 consecutive voxels of one
+// channel per lane, so rows of 64 voxels are kept transposed in LDS,
+// [channel][voxel].  A workgroup marches along y over pairs of rows of one
+// (z, x segment): a ring holds the X rows of the planes z-1, z, z+1, so each
+// row is transposed once per plane that uses it instead of once per tap row.
+// The x offset goes to G, kept in three shifted copies, which leaves every
+// fragment an aligned 16-byte read shared by three taps.  Wavefront (dz, half
+// h of the 16-channel tiles, K block kb) accumulates the 9 taps of its dz for
+// its half; the two K blocks are added through LDS at the end.  The rows of
+// the next pair are loaded while this one is computed.
+// What bounds it: the latency of those loads (one workgroup per CU); 64x64x64,
+// 32 x 32 channels 33 us against 97 with rows transposed per segment for every
+// tap and 2-byte LDS accesses; partials of 256 workgroups instead of 512.
 template <int CI, int CO>  // padded to multiples of 16
-__global__ __launch_bounds__(256) void k_dw(const bf16 *__restrict__ x, int cis, int ci_real,
-                                            const bf16 *__restrict__ g, int cos_, int co_real, int nx, int ny,
-                                            int nz, float *__restrict__ partial) {
-    constexpr int MT = CO / 16, NT = CI / 16, NTAP = 7;
-    __shared__ __align__(16) bf16 sg[CO * GS];
-    __shared__ __align__(16) bf16 sx[9 * CI * XS];
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, lr = lane & 15, lg = lane >> 4;
-    const int nsegx = (nx + DSEG - 1) / DSEG;
-    const long long nseg = (long long)nz * ny * nsegx;
-    f32x4 acc[NTAP][MT][NT];
-#pragma unroll
-    for (int s = 0; s < NTAP; ++s)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) acc[s][mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+constexpr int dw_lds_bytes() {
+    return (DRING * 3 * CI + 2 * 2 * 3 * CO) * DS * 2;
+}
 
-    for (long long seg = blockIdx.x; seg < nseg; seg += gridDim.x) {
-        const int sx0 = (int)(seg % nsegx) * DSEG;
-        const long long zy = seg / nsegx;
-        const int y = (int)(zy % ny), z = (int)(zy / ny);
-        __syncthreads();
-        // G of the segment, transposed: sg[co][v] (16-byte loads of 8 channels)
-        for (int e = t; e < DSEG * (CO / 8); e += 256) {
-            const int v = e / (CO / 8), c8 = e - v * (CO / 8);
-            const int gx = sx0 + v;
-            bf16x8 w = bf16x8{};
-            if (c8 * 8 < co_real && gx < nx)
-                w = *reinterpret_cast<const bf16x8 *>(g + (((long long)z * ny + y) * nx + gx) * cos_ + c8 * 8);
+template <int CI, int CO>
+__global__ __launch_bounds__(768, 3) void k_dw(const bf16 *__restrict__ x, int cis, const bf16 *__restrict__ g, int cos_,
+                                               int co_real, int nx, int ny, int nz, float *__restrict__ partial,
+                                               float *__restrict__ partial_b) {
+    constexpr int MT = CO / 16, NT = CI / 16;
+    constexpr int M = NT == 2 ? MT : 1;  // tiles of a wavefront
+    static_assert(MT * NT == 2 * M, "two halves");
+    extern __shared__ uint4 lds_raw[];
+    bf16 *const tx = reinterpret_cast<bf16 *>(lds_raw);  // [slot][dz][ci][DS]
+    bf16 *const tg = tx + DRING * 3 * CI * DS;           // [buffer][row][dx][co][DS]
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, lr = lane & 15, lg = lane >> 4;
+    const int dz = w % 3, h = (w / 3) % 2, kb = w / 6;
+    const int nseg = (nx + DSEG - 1) / DSEG, npair = (ny + 1) / 2;
+    const long long total = (long long)nz * nseg * npair;
+    const long long p0 = total * blockIdx.x / gridDim.x, p1 = total * (blockIdx.x + 1) / gridDim.x;
+    // padding channels stay zero
+    for (int e = t; e < dw_lds_bytes<CI, CO>() / 16; e += 768) lds_raw[e] = make_uint4(0, 0, 0, 0);
+
+    f32x4 acc[9][M];
 #pragma unroll
-            for (int q = 0; q < 8; ++q) sg[(c8 * 8 + q) * GS + v] = (c8 * 8 + q < co_real) ? w[q] : (bf16)0.f;
+    for (int s = 0; s < 9; ++s)
+#pragma unroll
+        for (int m = 0; m < M; ++m) acc[s][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float db[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+
+    // X task e: row, dz, voxel pair, channel group (fastest); G task: row, pair, group
+    const int nc = cis / 8, ng = cos_ / 8;
+    struct XPiece { uint4 v[2]; };
+    struct GPiece { uint4 v[4]; };
+    auto load_x = [&](int e, int z, int sx0, int row0) __attribute__((always_inline)) {
+        const int c8 = e % nc, pr = e / nc % 32, d = e / (32 * nc) % 3, row = row0 + e / (96 * nc);
+        const int zz = z + d - 1, yy = wrapn(row, ny);
+        XPiece q;
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const int xx = sx0 + 2 * pr + n;
+            q.v[n] = make_uint4(0, 0, 0, 0);
+            if (zz >= 0 && zz < nz && xx < nx)
+                q.v[n] = *reinterpret_cast<const uint4 *>(x + (((long long)zz * ny + yy) * nx + xx) * cis + c8 * 8);
         }
-        // X rows (z+dz, y+dy), x = sx0-1 .. sx0+DSEG, transposed: sx[row][ci][x]
-        for (int e = t; e < 9 * LW * (CI / 8); e += 256) {
-            const int row = e / (LW * (CI / 8)), r2 = e - row * (LW * (CI / 8));
-            const int col = r2 / (CI / 8), c8 = r2 - col * (CI / 8);
-            const int zz = z + row / 3 - 1, yy = wrapn(y + row % 3 - 1, ny), xx = wrapn(sx0 + col - 1, nx);
-            bf16x8 w = bf16x8{};
-            if (c8 * 8 < ci_real && zz >= 0 && zz < nz)
-                w = *reinterpret_cast<const bf16x8 *>(x + (((long long)zz * ny + yy) * nx + xx) * cis + c8 * 8);
+        return q;
+    };
+    // two voxels of 8 channels -> 8 words of (first, second) of one channel each
+    auto put_pair = [&](bf16 *row, int c8, int pr, const uint4 &a, const uint4 &b) __attribute__((always_inline)) {
+        const unsigned av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
-            for (int q = 0; q < 8; ++q) sx[(row * CI + c8 * 8 + q) * XS + col] = (c8 * 8 + q < ci_real) ? w[q] : (bf16)0.f;
+        for (int q = 0; q < 4; ++q) {
+            unsigned *const lo = reinterpret_cast<unsigned *>(row + (c8 * 8 + 2 * q) * DS + 2 * pr);
+            unsigned *const hi = reinterpret_cast<unsigned *>(row + (c8 * 8 + 2 * q + 1) * DS + 2 * pr);
+            *lo = __builtin_amdgcn_perm(bv[q], av[q], 0x05040100);
+            *hi = __builtin_amdgcn_perm(bv[q], av[q], 0x07060302);
         }
-        __syncthreads();
+    };
+    auto slot = [](int row) { return (row + 1) % DRING; };  // row >= -1
+    auto store_x = [&](int e, int row0, const XPiece &q) __attribute__((always_inline)) {
+        const int c8 = e % nc, pr = e / nc % 32, d = e / (32 * nc) % 3, row = row0 + e / (96 * nc);
+        put_pair(tx + (slot(row) * 3 + d) * CI * DS, c8, pr, q.v[0], q.v[1]);
+    };
+    const int gtasks = 2 * 32 * ng;
+    auto load_g = [&](int z, int sx0, int row0) __attribute__((always_inline)) {
+        GPiece q{};
+        if (t < gtasks) {
+            const int c8 = t % ng, pr = t / ng % 32, yy = wrapn(row0 + t / (32 * ng), ny);
 #pragma unroll
-        for (int s = 0; s < NTAP; ++s) {
-            const int tap = wv + 4 * s;
-            if (tap >= 27) break;
-            const int row = tap / 3, dx = tap % 3 - 1;  // row = 3(dz+1) + (dy+1)
-#pragma unroll
-            for (int kb = 0; kb < DSEG / 32; ++kb) {
-                const int k0 = kb * 32 + lg * 8;
-                bf16x8 a[MT], b[NT];
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt) a[mt] = *reinterpret_cast<const bf16x8 *>(&sg[(16 * mt + lr) * GS + k0]);
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-                    const bf16 *px = &sx[(row * CI + 16 * nt + lr) * XS + 1 + dx + k0];
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) b[nt][e] = px[e];
-                }
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                    for (int nt = 0; nt < NT; ++nt)
-                        acc[s][mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], b[nt], acc[s][mt][nt], 0, 0, 0);
+            for (int n = 0; n < 4; ++n) {
+                const int xx = wrapn(sx0 + 2 * pr - 1 + n, nx);
+                q.v[n] = *reinterpret_cast<const uint4 *>(g + (((long long)z * ny + yy) * nx + xx) * cos_ + c8 * 8);
             }
         }
-    }
-    // partial[blk][tap][co][ci]
+        return q;
+    };
+    auto store_g = [&](int sx0, int row0, int buf, const GPiece &q) __attribute__((always_inline)) {
+        if (t < gtasks) {
+            const int c8 = t % ng, pr = t / ng % 32, r = t / (32 * ng);
+            bf16 *const row = tg + (buf * 2 + r) * 3 * CO * DS;
 #pragma unroll
-    for (int s = 0; s < NTAP; ++s) {
-        const int tap = wv + 4 * s;
-        if (tap >= 27) break;
+            for (int dx = 0; dx < 3; ++dx) put_pair(row + dx * CO * DS, c8, pr, q.v[2 - dx], q.v[3 - dx]);
+            if (row0 + r < ny) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+                for (int n = 0; n < 2; ++n)
+                    if (sx0 + 2 * pr + n < nx) {
+                        const bf16x8 v = __builtin_bit_cast(bf16x8, q.v[1 + n]);
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
+                        for (int c = 0; c < 8; ++c) db[c] += (float)v[c];
+                    }
+            }
+        }
+    };
+
+    for (long long p = p0; p < p1;) {
+        const long long zs = p / npair;
+        int j = (int)(p - zs * npair);
+        const int z = (int)(zs / nseg), sx0 = (int)(zs % nseg) * DSEG;
+        const int jend = (int)min((long long)npair, j + (p1 - p));
+        p += jend - j;
+        __syncthreads();  // the last run's fragments are read
+        for (int e = t; e < 4 * 96 * nc; e += 768) store_x(e, 2 * j - 1, load_x(e, z, sx0, 2 * j - 1));
+        store_g(sx0, 2 * j, 0, load_g(z, sx0, 2 * j));
+        __syncthreads();
+        for (int buf = 0; j < jend; ++j, buf ^= 1) {
+            const bool more = j + 1 < jend;
+            XPiece xn{};
+            GPiece gn{};
+            if (more) {
+                if (t < 2 * 96 * nc) xn = load_x(t, z, sx0, 2 * j + 3);
+                gn = load_g(z, sx0, 2 * j + 2);
+            }
+            const int k0 = kb * 32 + lg * 8;
+            // X fragments of rows 2j-1 .. 2j+2 of plane z + dz - 1
+            auto xfrag = [&](int row, int nt) __attribute__((always_inline)) {
+                return *reinterpret_cast<const bf16x8 *>(tx + ((slot(row) * 3 + dz) * CI + 16 * nt + lr) * DS + k0);
+            };
+            bf16x8 xf[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int co = 16 * mt + 4 * lg + r, ci = 16 * nt + lr;
-                    partial[(((long long)blockIdx.x * 27 + tap) * CO + co) * CI + ci] = acc[s][mt][nt][r];
+            for (int n = 0; n < 4; ++n) xf[n] = xfrag(2 * j - 1 + n, NT == 2 ? h : 0);
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+                if (2 * j + r < ny) {
+#pragma unroll
+                    for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                        for (int m = 0; m < M; ++m) {
+                            const int mt = NT == 2 ? m : h;
+                            const bf16x8 a = *reinterpret_cast<const bf16x8 *>(
+                                tg + (((buf * 2 + r) * 3 + dx) * CO + 16 * mt + lr) * DS + k0);
+#pragma unroll
+                            for (int dy = 0; dy < 3; ++dy)
+                                acc[3 * dy + dx][m] =
+                                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, xf[r + dy], acc[3 * dy + dx][m], 0, 0, 0);
+                        }
                 }
+            if (more) {
+                if (t < 2 * 96 * nc) store_x(t, 2 * j + 3, xn);
+                store_g(sx0, 2 * j + 2, buf ^ 1, gn);
+            }
+            __syncthreads();
+        }
+    }
+
+    // add the two K blocks: those of kb = 1 pass theirs through LDS
+    f32x4 *const comb = reinterpret_cast<f32x4 *>(lds_raw);
+    static_assert(6 * 9 * M * 64 * 16 <= dw_lds_bytes<CI, CO>(), "the combined sums fit");
+    if (kb == 1)
+#pragma unroll
+        for (int s = 0; s < 9; ++s)
+#pragma unroll
+            for (int m = 0; m < M; ++m) comb[((w - 6) * 9 * M + s * M + m) * 64 + lane] = acc[s][m];
+    __syncthreads();
+    // partial[blk][tap][co][ci]
+    if (kb == 0)
+#pragma unroll
+        for (int s = 0; s < 9; ++s)
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const f32x4 v = acc[s][m] + comb[(w * 9 * M + s * M + m) * 64 + lane];
+                const int mt = NT == 2 ? m : h, nt = NT == 2 ? h : 0;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    partial[(((long long)blockIdx.x * 27 + 9 * dz + s) * CO + 16 * mt + 4 * lg + r) * CI + 16 * nt + lr] = v[r];
+            }
+    __syncthreads();
+    // bias partials: the sums of the threads that staged a channel, in thread order
+    float *const bred = reinterpret_cast<float *>(lds_raw);
+    if (t < gtasks)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) bred[t * 8 + c] = db[c];
+    __syncthreads();
+    if (t < co_real) {
+        float v = 0.f;
+        for (int e = t / 8; e < gtasks; e += ng) v += bred[e * 8 + t % 8];
+        partial_b[(long long)blockIdx.x * 32 + t] = v;
     }
 }
 
-// dW[co][tap][ci] (params order) = sum over the block partials: a workgroup
-// takes 32 consecutive outputs, its 8 thread groups sum the blocks c, c+8,
-// c+16, ... and the 8 group sums are added in order (deterministic).
-constexpr int DWR_OUT = 32, DWR_GRP = 8;
-__global__ __launch_bounds__(DWR_OUT *DWR_GRP) void k_dw_reduce(const float *__restrict__ partial, int nblk, int co_pad,
-                                                               int ci_pad, int co_real, int ci_real,
-                                                               float *__restrict__ dw) {
-    __shared__ float red[DWR_GRP][DWR_OUT];
-    const int j = threadIdx.x % DWR_OUT, c = threadIdx.x / DWR_OUT;
-    const int e = blockIdx.x * DWR_OUT + j;
-    const int ne = co_real * 27 * ci_real;
+// One layer as k_update sees it.
+struct LayerDev {
+    long long woff, boff;                    // in the parameter vector
+    int co, ci, co_pad, ci_pad, cis, cos_;   // channels, paddings of the partials, storage strides
+    int kpf, kpb;
+    const float *pw, *pb;                    // partials of k_dw
+    bf16 *wf, *wb;                           // weight panels
+};
+struct UpdateArgs {
+    LayerDev l[3];
+};
+
+// Gradient of every parameter as the sum of its nblk partials; with train
+// also the Adam step and the parameter's entries of the BF16 panels (the
+// padding of the panels was written by k_pack_w and stays).  A workgroup takes
+// 32 consecutive parameters: its 8 thread groups sum the partials c, c+8, ...
+// and the 8 sums are added in order (deterministic).  One launch in place of
+// three reductions, three bias reductions, Adam and three packings (62 + 26 +
+// 5 + 14 us of a 548 us iteration at 64x64x64; 13 us).
+constexpr int UPD_OUT = 32, UPD_GRP = 8;
+__global__ __launch_bounds__(UPD_OUT *UPD_GRP) void k_update(const UpdateArgs a, int nblk, long long nparam,
+                                                            float *__restrict__ grad, int train, float *__restrict__ p,
+                                                            float *__restrict__ am, float *__restrict__ av, float lr,
+                                                            float b1, float b2, float eps, float c1, float c2) {
+    __shared__ float red[UPD_GRP][UPD_OUT];
+    const int j = threadIdx.x % UPD_OUT, c = threadIdx.x / UPD_OUT;
+    const long long e = (long long)blockIdx.x * UPD_OUT + j;
+    const LayerDev &L = e < a.l[1].woff ? a.l[0] : e < a.l[2].woff ? a.l[1] : a.l[2];
+    const bool bias = e >= L.boff;
+    const int ew = (int)(e - L.woff);
+    const int co = bias ? (int)(e - L.boff) : ew / (27 * L.ci);
+    const int rem = bias ? 0 : ew - co * 27 * L.ci, tap = rem / L.ci, ci = rem - tap * L.ci;
     float s = 0.f;
-    if (e < ne) {
-        const int co = e / (27 * ci_real), r = e - co * 27 * ci_real, tap = r / ci_real, ci = r - tap * ci_real;
-        for (int b = c; b < nblk; b += DWR_GRP) s += partial[(((long long)b * 27 + tap) * co_pad + co) * ci_pad + ci];
+    if (e < nparam) {
+        const float *src = bias ? L.pb + co : L.pw + ((long long)tap * L.co_pad + co) * L.ci_pad + ci;
+        const long long step = bias ? 32 : 27LL * L.co_pad * L.ci_pad;
+#pragma unroll 8
+        for (int b = c; b < nblk; b += UPD_GRP) s += src[b * step];
     }
     red[c][j] = s;
     __syncthreads();
-    if (c == 0 && e < ne) {
-        float t = red[0][j];
-        for (int q = 1; q < DWR_GRP; ++q) t += red[q][j];
-        dw[e] = t;
-    }
-}
-
-// db partials: block b sums G over its voxel range.  A thread loads 8
-// channels (16 bytes) at a time; the per-channel sums of the threads are
-// then added in thread order (deterministic).
-__global__ __launch_bounds__(256) void k_db(const bf16 *__restrict__ g, int cos_, int co_real, long long nvox,
-                                            float *__restrict__ partial) {
-    __shared__ float red[256 * 8];
-    const int nch = cos_ / 8, vpb = 256 / nch;  // 16-byte chunks per voxel, voxels per pass
-    const int t = threadIdx.x, ch = t % nch, vt = t / nch;
-    const long long per = (nvox + gridDim.x - 1) / gridDim.x;
-    const long long v0 = blockIdx.x * per, v1 = min(nvox, v0 + per);
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (long long v = v0 + vt; v < v1; v += vpb) {
-        const bf16x8 w = *reinterpret_cast<const bf16x8 *>(g + v * cos_ + ch * 8);
-#pragma unroll
-        for (int q = 0; q < 8; ++q) acc[q] += (float)w[q];
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) red[t * 8 + q] = acc[q];
-    __syncthreads();
-    if (t < co_real) {
-        const int cc = t / 8, q = t % 8;
-        float s = 0.f;
-        for (int u = 0; u < vpb; ++u) s += red[(u * nch + cc) * 8 + q];
-        partial[blockIdx.x * co_real + t] = s;
-    }
-}
-
-// db = sum over the block partials: 8 thread groups sum the blocks c, c+8,
-// ..., then the group sums are added in order (deterministic).
-__global__ __launch_bounds__(DWR_OUT *DWR_GRP) void k_db_reduce(const float *__restrict__ partial, int nblk,
-                                                               int co_real, float *__restrict__ db) {
-    __shared__ float red[DWR_GRP][DWR_OUT];
-    const int co = threadIdx.x % DWR_OUT, c = threadIdx.x / DWR_OUT;
-    float s = 0.f;
-    if (co < co_real)
-        for (int b = c; b < nblk; b += DWR_GRP) s += partial[b * co_real + co];
-    red[c][co] = s;
-    __syncthreads();
-    if (c == 0 && co < co_real) {
-        float t = red[0][co];
-        for (int q = 1; q < DWR_GRP; ++q) t += red[q][co];
-        db[co] = t;
+    if (c != 0 || e >= nparam) return;
+    float gr = red[0][j];
+    for (int q = 1; q < UPD_GRP; ++q) gr += red[q][j];
+    grad[e] = gr;
+    if (!train) return;
+    const float mm = b1 * am[e] + (1.f - b1) * gr;
+    const float vv = b2 * av[e] + (1.f - b2) * gr * gr;
+    am[e] = mm;
+    av[e] = vv;
+    const float pn = p[e] - lr * (mm / c1) / (sqrtf(vv / c2) + eps);
+    p[e] = pn;
+    if (!bias) {
+        L.wf[(long long)co * L.kpf + tap * L.cis + ci] = (bf16)pn;
+        L.wb[(long long)ci * L.kpb + (26 - tap) * L.cos_ + co] = (bf16)pn;
     }
 }
 
@@ -581,19 +675,6 @@ __global__ __launch_bounds__(256) void k_loss(const float *__restrict__ y, const
     if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-__global__ void k_adam(float *__restrict__ p, const float *__restrict__ grad, float *__restrict__ m,
-                       float *__restrict__ v, long long n, float lr, float b1, float b2, float eps, float c1,
-                       float c2) {
-    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n) return;
-    const float gr = grad[e];
-    const float mm = b1 * m[e] + (1.f - b1) * gr;
-    const float vv = b2 * v[e] + (1.f - b2) * gr * gr;
-    m[e] = mm;
-    v[e] = vv;
-    p[e] -= lr * (mm / c1) / (sqrtf(vv / c2) + eps);
-}
-
 __global__ void k_f32_to_bf16(const float *__restrict__ a, bf16 *__restrict__ b, long long n, int cin, int cstr) {
     const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n * cstr) return;
@@ -631,9 +712,8 @@ struct mhd_net {
     long long cap = 0;
     bf16 *a0 = nullptr, *a1 = nullptr, *a2 = nullptr, *g1 = nullptr, *g2 = nullptr, *g3 = nullptr;
     float *z1 = nullptr, *z2 = nullptr, *y = nullptr, *tmp32 = nullptr, *dx32 = nullptr;
-    float *partial = nullptr;
+    float *partial = nullptr;  // of the three layers: weights, then biases
     double *lpart = nullptr;
-    int nblk_dw = 512;
     std::vector<Sample> samples;
     char err[512] = {0};
 };
@@ -761,50 +841,71 @@ static hipError_t forward_on(mhd_net_t *n, hipStream_t s, const bf16 *x, int nx,
     return e;
 }
 
-static hipError_t forward(mhd_net_t *n, int nx, int ny, int nz, bool keep) {
-    return forward_on(n, n->stream, n->a0, nx, ny, nz, keep);
+// Workgroups of k_dw for a volume: a share of the row pairs each.
+static int dw_blocks(int nx, int ny, int nz) {
+    return (int)std::min<long long>(DBLK, (long long)nz * ((nx + DSEG - 1) / DSEG) * ((ny + 1) / 2));
+}
+
+// Partials of layer l in n->partial: DBLK blocks of weights, then of biases;
+// l = 3: the length.
+static size_t partial_offset(const mhd_net_t *n, int l) {
+    size_t off = 0;
+    for (int i = 0; i < l; ++i) off += (size_t)DBLK * (27 * n->L[i].co_pad * n->L[i].ci_pad + 32);
+    return off;
+}
+static float *dw_weights(const mhd_net_t *n, int l) { return n->partial + partial_offset(n, l); }
+static float *dw_biases(const mhd_net_t *n, int l) {
+    return dw_weights(n, l) + (size_t)DBLK * 27 * n->L[l].co_pad * n->L[l].ci_pad;
 }
 
 template <int CI, int CO>
-static hipError_t dw(mhd_net_t *n, const bf16 *x, const Layer &L, const bf16 *g, int nx, int ny, int nz) {
-    const long long nseg = (long long)nz * ny * ((nx + DSEG - 1) / DSEG);
-    const int nblk = (int)std::min<long long>(n->nblk_dw, nseg);
-    hipLaunchKernelGGL((k_dw<CI, CO>), dim3(nblk), dim3(256), 0, n->stream, x, L.cis, L.ci, g, L.cos_, L.co, nx, ny, nz,
-                       n->partial);
-    hipError_t e = hipGetLastError();
+static hipError_t dw(mhd_net_t *n, const bf16 *x, int l, const bf16 *g, int nx, int ny, int nz) {
+    const Layer &L = n->L[l];
+    if (L.ci_pad != CI || L.co_pad != CO) return hipErrorInvalidValue;
+    constexpr int lds = dw_lds_bytes<CI, CO>();
+    static_assert(lds <= 160 * 1024, "the LDS of a CU");
+    static std::atomic<unsigned long long> attr{0};
+    hipError_t e = rmhd::lds_limit_once(attr, reinterpret_cast<const void *>(&k_dw<CI, CO>), lds);
     if (e != hipSuccess) return e;
-    const int ne = L.co * 27 * L.ci;
-    hipLaunchKernelGGL(k_dw_reduce, dim3((ne + DWR_OUT - 1) / DWR_OUT), dim3(DWR_OUT * DWR_GRP), 0, n->stream,
-                       n->partial, nblk, CO, CI, L.co, L.ci, n->grad + L.woff);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const long long nvox = (long long)nx * ny * nz;
-    const int nb = (int)std::min<long long>(256, (nvox + 255) / 256);
-    hipLaunchKernelGGL(k_db, dim3(nb), dim3(256), 0, n->stream, g, L.cos_, L.co, nvox, n->partial);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_db_reduce, dim3(1), dim3(DWR_OUT * DWR_GRP), 0, n->stream, n->partial, nb, L.co,
-                       n->grad + L.boff);
+    hipLaunchKernelGGL((k_dw<CI, CO>), dim3(dw_blocks(nx, ny, nz)), dim3(768), lds, n->stream, x, L.cis, g, L.cos_, L.co,
+                       nx, ny, nz, dw_weights(n, l), dw_biases(n, l));
     return hipGetLastError();
 }
 
-// backward from g3 (BF16, stride 8): parameter gradients into grad; with
-// want_dx the input gradient (FP32, stride 8) into dx32.
-static hipError_t backward(mhd_net_t *n, int nx, int ny, int nz, bool want_dx) {
+// backward from the input x and g3 (both BF16, stride 8): the layers' gradient
+// partials; with want_dx the input gradient (FP32, stride 8) into dx32.
+static hipError_t backward(mhd_net_t *n, const bf16 *x, int nx, int ny, int nz, bool want_dx) {
     const Layer *L = n->L;
-    hipError_t e = dw<32, 16>(n, n->a2, L[2], n->g3, nx, ny, nz);
+    hipError_t e = dw<32, 16>(n, n->a2, 2, n->g3, nx, ny, nz);
     if (e == hipSuccess)
         e = conv<8, 2, 2>(n->stream, n->g3, L[2].wb, L[2].kpb, nullptr, n->z2, n->g2, nullptr, nullptr, L[2].ci,
                           L[2].cis, nx, ny, nz);
-    if (e == hipSuccess) e = dw<32, 32>(n, n->a1, L[1], n->g2, nx, ny, nz);
+    if (e == hipSuccess) e = dw<32, 32>(n, n->a1, 1, n->g2, nx, ny, nz);
     if (e == hipSuccess)
         e = conv<32, 2, 2>(n->stream, n->g2, L[1].wb, L[1].kpb, nullptr, n->z1, n->g1, nullptr, nullptr, L[1].ci,
                            L[1].cis, nx, ny, nz);
-    if (e == hipSuccess) e = dw<16, 32>(n, n->a0, L[0], n->g1, nx, ny, nz);
+    if (e == hipSuccess) e = dw<16, 32>(n, x, 0, n->g1, nx, ny, nz);
     if (e == hipSuccess && want_dx)
         e = conv<32, 1, 3>(n->stream, n->g1, L[0].wb, L[0].kpb, nullptr, nullptr, nullptr, n->dx32, nullptr, L[0].ci,
                            8, nx, ny, nz);
     return e;
+}
+
+// Gradients from the partials of backward() into n->grad; with train the Adam
+// step number n->adam_t and the new weight panels.
+static hipError_t update(mhd_net_t *n, int nx, int ny, int nz, bool train, float lr) {
+    UpdateArgs a;
+    for (int l = 0; l < 3; ++l) {
+        const Layer &L = n->L[l];
+        a.l[l] = LayerDev{L.woff, L.boff, L.co, L.ci, L.co_pad, L.ci_pad, L.cis, L.cos_, L.kpf, L.kpb,
+                          dw_weights(n, l), dw_biases(n, l), L.wf, L.wb};
+    }
+    const float b1 = 0.9f, b2 = 0.999f;
+    const float c1 = 1.f - powf(b1, (float)n->adam_t), c2 = 1.f - powf(b2, (float)n->adam_t);
+    hipLaunchKernelGGL(k_update, dim3((unsigned)((n->nparam + UPD_OUT - 1) / UPD_OUT)), dim3(UPD_OUT * UPD_GRP), 0,
+                       n->stream, a, dw_blocks(nx, ny, nz), n->nparam, n->grad, train ? 1 : 0, n->p, n->am, n->av, lr, b1,
+                       b2, 1e-8f, c1, c2);
+    return hipGetLastError();
 }
 
 static int upload_input(mhd_net_t *n, const float *x, long long nvox, bf16 *dst) {
@@ -860,7 +961,7 @@ extern "C" int mhd_net_create(int cin, int width, int cout, mhd_net_t **out) {
         e = hipMalloc(&L.wf, (size_t)L.co_pad * L.kpf * sizeof(bf16));
         if (e == hipSuccess) e = hipMalloc(&L.wb, (size_t)L.ci_pad * L.kpb * sizeof(bf16));
     }
-    if (e == hipSuccess) e = hipMalloc(&n->partial, (size_t)n->nblk_dw * 27 * 32 * 32 * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc(&n->partial, partial_offset(n, 3) * sizeof(float));
     if (e == hipSuccess) e = hipMalloc(&n->lpart, 1024 * sizeof(double));
     if (e == hipSuccess) e = hipMemset(n->p, 0, off * sizeof(float));
     if (e == hipSuccess) e = hipMemset(n->am, 0, off * sizeof(float));
@@ -906,7 +1007,7 @@ extern "C" int mhd_net_forward(mhd_net_t *n, int nx, int ny, int nz, const float
     if (rc) return rc;
     rc = upload_input(n, x, nvox, n->a0);
     if (rc) return rc;
-    NHIP(n, forward(n, nx, ny, nz, false));
+    NHIP(n, forward_on(n, n->stream, n->a0, nx, ny, nz, false));
     // y (stride 8) -> host (stride cout)
     std::vector<float> tmp((size_t)nvox * 8);
     NHIP(n, hipMemcpyAsync(tmp.data(), n->y, nvox * 8 * sizeof(float), hipMemcpyDeviceToHost, n->stream));
@@ -927,7 +1028,7 @@ extern "C" int mhd_net_gradient(mhd_net_t *n, int nx, int ny, int nz, const floa
     if (rc) return rc;
     rc = upload_input(n, x, nvox, n->a0);
     if (rc) return rc;
-    NHIP(n, forward(n, nx, ny, nz, true));
+    NHIP(n, forward_on(n, n->stream, n->a0, nx, ny, nz, true));
     std::vector<float> g8((size_t)nvox * 8, 0.f);
     for (long long v = 0; v < nvox; ++v)
         for (int c = 0; c < n->cout; ++c) g8[(size_t)v * 8 + c] = dy[v * n->cout + c];
@@ -935,7 +1036,8 @@ extern "C" int mhd_net_gradient(mhd_net_t *n, int nx, int ny, int nz, const floa
     hipLaunchKernelGGL(k_f32_to_bf16, dim3((unsigned)((nvox * 8 + 255) / 256)), dim3(256), 0, n->stream, n->tmp32,
                        n->g3, nvox, 8, 8);
     NHIP(n, hipGetLastError());
-    NHIP(n, backward(n, nx, ny, nz, dx != nullptr));
+    NHIP(n, backward(n, n->a0, nx, ny, nz, dx != nullptr));
+    NHIP(n, update(n, nx, ny, nz, false, 0.f));
     NHIP(n, hipMemcpyAsync(dparams, n->grad, n->nparam * sizeof(float), hipMemcpyDeviceToHost, n->stream));
     if (dx) {
         NHIP(n, hipMemcpyAsync(g8.data(), n->dx32, nvox * 8 * sizeof(float), hipMemcpyDeviceToHost, n->stream));
@@ -992,22 +1094,16 @@ extern "C" int mhd_net_clear_samples(mhd_net_t *n) {
 static int sample_step(mhd_net_t *n, int s, bool train, float lr, double *loss) {
     const Sample &S = n->samples[s];
     const long long nvox = (long long)S.nx * S.ny * S.nz;
-    NHIP(n, hipMemcpyAsync(n->a0, S.x, nvox * 8 * sizeof(bf16), hipMemcpyDeviceToDevice, n->stream));
-    NHIP(n, forward(n, S.nx, S.ny, S.nz, train));
+    NHIP(n, forward_on(n, n->stream, S.x, S.nx, S.ny, S.nz, train));
     const int nb = (int)std::min<long long>(1024, (nvox * 8 + 255) / 256);
     const float gscale = (float)(2.0 / ((double)nvox * n->cout));
     hipLaunchKernelGGL(k_loss, dim3(nb), dim3(256), 0, n->stream, n->y, S.t, n->cout, nvox, gscale,
                        train ? n->g3 : nullptr, n->lpart);
     NHIP(n, hipGetLastError());
     if (train) {
-        NHIP(n, backward(n, S.nx, S.ny, S.nz, false));
+        NHIP(n, backward(n, S.x, S.nx, S.ny, S.nz, false));
         ++n->adam_t;
-        const float b1 = 0.9f, b2 = 0.999f;
-        const float c1 = 1.f - powf(b1, (float)n->adam_t), c2 = 1.f - powf(b2, (float)n->adam_t);
-        hipLaunchKernelGGL(k_adam, dim3((unsigned)((n->nparam + 255) / 256)), dim3(256), 0, n->stream, n->p, n->grad,
-                           n->am, n->av, n->nparam, lr, b1, b2, 1e-8f, c1, c2);
-        NHIP(n, hipGetLastError());
-        NHIP(n, pack_weights(n));
+        NHIP(n, update(n, S.nx, S.ny, S.nz, true, lr));
     }
     if (loss) {
         std::vector<double> lp(nb);
@@ -1049,12 +1145,12 @@ extern "C" int mhd_net_time_forward(mhd_net_t *n, int nx, int ny, int nz, int re
     NHIP(n, hipSetDevice(n->dev));
     rc = ensure_workspace(n, (long long)nx * ny * nz);
     if (rc) return rc;
-    NHIP(n, forward(n, nx, ny, nz, false));  // warm-up (also sets kernel attributes)
+    NHIP(n, forward_on(n, n->stream, n->a0, nx, ny, nz, false));  // warm-up (also sets kernel attributes)
     hipEvent_t a, b;
     NHIP(n, hipEventCreate(&a));
     NHIP(n, hipEventCreate(&b));
     NHIP(n, hipEventRecord(a, n->stream));
-    for (int r = 0; r < reps; ++r) NHIP(n, forward(n, nx, ny, nz, false));
+    for (int r = 0; r < reps; ++r) NHIP(n, forward_on(n, n->stream, n->a0, nx, ny, nz, false));
     NHIP(n, hipEventRecord(b, n->stream));
     NHIP(n, hipEventSynchronize(b));
     float t = 0;
