@@ -10,6 +10,13 @@ __device__ __forceinline__ int wrapi(int x, int n) {
     return r < 0 ? r + n : r;
 }
 
+// The same without a division where x lies in [-n, 2n); further right it is
+// some column of the box (lanes of a tile past the box's right neighbour,
+// whose values nothing uses).
+__device__ __forceinline__ int wrapc(int x, int n) {
+    return x < 0 ? x + n : x < n ? x : x < 2 * n ? x - n : n - 1;
+}
+
 // XCD-aware block order.  The hardware deals consecutive workgroup ids to
 // the 8 XCDs in turn; remap so that each XCD receives a contiguous run of
 // tiles (tiles that share halo rows then share an L2).  A bijection for any
@@ -151,7 +158,9 @@ __device__ __forceinline__ void cfl_publish(const unsigned long long *k, DevScal
     unsigned long long old = 0;
     if (lane < (lmag ? CFL_KEYS : CFL_KEYS - 1)) {
         unsigned long long *const w = &cs->key[lane][rep].v;
-        if (v < __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        // (a small launch has few atomics per line, and the read would only
+        // lengthen its tail)
+        if (total <= 512 || v < __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
             old = __hip_atomic_fetch_min(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     // the key updates have been performed: their results are here

@@ -79,7 +79,7 @@ inline int check_desc(const mhd_desc *d, char *msg, size_t len) {
 // time of a plane, which grows with the workgroups that share the CU (FP64:
 // 3.3 us alone, 5.7 us with two; mixed: 2.6, 3.5, 4.4 us).  The count with
 // the least sum wins: small boxes split until the chip is about full (64x64x32
-// FP64: 11 chunks of 3 planes, a stage of 20 us against 38 with 4 chunks on 64
+// FP64: 11 chunks of up to 3 planes, a stage of 18 us against 38 with 4 chunks on 64
 // of 256 CUs), larger ones take whole rounds (256x256x128 mixed: 6 chunks, two
 // full rounds, 230 us against 254 with 16 chunks of 5.3 rounds).  Chunks are
 // at most 32 planes: over a longer march the tiles that share halo rows drift
@@ -93,7 +93,7 @@ inline int z_chunks(int npz, int ntiles, int occ, double alone, double more) {
         const long long n = (long long)ntiles * nc, slots = (long long)CUS * occ;
         const long long rest = (n % slots + CUS - 1) / CUS;
         const double round = alone + (occ - 1) * more, last = rest ? alone + (rest - 1) * more : 0.0;
-        const double t = ((npz + nc - 1) / nc + 1.5) * ((double)(n / slots) * round + last);
+        const double t = (chunk_depth(npz, nc) + 1.5) * ((double)(n / slots) * round + last);
         if (tbest == 0.0 || t < tbest) {
             tbest = t;
             best = nc;

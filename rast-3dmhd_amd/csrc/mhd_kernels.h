@@ -166,13 +166,24 @@ struct StageItem {
     int box, i0, j0, kbeg, kend, seq, total;
 };
 
-// Planes 1..npz of a box split into nc chunks of sizes that differ by at most
-// one: chunk c covers planes chunk_begin(npz, nc, c) .. chunk_begin(npz, nc,
-// c + 1) - 1.  A chunk with a boundary plane also applies the boundary
-// conditions there, which read the two planes next to it, so a chunk has at
-// least three planes: nc <= max_chunks(npz).
-__host__ __device__ inline int chunk_begin(int npz, int nc, int c) { return 1 + (int)((long long)c * npz / nc); }
-__host__ __device__ inline int max_chunks(int npz) { return npz / 3 > 0 ? npz / 3 : 1; }
+// Planes 1..npz of a box split into nc chunks: chunk c covers the planes
+// chunk_begin(npz, nc, c) .. chunk_begin(npz, nc, c + 1) - 1, at most
+// chunk_depth(npz, nc) of them.  The first and the last chunk hold a boundary
+// plane and apply the boundary conditions there, which read the two planes
+// next to it, so they have at least three planes (as many as the deepest); the
+// others share the rest evenly, down to one plane each.
+__host__ __device__ inline int max_chunks(int npz) { return npz < 6 ? 1 : npz - 4; }
+__host__ __device__ inline int chunk_depth(int npz, int nc) {
+    const int d = (npz + nc - 1) / nc;
+    return d < 3 ? 3 : d;
+}
+__host__ __device__ inline int chunk_begin(int npz, int nc, int c) {
+    if (c == 0) return 1;
+    if (c == nc) return npz + 1;
+    if (nc == 2) return 1 + npz / 2;
+    const int e = chunk_depth(npz, nc), rest = npz - 2 * e;
+    return 1 + e + (int)((long long)(c - 1) * rest / (nc - 2));
+}
 
 __host__ __device__ inline unsigned long long dkey(double v) {
     unsigned long long b = __builtin_bit_cast(unsigned long long, v);

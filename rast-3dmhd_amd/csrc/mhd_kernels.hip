@@ -29,8 +29,8 @@
 // (2.86 / 3.59 / 3.13 ms for 12.9 / 17.2 / 12.9 GB of algorithmic bytes); on
 // small boxes the latency of a plane's march (3.3 us with one workgroup on a
 // CU) and of the launch, hence few planes per chunk (z_chunks) and three
-// launches per step (64x64x32: 72 us per step, 132 with boundary, CFL and
-// 8-plane launches of their own; 16x16x12 by single steps: 88 against 210).
+// launches per step (64x64x32: 56 us per step, 132 with boundary, CFL and
+// 8-plane launches of their own; 16x16x12 by single steps: 82 against 210).
 //
 // Arithmetic: every expression keeps the reference's left-to-right
 // association and the file is compiled with -ffp-contract=off, so results
@@ -142,8 +142,11 @@ __device__ void cfl_reduce(double mach, double w1, double w2, double w3, double 
 // it owns when its chunk holds a boundary plane and so, with at least three
 // planes, everything BCON reads: the conditions then need no launch of their
 // own (5, 5 and 10 us of a 130 us step at 64x64x32, 8, 8 and 23 us of 1280
-// at 256x256x128).  With CFL set (stage 3), the boundary planes' CFL limits
-// of the final state are added to the accumulators.
+// at 256x256x128).  It is a chain of loads at the end of a workgroup's march:
+// all of them are issued before the first store, which the compiler could not
+// move them across itself (64x64x32, stage 3: 26.8 us with a wait per field,
+// 21.3 so).  With CFL set (stage 3), the boundary planes' CFL limits of the
+// final state are added to the accumulators.
 template <bool MAG, bool CFL>
 __device__ __forceinline__ void bcon_column(const Params &p, const Metrics &m, const double *__restrict__ qin,
                                             double *q, const DevScalars *sc, int i, int j, bool top, bool bot,
@@ -151,76 +154,71 @@ __device__ __forceinline__ void bcon_column(const Params &p, const Metrics &m, c
     const long long fs = p.fsize, pl = p.plane, idx = (long long)j * p.npx + i;
     const int nz = p.npz;
     const double C13 = p.c13, C23 = p.c23, C43 = p.c43;
-    double *RU = q, *RV = q + fs, *RW = q + 2 * fs, *RO = q + 3 * fs, *TT = q + 4 * fs, *BZ = q + 7 * fs;
     const double *ROi = qin + 3 * fs;
     // shear boundaries: RRT = 1, RRB = -1, RPP = 0 (sub:2751-2756)
     const double shear = p.lshr ? cos(0.0 * sc->timt) : 0.0;
-    auto limits = [&](int k) __attribute__((always_inline)) {
-        const long long o = (long long)k * pl + idx;
+#pragma unroll 1
+    for (int side = 0; side < 2; ++side) {
+        if (side ? !bot : !top) continue;
+        const int k = side ? nz : 1, in = side ? -1 : 1;  // boundary plane, direction inwards
+        const long long o = (long long)k * pl + idx, b = o + in * pl, c = b + in * pl;
+        // everything that is read, before the first store (one wait, not one per
+        // store): the plane's own values, RU, RV, RO, TT of the next two, and RO
+        // of the ghost plane
         double v[8];
+        v[F_RO] = q[3 * fs + o];
+        v[F_TT] = q[4 * fs + o];
+        if (MAG) {
 #pragma unroll
-        for (int f = 0; f < (MAG ? 8 : 5); ++f) v[f] = q[f * fs + o];
-        cfl_point<MAG>(p, v, m.ddx[i + 1], m.ddy[j + 1], m.ddz[k], m.rkcfl[k], c_mach, c_w1, c_w2, c_w3, c_w4);
-    };
-    if (top) {  // sub:2771-2868
-        const long long a = pl + idx, b = 2 * pl + idx, c = 3 * pl + idx;
-        if (p.lshr) {
-            RU[a] = 0.0;
-            RV[a] = 1.0 * shear * RO[a];
-        } else {
-            RU[a] = RO[a] * (C43 * RU[b] / RO[b] - C13 * RU[c] / RO[c]);
-            RV[a] = RO[a] * (C43 * RV[b] / RO[b] - C13 * RV[c] / RO[c]);
+            for (int f = F_BX; f <= F_BZ; ++f) v[f] = q[f * fs + o];
         }
-        RW[a] = 0.0;
-        if (p.tp != 0.0 && (p.itc == 0 || p.itc == 1)) {
+        const double rub = q[b], ruc = q[c], rvb = q[fs + b], rvc = q[fs + c];
+        const double rob = q[3 * fs + b], roc = q[3 * fs + c], ttb = q[4 * fs + b], ttc = q[4 * fs + c];
+        // the z ghost plane of RO flips to 1/RO once per FLUXES call; with ID or
+        // LREM it held the mirrored RO of the plane next to the boundary
+        // (sub:1301-1310)
+        const int kg = side ? nz + 1 : 0;
+        const double rog = ROi[(long long)(p.mirror ? k + in : kg) * pl + idx];
+        const double dz = p.dzf / m.dzzdz[k];
+        if (p.lshr) {
+            v[F_RU] = 0.0;
+            v[F_RV] = (side ? -1.0 : 1.0) * shear * v[F_RO];
+        } else {
+            v[F_RU] = v[F_RO] * (C43 * rub / rob - C13 * ruc / roc);
+            v[F_RV] = v[F_RO] * (C43 * rvb / rob - C13 * rvc / roc);
+        }
+        v[F_RW] = 0.0;
+        bool sett = true;
+        if (side) {  // sub:2873-2955
+            if (p.izc == 0) v[F_TT] = p.tb;
+            else if (p.lrem) v[F_TT] = C43 * ttb - C13 * ttc + p.dztb;
+            else v[F_TT] = C43 * ttb - C13 * ttc + C23 * dz * p.theta / m.rkapa[nz];
+        } else if (p.tp != 0.0 && (p.itc == 0 || p.itc == 1)) {
             // Gaussian top temperature or flux (sub:2790-2827)
             const double HH = p.hh, ex = p.gx[i + 1], ey = p.gy[j + 1];
-            if (p.itc == 0) {
-                TT[a] = 1.0 - (1.0 - p.tpr) * ex / HH * ey / HH;
-            } else {
-                const double dz = p.dzf / m.dzzdz[1];
-                TT[a] = C43 * TT[b] - C13 * TT[c] - C23 * dz * (p.theta - (p.theta - p.tpr) * ex / HH * ey / HH);
-            }
+            if (p.itc == 0) v[F_TT] = 1.0 - (1.0 - p.tpr) * ex / HH * ey / HH;
+            else v[F_TT] = C43 * ttb - C13 * ttc - C23 * dz * (p.theta - (p.theta - p.tpr) * ex / HH * ey / HH);
         } else if (p.itc == 0 || p.itc == 2 || p.itc == 4) {
             // fixed T; TU with LREM; ITC=4: TP cooler on I <= NX/2 (sub:2828-2850)
-            if (p.lrem) TT[a] = p.tu;
-            else TT[a] = (p.itc == 4 && i + 2 <= (p.npx + 2) / 2) ? 1.0 - p.tp : 1.0;
+            if (p.lrem) v[F_TT] = p.tu;
+            else v[F_TT] = (p.itc == 4 && i + 2 <= (p.npx + 2) / 2) ? 1.0 - p.tp : 1.0;
         } else if (p.itc == 1) {
-            if (p.lrem) {
-                TT[a] = C43 * TT[b] - C13 * TT[c] + p.dztu;
-            } else {
-                const double dz = p.dzf / m.dzzdz[1];
-                TT[a] = C43 * TT[b] - C13 * TT[c] - C23 * dz * p.theta;
-            }
-        }  // ITC=3: the top temperature is left to the equations
-        if (MAG && p.ibc == 0) BZ[a] = 0.0;
-        // the z ghost plane of RO flips to 1/RO once per FLUXES call; with ID
-        // or LREM it held the mirrored RO of plane 2 (sub:1301-1310)
-        RO[idx] = 1.0 / ROi[(p.mirror ? 2 * pl : 0) + idx];
-        if (CFL) limits(1);
-    }
-    if (bot) {  // sub:2873-2955
-        const long long a = (long long)nz * pl + idx, b = (long long)(nz - 1) * pl + idx,
-                        c = (long long)(nz - 2) * pl + idx;
-        if (p.lshr) {
-            RU[a] = 0.0;
-            RV[a] = -1.0 * shear * RO[a];
+            if (p.lrem) v[F_TT] = C43 * ttb - C13 * ttc + p.dztu;
+            else v[F_TT] = C43 * ttb - C13 * ttc - C23 * dz * p.theta;
         } else {
-            RU[a] = RO[a] * (C43 * RU[b] / RO[b] - C13 * RU[c] / RO[c]);
-            RV[a] = RO[a] * (C43 * RV[b] / RO[b] - C13 * RV[c] / RO[c]);
+            sett = false;  // ITC=3: the top temperature is left to the equations
         }
-        RW[a] = 0.0;
-        if (p.izc == 0) {
-            TT[a] = p.tb;
-        } else if (p.lrem) {
-            TT[a] = C43 * TT[b] - C13 * TT[c] + p.dztb;
-        } else {
-            const double dz = p.dzf / m.dzzdz[nz];
-            TT[a] = C43 * TT[b] - C13 * TT[c] + C23 * dz * p.theta / m.rkapa[nz];
+        q[o] = v[F_RU];
+        q[fs + o] = v[F_RV];
+        q[2 * fs + o] = v[F_RW];
+        if (sett) q[4 * fs + o] = v[F_TT];
+        if (MAG && p.ibc == 0) {
+            v[F_BZ] = 0.0;
+            q[7 * fs + o] = 0.0;
         }
-        if (MAG && p.ibc == 0) BZ[a] = 0.0;
-        RO[(long long)(nz + 1) * pl + idx] = 1.0 / ROi[(long long)(p.mirror ? nz - 1 : nz + 1) * pl + idx];
-        if (CFL) limits(nz);
+        q[3 * fs + (long long)kg * pl + idx] = 1.0 / rog;
+        if (CFL)
+            cfl_point<MAG>(p, v, m.ddx[i + 1], m.ddy[j + 1], m.ddz[k], m.rkcfl[k], c_mach, c_w1, c_w2, c_w3, c_w4);
     }
 }
 
@@ -261,7 +259,8 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
     const int opt = oly * SW + olx;
     const int gi = i0 + olx - 1, gj = j0 + oly - 1;
     const bool valid = (gi < npx) && (gj < npy);
-    const long long ooff = (long long)wrapi(gj, npy) * npx + wrapi(gi, npx);
+    const int gci = wrapc(gi, npx), gcj = wrapc(gj, npy);  // this lane's column
+    const long long ooff = (long long)gcj * npx + gci;
     // halo point (t < NHALO): top row, bottom row, left column, right column
     int hpt = -1;
     long long hoff = 0;
@@ -272,7 +271,7 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
         else if (t < 2 * SW + TY) { hlx = 0; hly = t - 2 * SW + 1; }
         else { hlx = SW - 1; hly = t - 2 * SW - TY + 1; }
         hpt = hly * SW + hlx;
-        hoff = (long long)wrapi(j0 + hly - 1, npy) * npx + wrapi(i0 + hlx - 1, npx);
+        hoff = (long long)wrapc(j0 + hly - 1, npy) * npx + wrapc(i0 + hlx - 1, npx);
     }
     const bool has_h = hpt >= 0;
 
@@ -289,6 +288,26 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
         ring(k, 2, pt) = r.v[S_RW] * ri;
     };
 
+    // the per-column values are on their way before the warm-up's loads
+    const double HX = p.hx, H2X = p.h2x, HY = p.hy, H2Y = p.h2y, HZ = p.hz, H2Z = p.h2z;
+    const double C43 = p.c43, OCV = p.ocv, ORE = p.ore, ORM = p.orm, OBETA = p.obeta;
+    const int gix = gci + 1, gjy = gcj + 1;
+    const double dx = m.dxxdx[gix], d2x = m.d2xxdx2[gix];
+    const double dy = m.dyydy[gjy], d2y = m.d2yydy2[gjy];
+    const double tmpy = HY * dy;
+    const double tmpy1 = HY * d2y;
+    const double tmpy2 = H2Y * dy * dy;
+    double coefg = 0.0, coefz = 0.0;
+    if (MODE > 0) {
+        const double dt = sc->dt;
+        coefg = (MODE == 1 ? p.gam1 : MODE == 2 ? p.gam2 : p.gam3) * dt;
+        coefz = (MODE == 1 ? p.zeta1 : p.zeta2) * dt;
+    }
+    // CFL accumulators of the new state (stage 3 only)
+    double c_mach = 0.0, c_w1 = INFINITY, c_w2 = INFINITY, c_w3 = INFINITY, c_w4 = INFINITY;
+    const double c_ddx = MODE == 3 ? m.ddx[gix] : 0.0, c_ddy = MODE == 3 ? m.ddy[gjy] : 0.0;
+    // the embedded heat loss's per-column Gaussians, read once
+    const double c_gx = (OPT && p.itc == 2) ? p.gx[gix] : 0.0, c_gy = (OPT && p.itc == 2) ? p.gy[gjy] : 0.0;
     // Warm-up: planes kbeg-1 (own values + ring), kbeg and kbeg+1 (LDS + ring).
     // Every load is issued before the first is used: a chunk then pays one
     // memory latency before its march instead of three.
@@ -325,25 +344,6 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
         }
     }
 
-    const double HX = p.hx, H2X = p.h2x, HY = p.hy, H2Y = p.h2y, HZ = p.hz, H2Z = p.h2z;
-    const double C43 = p.c43, OCV = p.ocv, ORE = p.ore, ORM = p.orm, OBETA = p.obeta;
-    const int gix = wrapi(gi, npx) + 1, gjy = wrapi(gj, npy) + 1;
-    const double dx = m.dxxdx[gix], d2x = m.d2xxdx2[gix];
-    const double dy = m.dyydy[gjy], d2y = m.d2yydy2[gjy];
-    const double tmpy = HY * dy;
-    const double tmpy1 = HY * d2y;
-    const double tmpy2 = H2Y * dy * dy;
-    double coefg = 0.0, coefz = 0.0;
-    if (MODE > 0) {
-        const double dt = sc->dt;
-        coefg = (MODE == 1 ? p.gam1 : MODE == 2 ? p.gam2 : p.gam3) * dt;
-        coefz = (MODE == 1 ? p.zeta1 : p.zeta2) * dt;
-    }
-    // CFL accumulators of the new state (stage 3 only)
-    double c_mach = 0.0, c_w1 = INFINITY, c_w2 = INFINITY, c_w3 = INFINITY, c_w4 = INFINITY;
-    const double c_ddx = MODE == 3 ? m.ddx[gix] : 0.0, c_ddy = MODE == 3 ? m.ddy[gjy] : 0.0;
-    // the embedded heat loss's per-column Gaussians, read once
-    const double c_gx = (OPT && p.itc == 2) ? p.gx[gix] : 0.0, c_gy = (OPT && p.itc == 2) ? p.gy[gjy] : 0.0;
     // the per-column metrics arrive before the march, not inside its first plane
     settle(dx), settle(d2x), settle(dy), settle(d2y), settle(c_ddx), settle(c_ddy);
     if (OPT) settle(c_gx), settle(c_gy);
@@ -366,11 +366,11 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
 #pragma unroll
             for (int f = 0; f < NF; ++f) zk[f] = __builtin_nontemporal_load(&zr[f * fs + o]);
         }
+        const double dz = uload(m.dzzdz, k), d2z = uload(m.d2zzdz2, k);
+        const double rk = uload(m.rkapa, k), dk = uload(m.dkapa, k);
         __syncthreads();
         if (valid) {
             const bool top = BND && k == 1, bot = BND && k == npz;
-            const double dz = uload(m.dzzdz, k), d2z = uload(m.d2zzdz2, k);
-            const double rk = uload(m.rkapa, k), dk = uload(m.dkapa, k);
             const double tmpz = HZ * dz;
             const double tmpz1 = HZ * d2z;
             const double tmpz2 = H2Z * dz * dz;
@@ -663,7 +663,10 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
 #undef RNG
             // ---- output
             if (OPT && p.lshr) p.ftacc[o] = ft;
-            const double F[8] = {fu, fv, fw, fr, ft, w1, w2, w3};
+            // (the boundary conditions overwrite RU, RV and RW of a boundary plane
+            // after every stage: their right-hand sides are not needed there)
+            constexpr bool MOM = !BND || MODE == 0;
+            const double F[8] = {MOM ? fu : 0.0, MOM ? fv : 0.0, MOM ? fw : 0.0, fr, ft, w1, w2, w3};
             if (MODE == 0) {
 #pragma unroll
                 for (int f = 0; f < NF; ++f) fout[f * fs + o] = F[f];

@@ -179,57 +179,83 @@ __device__ __forceinline__ void bcon_column_m(const Params &p, const Metrics &m,
     const long long fs = p.fsize, pl = p.plane, idx = (long long)j * p.npx + i;
     const int nz = p.npz;
     const double C13 = p.c13, C23 = p.c23, C43 = p.c43;
-    auto full = [&](int f, int k) -> double {
-        const long long o = f * fs + (long long)k * pl + idx;
-        double v = f == 4 ? (double)trep(bg.ro32[k], bg.tt32[k], h[o - fs], h[o]) : (double)h[o];
-        if (LAST) v += (double)r_get(rr, fs, f, (long long)k * pl + idx);
-        if (f == 3) v += bg.ro[k];
-        if (f == 4) v += bg.tt[k];
-        return v;
-    };
-    auto residual = [&](int f, int k, double r) {
-        if (LAST) r_put(rr, fs, f, (long long)k * pl + idx, (float)r);
-        else dr[f * fs + (long long)k * pl + idx] = (float)r;
-    };
-    auto put = [&](int f, int k, double v) {
-        const long long o = f * fs + (long long)k * pl + idx;
-        if (f == 4) {
-            const double tp = v - bg.tt[k];
-            const float rh = h[o - fs];
-            const double rhx = LAST ? (double)rh + (double)r_get(rr, fs, 3, (long long)k * pl + idx) : (double)rh;
-            const float hp = (float)pprime(bg.ro[k], bg.tt[k], rhx, tp);
-            h[o] = hp;
-            residual(4, k, tp - (double)trep(bg.ro32[k], bg.tt32[k], rh, hp));
-            return;
-        }
-        if (f == 3) v -= bg.ro[k];
-        const float hn = (float)v;
-        h[o] = hn;
-        residual(f, k, v - (double)hn);
-    };
 #pragma unroll 1
     for (int side = 0; side < 2; ++side) {
         if (side ? !bot : !top) continue;
-        const int a = side ? nz : 1, b = side ? nz - 1 : 2, c = side ? nz - 2 : 3;
-        const double roa = full(3, a), rob = full(3, b), roc = full(3, c);
-        put(0, a, roa * (C43 * full(0, b) / rob - C13 * full(0, c) / roc));
-        put(1, a, roa * (C43 * full(1, b) / rob - C13 * full(1, c) / roc));
-        put(2, a, 0.0);
+        const int a = side ? nz : 1, in = side ? -1 : 1, b = a + in, c = b + in;
+        // everything that is read, before the first store (one wait, not one per
+        // store): stored values (and R words) of the plane and the next two
+        float ha[8], hb[5], hc[5];
+        unsigned wa[4], wb[3], wc[3];
+        const long long oa = (long long)a * pl + idx, ob = (long long)b * pl + idx, oc = (long long)c * pl + idx;
+#pragma unroll
+        for (int f = 0; f < (MAG ? 8 : 5); ++f) ha[f] = h[f * fs + oa];
+#pragma unroll
+        for (int f = 0; f < 5; ++f)
+            if (f != 2) {
+                hb[f] = h[f * fs + ob];
+                hc[f] = h[f * fs + oc];
+            }
+        if (LAST) {
+#pragma unroll
+            for (int w = 0; w < (MAG ? 4 : 3); ++w) wa[w] = rr[w * fs + oa];
+#pragma unroll
+            for (int w = 0; w < 3; ++w) {
+                wb[w] = rr[w * fs + ob];
+                wc[w] = rr[w * fs + oc];
+            }
+        }
+        // full value of field f of plane k from its stored values and R words
+        auto full = [&](int f, int k, const float *hv, const unsigned *wv) __attribute__((always_inline)) {
+            double v = f == 4 ? (double)trep(bg.ro32[k], bg.tt32[k], hv[3], hv[4]) : (double)hv[f];
+            if (LAST) v += (double)r_half(wv[f >> 1], f);
+            if (f == 3) v += bg.ro[k];
+            if (f == 4) v += bg.tt[k];
+            return v;
+        };
+        // new value v of field f of the boundary plane: its split
+        auto put = [&](int f, double v) __attribute__((always_inline)) {
+            float hn, r;
+            if (f == 4) {
+                const double tp = v - bg.tt[a];
+                const double rhx = LAST ? (double)ha[3] + (double)r_half(wa[1], 3) : (double)ha[3];
+                hn = (float)pprime(bg.ro[a], bg.tt[a], rhx, tp);
+                r = (float)(tp - (double)trep(bg.ro32[a], bg.tt32[a], ha[3], hn));
+            } else {
+                hn = (float)v;
+                r = (float)(v - (double)hn);
+            }
+            ha[f] = hn;
+            h[f * fs + oa] = hn;
+            if (LAST) {
+                const unsigned rb = to_bf16(r);
+                unsigned &w = wa[f >> 1];
+                w = (f & 1) ? ((w & 0x0000ffffu) | (rb << 16)) : ((w & 0xffff0000u) | rb);
+            } else {
+                dr[f * fs + oa] = r;
+            }
+        };
+        const double roa = full(3, a, ha, wa), rob = full(3, b, hb, wb), roc = full(3, c, hc, wc);
+        put(0, roa * (C43 * full(0, b, hb, wb) / rob - C13 * full(0, c, hc, wc) / roc));
+        put(1, roa * (C43 * full(1, b, hb, wb) / rob - C13 * full(1, c, hc, wc) / roc));
+        put(2, 0.0);
         const int code = side ? p.izc : p.itc;
         double tnew;
         if (code == 0) {
             tnew = side ? p.tb : 1.0;
         } else {
             const double dz = p.dzf / m.dzzdz[a];
-            tnew = side ? C43 * full(4, b) - C13 * full(4, c) + C23 * dz * p.theta / m.rkapa[a]
-                        : C43 * full(4, b) - C13 * full(4, c) - C23 * dz * p.theta;
+            const double tb = full(4, b, hb, wb), tc = full(4, c, hc, wc);
+            tnew = side ? C43 * tb - C13 * tc + C23 * dz * p.theta / m.rkapa[a] : C43 * tb - C13 * tc - C23 * dz * p.theta;
         }
-        put(4, a, tnew);
-        if (MAG && p.ibc == 0) put(7, a, 0.0);
+        put(4, tnew);
+        if (MAG && p.ibc == 0) put(7, 0.0);
         if (LAST) {
+#pragma unroll
+            for (int w = 0; w < (MAG ? 4 : 3); ++w) rr[w * fs + oa] = wa[w];
             double v[8];
 #pragma unroll
-            for (int f = 0; f < (MAG ? 8 : 5); ++f) v[f] = full(f, a);
+            for (int f = 0; f < (MAG ? 8 : 5); ++f) v[f] = full(f, a, ha, wa);
             const DdPair d = ddpair(m.ddx[i + 1], m.ddy[j + 1], m.ddz[a]);
             cflf_point<MAG>(p, v, d.dd2, d.idd2, 1.0 / m.rkapa[a], cfl);
         }
@@ -264,7 +290,8 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
     const int opt = oly * SW + olx;
     const int gi = i0 + olx - 1, gj = j0 + oly - 1;
     const bool valid = (gi < npx) && (gj < npy);
-    const long long ooff = (long long)wrapi(gj, npy) * npx + wrapi(gi, npx);
+    const int gci = wrapc(gi, npx), gcj = wrapc(gj, npy);  // this lane's column
+    const long long ooff = (long long)gcj * npx + gci;
     int hpt = -1;
     long long hoff = 0;
     if (t < T::NHALO) {
@@ -274,7 +301,7 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
         else if (t < 2 * SW + TY) { hlx = 0; hly = t - 2 * SW + 1; }
         else { hlx = SW - 1; hly = t - 2 * SW - TY + 1; }
         hpt = hly * SW + hlx;
-        hoff = (long long)wrapi(j0 + hly - 1, npy) * npx + wrapi(i0 + hlx - 1, npx);
+        hoff = (long long)wrapc(j0 + hly - 1, npy) * npx + wrapc(i0 + hlx - 1, npx);
     }
     const bool has_h = hpt >= 0;
 
@@ -292,6 +319,27 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
         ring(k, 3, pt) = trep(PLB(ro32, k), PLB(tt32, k), r.v[3], r.v[4]);  // temperature perturbation
     };
 
+    // the per-column values are on their way before the warm-up's loads
+    const rhs_t HX = (rhs_t)p.hx, H2X = (rhs_t)p.h2x, HY = (rhs_t)p.hy, H2Y = (rhs_t)p.h2y;
+    const rhs_t HZ = (rhs_t)p.hz, H2Z = (rhs_t)p.h2z;
+    const int gix = gci + 1, gjy = gcj + 1;
+    const rhs_t dx = (rhs_t)m.dxxdx[gix], d2x = (rhs_t)m.d2xxdx2[gix];
+    const rhs_t dy = (rhs_t)m.dyydy[gjy], d2y = (rhs_t)m.d2yydy2[gjy];
+    const rhs_t hxdx = HX * dx, hydy = HY * dy;
+    const rhs_t h2xdx2 = H2X * dx * dx, h2ydy2 = H2Y * dy * dy;
+    const rhs_t hxd2x = HX * d2x, hyd2y = HY * d2y;
+    const double dt = sc->dt;
+    const double coefg = (MODE == 1 ? p.gam1 : MODE == 2 ? p.gam2 : p.gam3) * dt;
+    const double coefz = (MODE == 1 ? p.zeta1 : p.zeta2) * dt;
+    // stage 3: this column's part of min(dd^2) and its inverse; per plane
+    // the CFL takes dd^2 = min(c_d2, ddz^2) and 1/dd^2 = max(c_id2, 1/ddz^2),
+    // which is 1/min(...) exactly (correctly rounded division is monotone)
+    double c_d2 = 0.0, c_id2 = 0.0;
+    if (MODE == 3) {
+        const double ddx = m.ddx[gix], ddy = m.ddy[gjy];
+        c_d2 = fmin(ddx * ddx, ddy * ddy);
+        c_id2 = 1.0 / c_d2;
+    }
     // warm-up: planes kbeg-1 .. kbeg+1, every load issued before the first is
     // used (lanes without a halo point re-read their own)
     RawF rm_, rp_o, rp_h;
@@ -319,26 +367,6 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
         }
     }
 
-    const rhs_t HX = (rhs_t)p.hx, H2X = (rhs_t)p.h2x, HY = (rhs_t)p.hy, H2Y = (rhs_t)p.h2y;
-    const rhs_t HZ = (rhs_t)p.hz, H2Z = (rhs_t)p.h2z;
-    const int gix = wrapi(gi, npx) + 1, gjy = wrapi(gj, npy) + 1;
-    const rhs_t dx = (rhs_t)m.dxxdx[gix], d2x = (rhs_t)m.d2xxdx2[gix];
-    const rhs_t dy = (rhs_t)m.dyydy[gjy], d2y = (rhs_t)m.d2yydy2[gjy];
-    const rhs_t hxdx = HX * dx, hydy = HY * dy;
-    const rhs_t h2xdx2 = H2X * dx * dx, h2ydy2 = H2Y * dy * dy;
-    const rhs_t hxd2x = HX * d2x, hyd2y = HY * d2y;
-    const double dt = sc->dt;
-    const double coefg = (MODE == 1 ? p.gam1 : MODE == 2 ? p.gam2 : p.gam3) * dt;
-    const double coefz = (MODE == 1 ? p.zeta1 : p.zeta2) * dt;
-    // stage 3: this column's part of min(dd^2) and its inverse; per plane
-    // the CFL takes dd^2 = min(c_d2, ddz^2) and 1/dd^2 = max(c_id2, 1/ddz^2),
-    // which is 1/min(...) exactly (correctly rounded division is monotone)
-    double c_d2 = 0.0, c_id2 = 0.0;
-    if (MODE == 3) {
-        const double ddx = m.ddx[gix], ddy = m.ddy[gjy];
-        c_d2 = fmin(ddx * ddx, ddy * ddy);
-        c_id2 = 1.0 / c_d2;
-    }
     // stage 3: this thread's running CFL maxima/minima over its column
     CflFast cfl_acc = cflf_init();
     const bool frc = bg.force != nullptr && *bg.force_on != 0;
@@ -542,7 +570,9 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
             // FP32 values and carry the residual (+ zeta dt F) in D.  The
             // products dt F are fused into their sums; the residual itself
             // (X minus its stored representation) is exact either way.
-            double Fd[8] = {fu, fv, fw, fr, ft, w1, w2, w3};
+            // (The boundary conditions overwrite RU, RV, RW and T of a boundary
+            // plane after every stage: their right-hand sides are not needed.)
+            double Fd[8] = {BND ? 0.0f : fu, BND ? 0.0f : fv, BND ? 0.0f : fw, fr, BND ? 0.0f : ft, w1, w2, w3};
             Fd[2] += PLB(fwbg, k);
             Fd[4] += PLB(ftbg, k);
             if (frc) {

@@ -23,7 +23,7 @@ def _box(npx, npy, npz, lmag, seed=3):
     return meta, st
 
 
-# 3-plane chunks need npz / 3 of them; 64x32 has 8 tiles, 130x33 27, 200x16 16
+# at most npz - 4 chunks (the first and the last hold three planes); 64x32 has 8 tiles, 130x33 27, 200x16 16
 SIZES = [(9, 6, 4), (64, 32, 5), (64, 32, 6), (64, 32, 7), (130, 33, 10), (200, 16, 23), (66, 5, 33)]
 
 
