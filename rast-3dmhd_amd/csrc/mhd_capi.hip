@@ -56,6 +56,7 @@ struct mhd_ctx {
     std::vector<double> dzzdz, d2zzdz2, ddz, rkapa, dkapa;  // host copies for the background
     DevScalars *sc = nullptr;
     CflSlots *cs = nullptr;             // CFL reduction slots (after sc)
+    DevScalars *report = nullptr;       // pinned: the scalars of the last step of a call (Params::report)
     // closure-corrected step (mixed form)
     mhd_net_t *net = nullptr;
     float *force = nullptr;    // [7][fsize]
@@ -115,11 +116,12 @@ static void free_all(mhd_t *h) {
     if (!h) return;
     (void)hipSetDevice(h->dev);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
-    void *bufs[26] = {h->q[0], h->q[1], h->z, h->hq[0], h->hq[1], h->dr, h->rr, h->bgd, h->bgf, h->bgp,
-                      h->f, h->stage, h->met, h->sc, h->force, h->force_on, h->cx, h->nrm,
+    void *bufs[] = {h->q[0], h->q[1], h->z, h->hq[0], h->hq[1], h->dr, h->rr, h->bgd, h->bgf, h->bgp,
+                      h->f, h->stage, h->sc, h->force, h->force_on, h->cx, h->nrm,
                       h->optmem, h->rs, h->ftacc, h->bgd2, h->bgf2, h->bgp2, h->prof, h->out};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
+    if (h->report) (void)hipHostFree(h->report);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     copy_release();
 }
@@ -216,10 +218,14 @@ extern "C" int mhd_create(const mhd_desc *d, mhd_t **out) {
     }
     h->stage_n = stage_fields(nf, pbytes);
     if (e == hipSuccess) e = hipMalloc(&h->stage, h->stage_n * pbytes);
-    if (e == hipSuccess) e = hipMalloc(&h->met, sizeof(double) * (3 * (d->npx + 2) + 3 * (d->npy + 2) + 5 * (d->npz + 2)));
-    static_assert(sizeof(DevScalars) <= 256, "the slots follow the scalars in one allocation");
-    if (e == hipSuccess) e = hipMalloc(&h->sc, 256 + sizeof(CflSlots));
-    if (e == hipSuccess) h->cs = reinterpret_cast<CflSlots *>(reinterpret_cast<char *>(h->sc) + 256);
+    static_assert(sizeof(DevScalars) <= 256, "the slots and the metrics follow the scalars in one allocation");
+    const size_t nmet = 3 * ((size_t)d->npx + 2) + 3 * ((size_t)d->npy + 2) + 5 * nzp;
+    if (e == hipSuccess) e = hipMalloc(&h->sc, 256 + sizeof(CflSlots) + nmet * sizeof(double));
+    if (e == hipSuccess) {
+        h->cs = reinterpret_cast<CflSlots *>(reinterpret_cast<char *>(h->sc) + 256);
+        h->met = reinterpret_cast<double *>(h->cs + 1);
+    }
+    if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void **>(&h->report), sizeof(DevScalars), hipHostMallocCoherent);
     if (e != hipSuccess) {
         rc = fail(nullptr, MHD_ERR_HIP, "mhd_create: device allocation failed: %s", hipGetErrorString(e));
         free_all(h);
@@ -487,13 +493,15 @@ extern "C" int mhd_download(mhd_t *h, double *ru, double *rv, double *rw, double
 constexpr int STEP_EVENTS = 8;
 
 // The launches of one STEP, optionally bracketed by events (ev[0..7]: pairs
-// around CFL and the three stages).  The stage launches apply the boundary
+// around CFL and the three stages); report: the close writes the step's scalars
+// to the host.  The stage launches apply the boundary
 // conditions, and the third closes the step: the CFL limits of the state a
 // step starts from are reduced by the previous step's third stage.  Only the
 // first step after an upload runs the stand-alone reduction.
-static hipError_t launches(mhd_t *h, hipEvent_t *ev) {
-    const Params &p = h->p;
+static hipError_t launches(mhd_t *h, hipEvent_t *ev, bool report = false) {
     hipError_t e = time_factors(h);
+    Params p = h->p;
+    if (report) p.report = h->report;
     auto rec = [&](int i) {
         if (ev && e == hipSuccess) e = hipEventRecord(ev[i], h->stream);
     };
@@ -529,10 +537,12 @@ static hipError_t launches(mhd_t *h, hipEvent_t *ev) {
     return e;
 }
 
-static int finish(mhd_t *h, double *dt, double *umach) {
+// reported: the last step wrote its scalars to h->report.
+static int finish(mhd_t *h, double *dt, double *umach, bool reported) {
     DevScalars s;
-    HIPCHK(h, hipMemcpyAsync(&s, h->sc, sizeof(s), hipMemcpyDeviceToHost, h->stream));
+    if (!reported) HIPCHK(h, hipMemcpyAsync(&s, h->sc, sizeof(s), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
+    if (reported) s = *h->report;
     if (dt) *dt = s.dt_used;
     if (umach) *umach = s.umach_used;
     if (s.nonfinite)
@@ -570,8 +580,8 @@ extern "C" int mhd_step(mhd_t *h, double *dt, double *umach) {
     int rc = ready(h, "mhd_step");
     if (rc) return rc;
     HIPCHK(h, hipSetDevice(h->dev));
-    HIPCHK(h, launches(h, nullptr));
-    rc = finish(h, dt, umach);
+    HIPCHK(h, launches(h, nullptr, true));
+    rc = finish(h, dt, umach, true);
     return rc ? rc : after_step(h);
 }
 
@@ -581,15 +591,16 @@ extern "C" int mhd_steps(mhd_t *h, int n, double *dt, double *umach) {
     if (n < 0) return fail(h, MHD_ERR_ARG, "mhd_steps: n=%d", n);
     HIPCHK(h, hipSetDevice(h->dev));
     for (int i = 0; i < n; ++i) {
-        HIPCHK(h, launches(h, nullptr));
-        if (h->rebase_every && ++h->since_rebase >= h->rebase_every) {
+        const bool due = h->rebase_every && ++h->since_rebase >= h->rebase_every;
+        HIPCHK(h, launches(h, nullptr, due || i == n - 1));
+        if (due) {
             // the step's DT and UMACH are read (and checked) before the re-centring
-            rc = finish(h, dt, umach);
+            rc = finish(h, dt, umach, true);
             if (rc == MHD_OK) rc = rebase(h);
             if (rc) return rc;
         }
     }
-    return finish(h, dt, umach);
+    return finish(h, dt, umach, n > 0);
 }
 
 extern "C" int mhd_time_steps(mhd_t *h, int n, double *ms_step, double *ms_stage, double *ms_cfl,
@@ -631,7 +642,7 @@ extern "C" int mhd_time_steps(mhd_t *h, int n, double *ms_step, double *ms_stage
     if (ms_stage) *ms_stage = tstage / (3.0 * n);
     if (ms_cfl) *ms_cfl = tcfl / n;
     if (ms_bcon) *ms_bcon = 0.0;  // no launch of its own: part of the stages
-    return finish(h, nullptr, nullptr);
+    return finish(h, nullptr, nullptr, false);
 }
 
 extern "C" int mhd_get_clock(mhd_t *h, int *nit, double *timc, double *timt) {

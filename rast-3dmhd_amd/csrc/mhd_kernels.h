@@ -37,6 +37,8 @@ constexpr long long FIELD_PAD = 1184;
 // Scalars of the step, all as the driver computed them, plus products the
 // reference forms once per FLUXES call (e.g. TMP=OCV*ORE), computed on the
 // host with the same association.
+struct DevScalars;
+
 struct Params {
     int npx, npy, npz;          // interior sizes
     int lmag, lrot, izc, itc, ibc;
@@ -65,6 +67,7 @@ struct Params {
     const double *rom, *wwz, *ttm, *hrad, *radd;
     const double *gx, *gy, *gz; // EXP(CLN*(EXX(I)-XP)**2) etc. per padded index
     double *ftacc;              // LSHR: FT carried between evaluations (one field)
+    DevScalars *report;         // pinned host memory: the step's close also writes its scalars there (null: no)
 };
 
 // Device metric table: padded arrays, same indexing as the reference
@@ -229,6 +232,13 @@ hipError_t launch_cfl(const Params &p, const Metrics &m, const double *q, DevSca
 // Arms the CFL reduction slots of n boxes.
 hipError_t launch_cfl_arm(CflSlots *cs, int n, hipStream_t s);
 hipError_t launch_pack(const Params &p, const double *padded, double *field, hipStream_t s);
+// Upload of all fields and the first CFL reduction in one launch: the padded
+// device arrays f[] into register q0, their z ghost planes into q1 too.
+struct FieldSrc {
+    const double *f[NFIELD];
+};
+hipError_t launch_load(const Params &p, const Metrics &m, const FieldSrc &src, double *q0, double *q1, DevScalars *sc,
+                       CflSlots *cs, hipStream_t s);
 // n fields f[0..n) of register q into the padded arrays dst[0..n), one launch:
 // mode 1 with periodic ghosts, mode 0 with zero ghosts (right-hand sides).
 struct FieldList {

@@ -30,7 +30,7 @@
 // small boxes the latency of a plane's march (3.3 us with one workgroup on a
 // CU) and of the launch, hence few planes per chunk (z_chunks) and three
 // launches per step (64x64x32: 56 us per step, 132 with boundary, CFL and
-// 8-plane launches of their own; 16x16x12 by single steps: 82 against 210).
+// 8-plane launches of their own; 16x16x12 by single steps: 73 against 210).
 //
 // Arithmetic: every expression keeps the reference's left-to-right
 // association and the file is compiled with -ffp-contract=off, so results
@@ -100,7 +100,8 @@ __device__ __forceinline__ void cfl_point(const Params &p, const double *q, doub
 // total.  NaN keys sort above +Inf: they win the max and, through the key of
 // -NaN (below -Inf), the min, so a non-finite state cannot go unnoticed.
 __device__ void cfl_reduce(double mach, double w1, double w2, double w3, double w4, double sf, int lmag,
-                           int clock, DevScalars *__restrict__ sc, CflSlots *__restrict__ cs, int seq, int total) {
+                           int clock, DevScalars *__restrict__ sc, CflSlots *__restrict__ cs, int seq, int total,
+                           DevScalars *report = nullptr) {
     __shared__ unsigned long long red[16][5];
     unsigned long long km = dkey(mach), k1 = dkey(w1), k2 = dkey(w2), k3 = dkey(w3), k4 = dkey(w4);
     // a NaN limit becomes -NaN for the min reduction
@@ -131,7 +132,7 @@ __device__ void cfl_reduce(double mach, double w1, double w2, double w3, double 
     }
     if (threadIdx.x < 64) {
         const unsigned long long k[CFL_KEYS] = {~km, k1, k2, k3, k4};
-        cfl_publish(k, sc, cs, sf, lmag, clock, seq, total);
+        cfl_publish(k, sc, cs, sf, lmag, clock, seq, total, report);
     }
 }
 
@@ -726,7 +727,7 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
     }
     if (MODE == 3) {
         const BoxArgs &l = late_args(args);
-        cfl_reduce(c_mach, c_w1, c_w2, c_w3, c_w4, l.p.sf, l.p.lmag, 1, sc, cs, seq, total);
+        cfl_reduce(c_mach, c_w1, c_w2, c_w3, c_w4, l.p.sf, l.p.lmag, 1, sc, cs, seq, total, l.p.report);
     }
 }
 
@@ -787,6 +788,51 @@ __global__ __launch_bounds__(256) void k_cfl(const Params p, const Metrics m, co
     cfl_reduce(mach, w1, w2, w3, w4, p.sf, p.lmag, 0, sc, cs, blockIdx.x, gridDim.x);
 }
 
+// Upload of all fields at once: thread (column, plane k = 0..npz+1) copies the
+// padded arrays' point into q0, the z ghost planes (which no stage writes) into
+// q1 too, and adds the point's limits to the CFL reduction; the stages write
+// every other point of q1 before they read it.  One launch for what took a
+// pack launch per field and register and k_cfl (64x64x32: 12 us, 17 launches of 59 before,
+// mhd_step_noalloc 100 us, 171 before).
+template <bool MAG>
+__global__ __launch_bounds__(256) void k_load(const Params p, const Metrics m, const FieldSrc src,
+                                              double *__restrict__ q0, double *__restrict__ q1,
+                                              DevScalars *__restrict__ sc, CflSlots *__restrict__ cs) {
+    constexpr int NF = MAG ? 8 : 5, PTS = 2;  // points per thread: fewer workgroups queue at the reduction
+    const int k = blockIdx.y, nxp = p.npx + 2, nyp = p.npy + 2;
+    double mach = 0.0, w1 = INFINITY, w2 = INFINITY, w3 = INFINITY, w4 = INFINITY;
+    double v[PTS][8];
+    int i[PTS], j[PTS];
+    bool on[PTS];
+    long long o[PTS];
+#pragma unroll
+    for (int t = 0; t < PTS; ++t) {
+        const unsigned r = (blockIdx.x * PTS + t) * 256 + threadIdx.x;
+        on[t] = r < (unsigned)p.plane;
+        j[t] = r / (unsigned)p.npx;
+        i[t] = r - j[t] * p.npx;
+        o[t] = k * p.plane + r;
+        const long long a = ((long long)k * nyp + (j[t] + 1)) * nxp + (i[t] + 1);
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+            if (on[t]) v[t][f] = src.f[f][a];
+    }
+#pragma unroll
+    for (int t = 0; t < PTS; ++t)
+        if (on[t]) {
+#pragma unroll
+            for (int f = 0; f < NF; ++f) q0[f * p.fsize + o[t]] = v[t][f];
+            if (k == 0 || k == p.npz + 1) {
+#pragma unroll
+                for (int f = 0; f < NF; ++f) q1[f * p.fsize + o[t]] = v[t][f];
+            } else {
+                cfl_point<MAG>(p, v[t], m.ddx[i[t] + 1], m.ddy[j[t] + 1], m.ddz[k], m.rkcfl[k], mach, w1, w2, w3, w4);
+            }
+        }
+    cfl_reduce(mach, w1, w2, w3, w4, p.sf, p.lmag, 0, sc, cs, blockIdx.y * gridDim.x + blockIdx.x,
+               gridDim.x * gridDim.y);
+}
+
 // Arms the reduction slots of one box per workgroup (a new handle).
 __global__ __launch_bounds__(64) void k_cfl_arm(CflSlots *cs) { cfl_arm(cs + blockIdx.x, threadIdx.x); }
 
@@ -803,25 +849,21 @@ __global__ void k_pack(const Params p, const double *__restrict__ padded, double
     }
 }
 
-// resident fields -> padded Fortran arrays (one field per blockIdx.y);
-// periodic ghost fill (mode 1) or zero ghosts and zero z ghost planes (mode 0,
-// for right-hand sides)
+// resident fields -> padded Fortran arrays (one field per blockIdx.z, planes
+// over blockIdx.y: a point's column is one 32-bit division away); periodic
+// ghost fill (mode 1) or zero ghosts and zero z ghost planes (mode 0, for
+// right-hand sides)
 __global__ void k_unpack(const Params p, const double *__restrict__ q, const FieldList l, int mode) {
-    const double *__restrict__ const field = q + l.f[blockIdx.y] * p.fsize;
-    double *__restrict__ const padded = l.dst[blockIdx.y];
-    const int nxp = p.npx + 2, nyp = p.npy + 2, nzp = p.npz + 2;
-    const long long n = (long long)nxp * nyp * nzp;
-    for (long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x; idx < n;
-         idx += (long long)gridDim.x * blockDim.x) {
-        const long long k = idx / ((long long)nxp * nyp);
-        const long long r = idx - k * nxp * nyp;
-        const int J = (int)(r / nxp), I = (int)(r - (long long)J * nxp);
-        if (mode == 0) {
-            const bool inner = I >= 1 && I <= p.npx && J >= 1 && J <= p.npy && k >= 1 && k <= p.npz;
-            padded[idx] = inner ? field[k * p.plane + (long long)(J - 1) * p.npx + (I - 1)] : 0.0;
-        } else {
-            const int i = wrapi(I - 1, p.npx), j = wrapi(J - 1, p.npy);
-            padded[idx] = field[k * p.plane + (long long)j * p.npx + i];
+    const double *__restrict__ const field = q + l.f[blockIdx.z] * p.fsize;
+    double *__restrict__ const padded = l.dst[blockIdx.z];
+    const unsigned nxp = p.npx + 2, nh = nxp * (unsigned)(p.npy + 2);
+    for (unsigned r = blockIdx.x * blockDim.x + threadIdx.x; r < nh; r += gridDim.x * blockDim.x) {
+        const int J = r / nxp, I = r - J * nxp;
+        const int j = J == 0 ? p.npy - 1 : J > p.npy ? 0 : J - 1, i = I == 0 ? p.npx - 1 : I > p.npx ? 0 : I - 1;
+        const bool ring = I == 0 || I > p.npx || J == 0 || J > p.npy;
+        for (int k = blockIdx.y; k < p.npz + 2; k += gridDim.y) {
+            const bool zero = mode == 0 && (ring || k == 0 || k > p.npz);
+            padded[(long long)k * nh + r] = zero ? 0.0 : field[k * p.plane + (long long)j * p.npx + i];
         }
     }
 }
@@ -978,11 +1020,20 @@ hipError_t launch_pack(const Params &p, const double *padded, double *field, hip
     return hipGetLastError();
 }
 
+hipError_t launch_load(const Params &p, const Metrics &m, const FieldSrc &src, double *q0, double *q1, DevScalars *sc,
+                       CflSlots *cs, hipStream_t s) {
+    if (p.plane > 0x7fffff00 || p.npz > 65533) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)((p.plane + 511) / 512), (unsigned)(p.npz + 2));
+    if (p.lmag) hipLaunchKernelGGL(k_load<true>, grid, dim3(256), 0, s, p, m, src, q0, q1, sc, cs);
+    else hipLaunchKernelGGL(k_load<false>, grid, dim3(256), 0, s, p, m, src, q0, q1, sc, cs);
+    return hipGetLastError();
+}
+
 hipError_t launch_unpack(const Params &p, const double *q, const FieldList &l, int mode, hipStream_t s) {
-    const long long n = (long long)(p.npx + 2) * (p.npy + 2) * (p.npz + 2);
-    long long nb = (n + 255) / 256;
-    if (nb > 8192) nb = 8192;
-    hipLaunchKernelGGL(k_unpack, dim3((unsigned)nb, l.n), dim3(256), 0, s, p, q, l, mode);
+    const long long nh = (long long)(p.npx + 2) * (p.npy + 2);
+    const unsigned gx = (unsigned)((nh + 255) / 256 > 4096 ? 4096 : (nh + 255) / 256);
+    const unsigned gy = (unsigned)(p.npz + 2 > 4096 ? 4096 : p.npz + 2);
+    hipLaunchKernelGGL(k_unpack, dim3(gx, gy, l.n), dim3(256), 0, s, p, q, l, mode);
     return hipGetLastError();
 }
 

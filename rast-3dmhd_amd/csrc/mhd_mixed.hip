@@ -150,7 +150,7 @@ __device__ void cflf_reduce(const Params &p, CflFast c, int clock, DevScalars *_
         k[0] = ~dkey(c.mach);
         // a NaN limit becomes -NaN for the min reduction
         for (int n = 0; n < 4; ++n) k[n + 1] = (w[n] == w[n]) ? dkey(w[n]) : 0ull;
-        cfl_publish(k, sc, cs, p.sf, p.lmag, clock, seq, total);
+        cfl_publish(k, sc, cs, p.sf, p.lmag, clock, seq, total, clock ? p.report : nullptr);
     }
 }
 

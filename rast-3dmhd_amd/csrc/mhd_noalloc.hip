@@ -15,14 +15,14 @@
 // On the host the name `scratch` stands for no device address: its address
 // on each device is looked up once per device with hipGetSymbolAddress and
 // only that pointer is passed to kernels.  Every call re-initialises the
-// scalars and slots with a one-wavefront kernel and overwrites the registers completely
-// (pack of every field, z ghost planes included), so no content of an
-// earlier call is read.  Calls that overlap on one GPU share the array and
+// scalars and slots with a one-wavefront kernel and overwrites what it reads of
+// the registers (k_load, then the stages), so no content of an earlier call is
+// read.  Calls that overlap on one GPU share the array and
 // race.
 //
-// The launches are those of mhd_upload + mhd_step + mhd_download on a
-// handle (the same kernels with the same arguments), so the result is the
-// handle's bit for bit.
+// The launches compute what mhd_upload + mhd_step + mhd_download compute on a
+// handle (the stages are the same kernels with the same arguments; the CFL
+// reduction is exact in any order), so the result is the handle's bit for bit.
 
 #include <hip/hip_runtime.h>
 
@@ -134,13 +134,10 @@ extern "C" int mhd_step_noalloc(const mhd_desc *d, const mhd_dev_metrics *met, d
     s0.timt = timi + *timc;
     hipLaunchKernelGGL(k_noalloc_init, dim3(1), dim3(64), 0, s, sc, s0, cs);
     NACHK(hipGetLastError());
-    // upload: both registers carry the z ghost planes (as mhd_upload)
-    for (int f = 0; f < nf; ++f) {
-        NACHK(launch_pack(p, state[f], q[0] + (size_t)f * p.fsize, s));
-        NACHK(launch_pack(p, state[f], q[1] + (size_t)f * p.fsize, s));
-    }
-    // step (as mhd_step on a freshly uploaded handle)
-    NACHK(launch_cfl(p, m, q[0], sc, cs, s));
+    // upload and the first CFL reduction (as mhd_upload and mhd_step on a fresh handle)
+    FieldSrc src{};
+    for (int f = 0; f < nf; ++f) src.f[f] = state[f];
+    NACHK(launch_load(p, m, src, q[0], q[1], sc, cs, s));
     int a = 0, b = 1;
     for (int st = 1; st <= 3; ++st) {
         NACHK(launch_stage(st, p, m, q[a], q[b], z, nullptr, sc, cs, s));
