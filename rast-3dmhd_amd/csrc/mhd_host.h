@@ -139,7 +139,7 @@ inline Params params_from_desc(const mhd_desc *d) {
     p.dh = d->dh; p.dv = d->dv; p.tu = d->tu; p.dztu = d->dztu; p.dztb = d->dztb;
     p.rlax = d->rlax; p.tstart = d->tstart; p.toff = d->toff; p.tp = d->tp; p.tc = d->tc; p.hh = d->hh;
     p.tpr = d->tp;
-    p.opt = (p.id != 0 || p.lrem || p.lshr || p.rlax > 0.0 || p.itc == 2) ? 1 : 0;
+    p.opt = p.lrem || p.lshr || p.rlax > 0.0 || p.itc == 2 ? 2 : p.id != 0 ? 1 : 0;
     return p;
 }
 

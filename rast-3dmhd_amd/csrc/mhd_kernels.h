@@ -57,7 +57,7 @@ struct Params {
     double t_cross;             // C13*ORE (sub:1930)
     double t_ohm;               // OBETA*ORM*OCV (sub:2287)
     // Optional branches of FLUXES/BCON (FP64 form; all zero: the main path).
-    int opt;                    // any branch below that the stage kernel must see
+    int opt;                    // branches below that the stage kernel must see: 0 none, 1 ID alone, 2 others
     int id, lrem, lshr, mirror; // mirror: ID or LREM (ghost RO planes mirrored, sub:1301-1310)
     int npey, npez;             // decomposition whose summation order the means follow
     double dh, dv, tu, dztu, dztb, rlax, tstart, toff, tp, tc, hh;

@@ -234,11 +234,13 @@ constexpr int stage_lds_bytes() {
 // right-hand side F to fout; MODE 1..3 performs RK3 stage s with the boundary
 // conditions on the boundary planes it holds.  The whole workgroup calls it
 // with the same arguments.
-// OPT instantiates the optional branches of FLUXES (density diffusion,
-// Rempel conduction, shear boundaries, flux relaxation, embedded heat loss;
-// the per-plane tables come from mhd_opt.hip); the main path has none of
-// their code.
-template <int TY, bool MAG, int MODE, bool OPT = false>
+// OPT instantiates the optional branches of FLUXES (Params::opt; the per-plane
+// tables come from mhd_opt.hip): 1 density diffusion alone, 2 any of density
+// diffusion, Rempel conduction, shear boundaries, flux relaxation and embedded
+// heat loss; the main path has none of their code.  Form 2 spills 60-90
+// registers of each lane, form 1 none (96x96x48 with density diffusion, stages
+// 1 to 3: 53, 81, 85 us as form 2, 35, 40, 44 us as form 1).
+template <int TY, bool MAG, int MODE, int OPT = 0>
 __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, ArgPtr args,
                                            const double *__restrict__ qin,
                                            double *__restrict__ qout, double *__restrict__ zr,
@@ -308,7 +310,7 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
     double c_mach = 0.0, c_w1 = INFINITY, c_w2 = INFINITY, c_w3 = INFINITY, c_w4 = INFINITY;
     const double c_ddx = MODE == 3 ? m.ddx[gix] : 0.0, c_ddy = MODE == 3 ? m.ddy[gjy] : 0.0;
     // the embedded heat loss's per-column Gaussians, read once
-    const double c_gx = (OPT && p.itc == 2) ? p.gx[gix] : 0.0, c_gy = (OPT && p.itc == 2) ? p.gy[gjy] : 0.0;
+    const double c_gx = (OPT == 2 && p.itc == 2) ? p.gx[gix] : 0.0, c_gy = (OPT == 2 && p.itc == 2) ? p.gy[gjy] : 0.0;
     // Warm-up: planes kbeg-1 (own values + ring), kbeg and kbeg+1 (LDS + ring).
     // Every load is issued before the first is used: a chunk then pays one
     // memory latency before its march instead of three.
@@ -347,7 +349,7 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
 
     // the per-column metrics arrive before the march, not inside its first plane
     settle(dx), settle(d2x), settle(dy), settle(d2y), settle(c_ddx), settle(c_ddy);
-    if (OPT) settle(c_gx), settle(c_gy);
+    if (OPT == 2) settle(c_gx), settle(c_gy);
 
     // One plane of the march.  BND instantiates the boundary-plane form
     // (one-sided z stencils, extra planes read directly); the interior form
@@ -464,7 +466,7 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
             const double typ = CUR(S_TT, SW), tym = CUR(S_TT, -SW);
             const double tzp = tt_p, tzm = tt_m;
             double ft;
-            if (OPT && p.lshr) {
+            if (OPT == 2 && p.lshr) {
                 // no advection; FT keeps the previous evaluation's values (sub:1493)
                 ft = p.ftacc[o];
             } else {
@@ -474,7 +476,7 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
             }
 
             // ---- conduction (sub:1584-1610)
-            if (OPT && p.lrem) {
+            if (OPT == 2 && p.lrem) {
                 // of the perturbations W1 = TT - TTM only, plus the mean profile's
                 // radiative heating HRAD (sub:1536-1581)
                 const double tc = p.t_cond, tmk = uload(p.ttm, k);
@@ -491,7 +493,7 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
                 ft = ft + ((tzp - tzm) * tmpz1 + (tzp - 2.0 * tt0 + tzm) * tmpz2) * rinv * tc * rk;
                 ft = ft + (tzp - tzm) * HZ * dz * rinv * tc * dk;
             }
-            if (OPT) {
+            if (OPT == 2) {
                 // flux relaxation (sub:1757-1765) and embedded heat loss (sub:1783-1806)
                 if (p.rlax > 0.0) ft = ft + uload(p.radd, k);
                 if (p.itc == 2) {
@@ -503,7 +505,7 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
                 }
             }
             // LSHR: no viscous or compressional heating (sub:1903-2101)
-            const bool heat = !(OPT && p.lshr);
+            const bool heat = !(OPT == 2 && p.lshr);
 
             // ---- viscous Laplacians (sub:1818-1886)
             fu = fu + ORE * (C43 * ((uxp - uxm) * HX * d2x + (uxp - 2.0 * u0 + uxm) * H2X * dx * dx)
@@ -663,7 +665,7 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
 #undef NXT
 #undef RNG
             // ---- output
-            if (OPT && p.lshr) p.ftacc[o] = ft;
+            if (OPT == 2 && p.lshr) p.ftacc[o] = ft;
             // (the boundary conditions overwrite RU, RV and RW of a boundary plane
             // after every stage: their right-hand sides are not needed there)
             constexpr bool MOM = !BND || MODE == 0;
@@ -682,7 +684,7 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
                     if (MODE < 3) __builtin_nontemporal_store(qn[f] + coefz * F[f], &zr[f * fs + o]);
                 }
                 if (MODE == 3 && !top && !bot)
-                    cfl_point<MAG>(p, qn, c_ddx, c_ddy, uload(m.ddz, k), OPT ? uload(m.rkcfl, k) : rk, c_mach, c_w1,
+                    cfl_point<MAG>(p, qn, c_ddx, c_ddy, uload(m.ddz, k), OPT == 2 ? uload(m.rkcfl, k) : rk, c_mach, c_w1,
                                    c_w2, c_w3, c_w4);
             }
             // own raw values of plane k become the k-1 values of the next plane
@@ -732,7 +734,7 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
 }
 
 // Single box: workgroup -> (tile, z chunk), XCD-aware.
-template <int TY, bool MAG, int MODE, bool OPT>
+template <int TY, bool MAG, int MODE, int OPT>
 __global__ __launch_bounds__(TX *TY, 2) void k_stage(const BoxArgs b,
                                                   const double *__restrict__ qin,
                                                   double *__restrict__ qout,
@@ -917,7 +919,7 @@ __global__ void k_box_filter(const Params p, const double *__restrict__ q, int n
 // ---------------------------------------------------------------------------
 // launchers
 
-template <int TY, bool MAG, int MODE, bool OPT>
+template <int TY, bool MAG, int MODE, int OPT>
 static hipError_t launch_stage_o(const Params &p, const Metrics &m, const double *qin, double *qout, double *z,
                                  double *fout, DevScalars *sc, CflSlots *cs, hipStream_t s) {
     constexpr int lds = stage_lds_bytes<TY, MAG>();
@@ -936,8 +938,10 @@ static hipError_t launch_stage_o(const Params &p, const Metrics &m, const double
 template <int TY, bool MAG, int MODE>
 static hipError_t launch_stage_t(const Params &p, const Metrics &m, const double *qin, double *qout, double *z,
                                  double *fout, DevScalars *sc, CflSlots *cs, hipStream_t s) {
-    if (p.opt) return launch_stage_o<TY, MAG, MODE, true>(p, m, qin, qout, z, fout, sc, cs, s);
-    return launch_stage_o<TY, MAG, MODE, false>(p, m, qin, qout, z, fout, sc, cs, s);
+    if (p.opt == 2 || (p.opt && TY != 4)) return launch_stage_o<TY, MAG, MODE, 2>(p, m, qin, qout, z, fout, sc, cs, s);
+    if constexpr (TY == 4)  // (8-row tiles are for trials: form 2 serves them)
+        if (p.opt) return launch_stage_o<TY, MAG, MODE, 1>(p, m, qin, qout, z, fout, sc, cs, s);
+    return launch_stage_o<TY, MAG, MODE, 0>(p, m, qin, qout, z, fout, sc, cs, s);
 }
 
 template <int TY>
