@@ -4,9 +4,9 @@
  * No counterpart in the reference, which steps one domain per MPI job.
  * An ensemble holds nbox independent boxes, each with its own sizes,
  * parameters (mhd_desc), metrics, state, adaptive DT and clock, resident on
- * the current HIP device.  One RK3 step of the whole ensemble is seven
- * launches: three persistent stage launches over a work table that covers
- * every box, three boundary-plane launches and one per-box DT/clock update.
+ * the current HIP device.  One RK3 step of the whole ensemble is three
+ * launches over a work table that covers every box: the stages, which apply
+ * the boundary conditions and, the third, close each box's step (DT, clock).
  * Repeated steps are replayed from a captured HIP graph.  The tile shape,
  * z-chunk depth and persistent grid size come from mhd_ens_autotune,
  * mhd_ens_set_tiling or mhd_ens_set_tile.
@@ -56,16 +56,16 @@ int mhd_ens_set_fixed_dt(mhd_ens_t *e, int box, double dt);
  * replay from a captured HIP graph (1) or direct launches (0). */
 int mhd_ens_steps(mhd_ens_t *e, int n, int use_graph, double *dt, double *umach);
 
-/* Tiling of the batched launches: tile_y (4 or 8 rows of 64 columns),
- * kdepth (planes per z chunk; 0 = whole column) and grid (persistent
+/* Tiling of the batched launches: tile_y (4: tiles of up to 256 points, 64x4 or
+ * of a shape fitted to each box's width; 8: 64x8), kdepth (planes per z chunk; 0 = whole column) and grid (persistent
  * workgroups; 0 = one workgroup per work item).  get_tiling reports the
  * rows of the current tile whatever its width. */
 int mhd_ens_set_tiling(mhd_ens_t *e, int tile_y, int kdepth, int grid);
 int mhd_ens_get_tiling(const mhd_ens_t *e, int *tile_y, int *kdepth, int *grid);
 
 /* The same with the tile width: tile_x x tile_y is 64x4, 64x8, or (mixed
- * form only) 32x8, which leaves fewer lanes idle on boxes whose rows are
- * not a multiple of 64 points.  The results do not depend on the tiling. */
+ * form only) 32x8; 64x4 is fitted to each box (see mhd_ens_set_tiling), 32x8
+ * is that shape for all.  The results do not depend on the tiling. */
 int mhd_ens_set_tile(mhd_ens_t *e, int tile_x, int tile_y, int kdepth, int grid);
 int mhd_ens_get_tile(const mhd_ens_t *e, int *tile_x, int *tile_y, int *kdepth, int *grid);
 

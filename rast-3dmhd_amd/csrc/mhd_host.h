@@ -85,18 +85,60 @@ inline int check_desc(const mhd_desc *d, char *msg, size_t len) {
 // at most 32 planes: over a longer march the tiles that share halo rows drift
 // apart and re-read them from HBM (512x512x256 FP64, 128 planes: 14% more
 // bytes fetched).
-inline int z_chunks(int npz, int ntiles, int occ, double alone, double more) {
+struct ZSplit {
+    int nc;
+    double time;  // of a launch, us
+};
+inline ZSplit z_chunks(int npz, int ntiles, int occ, double alone, double more) {
     constexpr int CUS = 256;
-    int best = 1;
-    double tbest = 0.0;
-    for (int nc = (npz + 31) / 32; nc <= max_chunks(npz) || nc == 1; ++nc) {
+    ZSplit best{0, 0.0};
+    for (int nc = (npz + 31) / 32; nc <= max_chunks(npz) || !best.nc; ++nc) {
         const long long n = (long long)ntiles * nc, slots = (long long)CUS * occ;
         const long long rest = (n % slots + CUS - 1) / CUS;
         const double round = alone + (occ - 1) * more, last = rest ? alone + (rest - 1) * more : 0.0;
         const double t = (chunk_depth(npz, nc) + 1.5) * ((double)(n / slots) * round + last);
-        if (tbest == 0.0 || t < tbest) {
-            tbest = t;
-            best = nc;
+        if (!best.nc || t < best.time) best = ZSplit{nc, t};
+    }
+    return best;
+}
+
+// The tile of a box: 64x4, or one of at most 256 points fitted to its width if
+// that saves 5% (mixed: 12%) of time(tiles) times a tile's own cost.  64-column
+// tiles leave up to half of the lanes of a narrow or ragged box idle (a 40-column
+// box: 24 of 64).  Fitted tiles are npx / m columns wide, so that whole rows of a
+// narrow box are one contiguous run of memory.  Against them speak the ends of a
+// tile's rows that are not on 64 bytes, where two tiles write a piece each (3% of
+// a tile's time per end in FP64, 9% in the mixed form: 320x320x100 mixed, 64x4 2.1
+// us a tile, 54x4 3.1, 40x6 3.3), and more, shorter rows (5% each).  Steps from
+// 64x4 to fitted, FP64: 40x72x54 64 -> 55 us (40x6), 72x200x64 249 -> 200 (72x3),
+// 130x90x41 hydro 91 -> 85 (44x5); mixed: 72x200x64 164 -> 119 (72x3), 150x300x100
+// 628 -> 559 (75x3).  Left at 64x4: 300x300x100 FP64 (1595; 50x5: 1852),
+// 160x160x64 mixed (185; 80x3: 189).
+template <class Time>
+inline TileShape fit_tile(int npx, int npy, bool mixed, Time time) {
+    const int esz = mixed ? 4 : 8, points = mixed ? FIT_POINTS_MIXED : FIT_POINTS_FP64;
+    auto cost = [&](TileShape t) {
+        const bool rows = t.w == npx;  // whole rows: the ends are the tile's two
+        const long long run = (long long)t.w * (rows ? t.h : 1) * esz, pitch = rows ? 64 : (long long)npx * esz;
+        int unit = 64;
+        while (run % unit || pitch % unit) unit /= 2;
+        const double ends = (rows ? 2 : 2 * t.h) * (1.0 - unit / 64.0);
+        const double more = rows || t.h < 4 ? 0.0 : 0.05 * (t.h - 4);
+        return time(tile_count(npx, npy, t)) * (1.0 + (mixed ? 0.09 : 0.03) * ends + more);
+    };
+    TileShape best{64, 4};
+    double least = (mixed ? 0.88 : 0.95) * cost(best);
+    for (int m = (npx + 95) / 96; m <= npx; ++m) {
+        const int w = (npx + m - 1) / m;
+        if (m > 1 && w < 32) break;
+        int h = 256 / w < npy ? 256 / w : npy;
+        while ((w + 2) * (h + 2) > points) --h;
+        const int n = (npy + h - 1) / h;
+        const TileShape t{w, (npy + n - 1) / n};
+        const double c = cost(t);
+        if (c < least) {
+            least = c;
+            best = t;
         }
     }
     return best;
@@ -111,13 +153,6 @@ inline Params params_from_desc(const mhd_desc *d) {
     p.izc = d->izcon; p.itc = d->itcon; p.ibc = d->ibcon;
     p.tile_y = 4;
     if (const char *ty = getenv("RAST3DMHD_TILE_Y")) p.tile_y = atoi(ty) == 8 ? 8 : 4;
-    {
-        // workgroups per CU by LDS and registers (64x8 tiles: half)
-        const bool mixed = d->precision == MHD_MIXED;
-        const int occ = (mixed ? (d->lmag ? 3 : 4) : 2) / (p.tile_y == 8 ? 2 : 1);
-        const int ntiles = ((d->npx + 63) / 64) * ((d->npy + p.tile_y - 1) / p.tile_y);
-        p.nchunks = z_chunks(d->npz, ntiles, occ, mixed ? 2.6 : 3.3, mixed ? 0.9 : 2.4);
-    }
     p.plane = (long long)d->npx * d->npy;
     p.fsize = p.plane * (d->npz + 2) + FIELD_PAD;
     p.hx = d->hx; p.h2x = d->h2x; p.hy = d->hy; p.h2y = d->h2y; p.hz = d->hz; p.h2z = d->h2z;
@@ -140,6 +175,20 @@ inline Params params_from_desc(const mhd_desc *d) {
     p.rlax = d->rlax; p.tstart = d->tstart; p.toff = d->toff; p.tp = d->tp; p.tc = d->tc; p.hh = d->hh;
     p.tpr = d->tp;
     p.opt = p.lrem || p.lshr || p.rlax > 0.0 || p.itc == 2 ? 2 : p.id != 0 ? 1 : 0;
+    {
+        // workgroups per CU by LDS and registers (64x8 tiles: half)
+        const bool mixed = d->precision == MHD_MIXED;
+        const int occ = (mixed ? (d->lmag ? 3 : 4) : 2) / (p.tile_y == 8 ? 2 : 1);
+        auto split = [&](int ntiles) { return z_chunks(d->npz, ntiles, occ, mixed ? 2.6 : 3.3, mixed ? 0.9 : 2.4); };
+        if (p.tile_y == 4 && p.opt != 2) {
+            const TileShape t = fit_tile(d->npx, d->npy, mixed, [&](int ntiles) { return split(ntiles).time; });
+            if (t.w != 64 || t.h != 4) {
+                p.tile_w = t.w;
+                p.tile_h = t.h;
+            }
+        }
+        p.nchunks = split(tiles_of(p)).nc;
+    }
     return p;
 }
 

@@ -43,6 +43,7 @@ struct Params {
     int npx, npy, npz;          // interior sizes
     int lmag, lrot, izc, itc, ibc;
     int tile_y;                 // rows per stage-kernel tile (4 or 8)
+    int tile_w, tile_h;         // fitted tile of at most 256 points (fit_tile); 0: 64 x tile_y
     int nchunks;                // z chunks of a stage launch (z_chunks)
     long long plane;            // npx*npy
     long long fsize;            // field stride: plane*(npz+2) values incl. z ghost planes, + FIELD_PAD
@@ -167,6 +168,7 @@ inline size_t resid_bytes(int nf, long long fsize) { return (size_t)((nf + 1) / 
 // number seq of the box's total items.
 struct StageItem {
     int box, i0, j0, kbeg, kend, seq, total;
+    int w, h;  // its tile's columns and rows
 };
 
 // Planes 1..npz of a box split into nc chunks: chunk c covers the planes
@@ -186,6 +188,19 @@ __host__ __device__ inline int chunk_begin(int npz, int nc, int c) {
     if (nc == 2) return 1 + npz / 2;
     const int e = chunk_depth(npz, nc), rest = npz - 2 * e;
     return 1 + e + (int)((long long)(c - 1) * rest / (nc - 2));
+}
+
+// Points of an LDS plane of a fitted tile with its halo: what lets two (FP64)
+// or three (mixed) workgroups share a CU's LDS.
+constexpr int FIT_POINTS_FP64 = 400, FIT_POINTS_MIXED = 416;
+
+// Tile of w columns x h rows, one point per thread.
+struct TileShape {
+    int w, h;
+};
+inline int tile_count(int npx, int npy, TileShape t) { return ((npx + t.w - 1) / t.w) * ((npy + t.h - 1) / t.h); }
+inline int tiles_of(const Params &p) {
+    return tile_count(p.npx, p.npy, p.tile_w ? TileShape{p.tile_w, p.tile_h} : TileShape{64, p.tile_y});
 }
 
 __host__ __device__ inline unsigned long long dkey(double v) {

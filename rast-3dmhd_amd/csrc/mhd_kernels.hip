@@ -17,8 +17,8 @@
 // bottom z ghost planes, planes 1..npz the reference's K=2..NPZ+1.  There are
 // no x/y ghost cells: neighbours wrap periodically.
 //
-// Stage kernel organisation.  A workgroup owns a 64 x TY column tile and
-// marches down a chunk of planes.  LDS holds the raw fields of planes k and
+// Stage kernel organisation.  A workgroup owns a 64 x TY column tile, or one of
+// up to 256 points fitted to the box (TY = 0, see fit_tile), and marches down a chunk of planes.  LDS holds the raw fields of planes k and
 // k+1 with a one-point halo (double buffer) and a three-plane ring of the
 // velocities u,v,w (needed at (i+-1,k+-1) and (j+-1,k+-1) by the cross terms
 // of the viscous stress).  Plane k+2 is loaded into registers while plane k
@@ -52,6 +52,11 @@ struct Tile {
     static constexpr int SP = SW * SH;      // points per LDS plane
     static constexpr int NHALO = SP - NT;   // halo points, one per thread for t < NHALO
     static_assert(NHALO <= NT, "one halo point per thread at most");
+};
+// Fitted tiles (Params::tile_w x tile_h, see fit_tile): 256 threads.
+template <>
+struct Tile<0> {
+    static constexpr int TY = 4, NT = 256, SW = 0, SP = FIT_POINTS_FP64;
 };
 
 // Raw-field slots of the LDS planes (resident field order).
@@ -246,9 +251,11 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
                                            double *__restrict__ qout, double *__restrict__ zr,
                                            double *__restrict__ fout, DevScalars *__restrict__ sc,
                                            CflSlots *__restrict__ cs, int i0, int j0, int kbeg, int kend, int seq,
-                                           int total, double *lds) {
+                                           int total, double *lds, int tw = 0, int th = 0) {
     using T = Tile<TY>;
-    constexpr int SW = T::SW, SP = T::SP;
+    constexpr bool FIT = TY == 0;
+    constexpr int SP = T::SP;
+    const int W = FIT ? tw : TX, H = FIT ? th : TY, SW = FIT ? tw + 2 : T::SW;
     constexpr int NF = MAG ? 8 : 5;
     double *const s_cur = lds;                  // [2][NF][SP]: raw planes k, k+1 (by parity)
     double *const s_ring = lds + 2 * NF * SP;   // [3][3][SP]: u, v, w of planes k-1, k, k+1
@@ -258,21 +265,23 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
     const long long fs = p.fsize, pl = p.plane;
 
     // own point
-    const int olx = t % TX + 1, oly = t / TX + 1;
+    // (threads past a fitted tile's last point double that point)
+    const int own = FIT && t >= W * H ? W * H - 1 : t;
+    const int oly = own / W + 1, olx = own - (oly - 1) * W + 1;
     const int opt = oly * SW + olx;
     const int gi = i0 + olx - 1, gj = j0 + oly - 1;
-    const bool valid = (gi < npx) && (gj < npy);
+    const bool valid = (gi < npx) && (gj < npy) && (!FIT || t < W * H);
     const int gci = wrapc(gi, npx), gcj = wrapc(gj, npy);  // this lane's column
     const long long ooff = (long long)gcj * npx + gci;
     // halo point (t < NHALO): top row, bottom row, left column, right column
     int hpt = -1;
     long long hoff = 0;
-    if (t < T::NHALO) {
+    if (t < 2 * (SW + H)) {
         int hlx, hly;
         if (t < SW) { hlx = t; hly = 0; }
-        else if (t < 2 * SW) { hlx = t - SW; hly = T::SH - 1; }
-        else if (t < 2 * SW + TY) { hlx = 0; hly = t - 2 * SW + 1; }
-        else { hlx = SW - 1; hly = t - 2 * SW - TY + 1; }
+        else if (t < 2 * SW) { hlx = t - SW; hly = H + 1; }
+        else if (t < 2 * SW + H) { hlx = 0; hly = t - 2 * SW + 1; }
+        else { hlx = SW - 1; hly = t - 2 * SW - H + 1; }
         hpt = hly * SW + hlx;
         hoff = (long long)wrapc(j0 + hly - 1, npy) * npx + wrapc(i0 + hlx - 1, npx);
     }
@@ -735,7 +744,7 @@ __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, Ar
 
 // Single box: workgroup -> (tile, z chunk), XCD-aware.
 template <int TY, bool MAG, int MODE, int OPT>
-__global__ __launch_bounds__(TX *TY, 2) void k_stage(const BoxArgs b,
+__global__ __launch_bounds__(Tile<TY>::NT, 2) void k_stage(const BoxArgs b,
                                                   const double *__restrict__ qin,
                                                   double *__restrict__ qout,
                                                   double *__restrict__ zr,
@@ -744,19 +753,20 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage(const BoxArgs b,
                                                   int nchunks) {
     extern __shared__ double lds[];
     const Params &p = b.p;
-    const int ntx = (p.npx + TX - 1) / TX, nty = (p.npy + TY - 1) / TY;
+    const int W = TY ? TX : p.tile_w, H = TY ? TY : p.tile_h;
+    const int ntx = (p.npx + W - 1) / W, nty = (p.npy + H - 1) / H;
     const TileChunk tc = tile_of(blockIdx.x, ntx * nty, nchunks);
     const int tz = tc.chunk, tyb = tc.tile / ntx, txb = tc.tile - tyb * ntx;
     const int kbeg = chunk_begin(p.npz, nchunks, tz), kend = chunk_begin(p.npz, nchunks, tz + 1) - 1;
-    stage_tile<TY, MAG, MODE, OPT>(p, b.m, kernel_args(), qin, qout, zr, fout, sc, cs, txb * TX, tyb * TY, kbeg, kend,
-                                   blockIdx.x, gridDim.x, lds);
+    stage_tile<TY, MAG, MODE, OPT>(p, b.m, kernel_args(), qin, qout, zr, fout, sc, cs, txb * W, tyb * H, kbeg, kend,
+                                   blockIdx.x, gridDim.x, lds, W, H);
 }
 
 // Ensemble: a persistent grid walks the work-item table of all boxes with a
 // static stride (deterministic; every workgroup leaves after its last item).
 // Register a of every box is the input, 1-a the output.
 template <int TY, bool MAG, int MODE>
-__global__ __launch_bounds__(TX *TY, 2) void k_stage_batch(const BoxDev *__restrict__ boxes,
+__global__ __launch_bounds__(Tile<TY>::NT, 2) void k_stage_batch(const BoxDev *__restrict__ boxes,
                                                         const StageItem *__restrict__ items, int nitems, int a) {
     extern __shared__ double lds[];
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
@@ -765,7 +775,7 @@ __global__ __launch_bounds__(TX *TY, 2) void k_stage_batch(const BoxDev *__restr
         const BoxDev &B = box_at(boxes, it.box);
         __syncthreads();  // the previous item's last LDS reads are done
         stage_tile<TY, MAG, MODE>(B.a.p, B.a.m, (ArgPtr)&B.a, B.q[a], B.q[1 - a], B.z, nullptr, B.sc, B.cs, it.i0, it.j0, it.kbeg,
-                                  it.kend, it.seq, it.total, lds);
+                                  it.kend, it.seq, it.total, lds, it.w, it.h);
     }
 }
 
@@ -929,8 +939,7 @@ static hipError_t launch_stage_o(const Params &p, const Metrics &m, const double
         if (e != hipSuccess) return e;
     }
     const int nch = p.nchunks;
-    const int ntiles = ((p.npx + TX - 1) / TX) * ((p.npy + TY - 1) / TY);
-    hipLaunchKernelGGL((k_stage<TY, MAG, MODE, OPT>), dim3(ntiles * nch), dim3(TX * TY), lds, s, BoxArgs{p, m, {}},
+    hipLaunchKernelGGL((k_stage<TY, MAG, MODE, OPT>), dim3(tiles_of(p) * nch), dim3(Tile<TY>::NT), lds, s, BoxArgs{p, m, {}},
                        qin, qout, z, fout, sc, cs, nch);
     return hipGetLastError();
 }
@@ -938,8 +947,9 @@ static hipError_t launch_stage_o(const Params &p, const Metrics &m, const double
 template <int TY, bool MAG, int MODE>
 static hipError_t launch_stage_t(const Params &p, const Metrics &m, const double *qin, double *qout, double *z,
                                  double *fout, DevScalars *sc, CflSlots *cs, hipStream_t s) {
-    if (p.opt == 2 || (p.opt && TY != 4)) return launch_stage_o<TY, MAG, MODE, 2>(p, m, qin, qout, z, fout, sc, cs, s);
-    if constexpr (TY == 4)  // (8-row tiles are for trials: form 2 serves them)
+    if constexpr (TY != 0)  // (fitted tiles are chosen without form 2, see params_from_desc)
+        if (p.opt == 2 || (p.opt && TY == 8)) return launch_stage_o<TY, MAG, MODE, 2>(p, m, qin, qout, z, fout, sc, cs, s);
+    if constexpr (TY != 8)  // (8-row tiles are for trials: form 2 serves them)
         if (p.opt) return launch_stage_o<TY, MAG, MODE, 1>(p, m, qin, qout, z, fout, sc, cs, s);
     return launch_stage_o<TY, MAG, MODE, 0>(p, m, qin, qout, z, fout, sc, cs, s);
 }
@@ -965,6 +975,7 @@ static hipError_t launch_stage_ty(int mode, const Params &p, const Metrics &m, c
 
 hipError_t launch_stage(int mode, const Params &p, const Metrics &m, const double *qin, double *qout,
                         double *z, double *fout, DevScalars *sc, CflSlots *cs, hipStream_t s) {
+    if (p.tile_w) return launch_stage_ty<0>(mode, p, m, qin, qout, z, fout, sc, cs, s);
     if (p.tile_y == 8) return launch_stage_ty<8>(mode, p, m, qin, qout, z, fout, sc, cs, s);
     return launch_stage_ty<4>(mode, p, m, qin, qout, z, fout, sc, cs, s);
 }
@@ -978,7 +989,7 @@ static hipError_t launch_batch_t(const BoxDev *boxes, const StageItem *items, in
         hipError_t e = lds_limit_once(attr, reinterpret_cast<const void *>(&k_stage_batch<TY, MAG, MODE>), lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((k_stage_batch<TY, MAG, MODE>), dim3(grid), dim3(TX * TY), lds, s, boxes, items, nitems, a);
+    hipLaunchKernelGGL((k_stage_batch<TY, MAG, MODE>), dim3(grid), dim3(Tile<TY>::NT), lds, s, boxes, items, nitems, a);
     return hipGetLastError();
 }
 
@@ -998,7 +1009,7 @@ static hipError_t launch_batch_ty(int mode, int lmag, const BoxDev *boxes, const
 hipError_t launch_stage_batch(int mode, int tile_y, int lmag, const BoxDev *boxes, const StageItem *items,
                               int nitems, int grid, int a, hipStream_t s) {
     if (tile_y == 8) return launch_batch_ty<8>(mode, lmag, boxes, items, nitems, grid, a, s);
-    return launch_batch_ty<4>(mode, lmag, boxes, items, nitems, grid, a, s);
+    return launch_batch_ty<0>(mode, lmag, boxes, items, nitems, grid, a, s);
 }
 
 hipError_t launch_cfl(const Params &p, const Metrics &m, const double *q, DevScalars *sc, CflSlots *cs,

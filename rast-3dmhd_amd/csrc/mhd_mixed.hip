@@ -46,25 +46,25 @@ constexpr int MTX = 64;
 // Arithmetic type of the perturbation right-hand side (storage stays FP32).
 typedef float rhs_t;
 
-// Tile of TX columns x TY rows, one point per thread (TX = 64: one row per
-// wavefront; TX = 32: two rows per wavefront, for narrow ensemble boxes).
-template <int TX_, int TY_>
+// Tile of MTX columns x TY rows, one point per thread; TY = 0: fitted tiles of
+// at most 256 points (Params::tile_w x tile_h, see fit_tile).
+template <int TY_>
 struct MTile {
-    static constexpr int TX = TX_;
-    static constexpr int TY = TY_;
-    static constexpr int NT = TX * TY;
-    static constexpr int SW = TX + 2;
-    static constexpr int SH = TY + 2;
-    static constexpr int SP = SW * SH;
-    static constexpr int NHALO = SP - NT;
-    static_assert(NHALO <= NT, "one halo point per thread at most");
+    static constexpr int NT = MTX * TY_;
+    static constexpr int SW = MTX + 2;
+    static constexpr int SP = SW * (TY_ + 2);
+    static_assert(SP - NT <= NT, "one halo point per thread at most");
+};
+template <>
+struct MTile<0> {
+    static constexpr int NT = 256, SW = 0, SP = FIT_POINTS_MIXED;
 };
 
 // LDS: raw planes k, k+1 (2 x NF fields) and a three-plane ring of u, v, w,
 // T'.
-template <int TY, bool MAG, int MODE, int TXW = MTX>
+template <int TY, bool MAG>
 constexpr int mixed_lds_bytes() {
-    return (2 * (MAG ? 8 : 5) + 12) * MTile<TXW, TY>::SP * (int)sizeof(float);
+    return (2 * (MAG ? 8 : 5) + 12) * MTile<TY>::SP * (int)sizeof(float);
 }
 
 // P' of temperature perturbation tp at density perturbation rh.  The
@@ -270,14 +270,16 @@ __device__ __forceinline__ void bcon_column_m(const Params &p, const Metrics &m,
 #define PLB(F, K) uload(&bg.planes[K].F, 0)
 #define PLP(F, K) uload(&bg.planes[K].F, 0)
 
-template <int TY, bool MAG, int MODE, int TXW = MTX>
+template <int TY, bool MAG, int MODE>
 __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, const Background &bg, ArgPtr args,
                                              const float *__restrict__ hin, float *__restrict__ hout,
                                              float *__restrict__ dr, unsigned *__restrict__ rr,
                                              DevScalars *__restrict__ sc, CflSlots *__restrict__ cs, int i0, int j0,
-                                             int kbeg, int kend, int seq, int total, float *ldsf) {
-    using T = MTile<TXW, TY>;
-    constexpr int SW = T::SW, SP = T::SP;
+                                             int kbeg, int kend, int seq, int total, float *ldsf, int tw, int th) {
+    using T = MTile<TY>;
+    constexpr bool FIT = TY == 0;
+    constexpr int SP = T::SP;
+    const int W = FIT ? tw : MTX, H = FIT ? th : TY, SW = FIT ? tw + 2 : T::SW;
     constexpr int NF = MAG ? 8 : 5;
     float *const s_cur = ldsf;
     float *const s_ring = ldsf + 2 * NF * SP;
@@ -286,20 +288,22 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
     const int npx = p.npx, npy = p.npy, npz = p.npz;
     const long long fs = p.fsize, pl = p.plane;
 
-    const int olx = t % TXW + 1, oly = t / TXW + 1;
+    // (threads past a fitted tile's last point double that point)
+    const int own = FIT && t >= W * H ? W * H - 1 : t;
+    const int oly = own / W + 1, olx = own - (oly - 1) * W + 1;
     const int opt = oly * SW + olx;
     const int gi = i0 + olx - 1, gj = j0 + oly - 1;
-    const bool valid = (gi < npx) && (gj < npy);
+    const bool valid = (gi < npx) && (gj < npy) && (!FIT || t < W * H);
     const int gci = wrapc(gi, npx), gcj = wrapc(gj, npy);  // this lane's column
     const long long ooff = (long long)gcj * npx + gci;
     int hpt = -1;
     long long hoff = 0;
-    if (t < T::NHALO) {
+    if (t < 2 * (SW + H)) {
         int hlx, hly;
         if (t < SW) { hlx = t; hly = 0; }
-        else if (t < 2 * SW) { hlx = t - SW; hly = T::SH - 1; }
-        else if (t < 2 * SW + TY) { hlx = 0; hly = t - 2 * SW + 1; }
-        else { hlx = SW - 1; hly = t - 2 * SW - TY + 1; }
+        else if (t < 2 * SW) { hlx = t - SW; hly = H + 1; }
+        else if (t < 2 * SW + H) { hlx = 0; hly = t - 2 * SW + 1; }
+        else { hlx = SW - 1; hly = t - 2 * SW - H + 1; }
         hpt = hly * SW + hlx;
         hoff = (long long)wrapc(j0 + hly - 1, npy) * npx + wrapc(i0 + hlx - 1, npx);
     }
@@ -663,25 +667,26 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
 }
 
 template <int TY, bool MAG, int MODE>
-__global__ __launch_bounds__(MTX *TY, 3) void k_stage_m(const BoxArgs b,
+__global__ __launch_bounds__(MTile<TY>::NT, 3) void k_stage_m(const BoxArgs b,
                                                      const float *__restrict__ hin, float *__restrict__ hout,
                                                      float *__restrict__ dr, unsigned *__restrict__ rr,
                                                      DevScalars *__restrict__ sc, CflSlots *__restrict__ cs,
                                                      int nchunks) {
     extern __shared__ float ldsf[];
     const Params &p = b.p;
-    const int ntx = (p.npx + MTX - 1) / MTX, nty = (p.npy + TY - 1) / TY;
+    const int W = TY ? MTX : p.tile_w, H = TY ? TY : p.tile_h;
+    const int ntx = (p.npx + W - 1) / W, nty = (p.npy + H - 1) / H;
     const TileChunk tc = tile_of(blockIdx.x, ntx * nty, nchunks);
     const int tz = tc.chunk, tyb = tc.tile / ntx, txb = tc.tile - tyb * ntx;
     const int kbeg = chunk_begin(p.npz, nchunks, tz), kend = chunk_begin(p.npz, nchunks, tz + 1) - 1;
-    stage_tile_m<TY, MAG, MODE>(p, b.m, b.bg, kernel_args(), hin, hout, dr, rr, sc, cs, txb * MTX, tyb * TY, kbeg, kend,
-                                blockIdx.x, gridDim.x, ldsf);
+    stage_tile_m<TY, MAG, MODE>(p, b.m, b.bg, kernel_args(), hin, hout, dr, rr, sc, cs, txb * W, tyb * H, kbeg, kend,
+                                blockIdx.x, gridDim.x, ldsf, W, H);
 }
 
 // Ensemble: persistent grid over the work items of all boxes (static stride);
-// items are TXW x TY tiles.
-template <int TY, bool MAG, int MODE, int TXW>
-__global__ __launch_bounds__(TXW *TY, 3) void k_stage_m_batch(const BoxDev *__restrict__ boxes,
+// each item carries its tile's shape.
+template <int TY, bool MAG, int MODE>
+__global__ __launch_bounds__(MTile<TY>::NT, 3) void k_stage_m_batch(const BoxDev *__restrict__ boxes,
                                                            const StageItem *__restrict__ items, int nitems, int a) {
     extern __shared__ float ldsf[];
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
@@ -689,8 +694,8 @@ __global__ __launch_bounds__(TXW *TY, 3) void k_stage_m_batch(const BoxDev *__re
         const StageItem it = items[w];
         const BoxDev &B = box_at(boxes, it.box);
         __syncthreads();  // the previous item's last LDS reads are done
-        stage_tile_m<TY, MAG, MODE, TXW>(B.a.p, B.a.m, B.a.bg, (ArgPtr)&B.a, B.h[a], B.h[1 - a], B.dr, B.rr, B.sc, B.cs, it.i0, it.j0,
-                                         it.kbeg, it.kend, it.seq, it.total, ldsf);
+        stage_tile_m<TY, MAG, MODE>(B.a.p, B.a.m, B.a.bg, (ArgPtr)&B.a, B.h[a], B.h[1 - a], B.dr, B.rr, B.sc, B.cs, it.i0, it.j0,
+                                    it.kbeg, it.kend, it.seq, it.total, ldsf, it.w, it.h);
     }
 }
 
@@ -850,15 +855,14 @@ __global__ void k_closure_forcing(const Params p, const float *__restrict__ y, c
 template <int TY, bool MAG, int MODE>
 static hipError_t launch_m(const Params &p, const Metrics &m, const Background &bg, const float *hin, float *hout,
                            float *dr, unsigned *rr, DevScalars *sc, CflSlots *cs, hipStream_t s) {
-    constexpr int lds = mixed_lds_bytes<TY, MAG, MODE>();
+    constexpr int lds = mixed_lds_bytes<TY, MAG>();
     static std::atomic<unsigned long long> attr{0};
     {
         hipError_t e = lds_limit_once(attr, reinterpret_cast<const void *>(&k_stage_m<TY, MAG, MODE>), lds);
         if (e != hipSuccess) return e;
     }
     const int nch = p.nchunks;
-    const int ntiles = ((p.npx + MTX - 1) / MTX) * ((p.npy + TY - 1) / TY);
-    hipLaunchKernelGGL((k_stage_m<TY, MAG, MODE>), dim3(ntiles * nch), dim3(MTX * TY), lds, s, BoxArgs{p, m, bg}, hin, hout,
+    hipLaunchKernelGGL((k_stage_m<TY, MAG, MODE>), dim3(tiles_of(p) * nch), dim3(MTile<TY>::NT), lds, s, BoxArgs{p, m, bg}, hin, hout,
                        dr, rr, sc, cs, nch);
     return hipGetLastError();
 }
@@ -878,6 +882,7 @@ static hipError_t launch_m_ty(int mode, const Params &p, const Metrics &m, const
 
 hipError_t launch_stage_mixed(int mode, const Params &p, const Metrics &m, const Background &bg, const float *hin,
                               float *hout, float *dr, unsigned *rr, DevScalars *sc, CflSlots *cs, hipStream_t s) {
+    if (p.tile_w) return launch_m_ty<0>(mode, p, m, bg, hin, hout, dr, rr, sc, cs, s);
     if (p.tile_y == 8) return launch_m_ty<8>(mode, p, m, bg, hin, hout, dr, rr, sc, cs, s);
     return launch_m_ty<4>(mode, p, m, bg, hin, hout, dr, rr, sc, cs, s);
 }
@@ -918,41 +923,38 @@ hipError_t launch_rebase_mixed(const Params &p, const Background &ob, const Back
     return hipGetLastError();
 }
 
-template <int TY, bool MAG, int MODE, int TXW>
+template <int TY, bool MAG, int MODE>
 static hipError_t launch_mb(const BoxDev *boxes, const StageItem *items, int nitems, int grid, int a,
                             hipStream_t s) {
-    constexpr int lds = mixed_lds_bytes<TY, MAG, MODE, TXW>();
+    constexpr int lds = mixed_lds_bytes<TY, MAG>();
     static std::atomic<unsigned long long> attr{0};
     {
-        hipError_t e =
-            lds_limit_once(attr, reinterpret_cast<const void *>(&k_stage_m_batch<TY, MAG, MODE, TXW>), lds);
+        hipError_t e = lds_limit_once(attr, reinterpret_cast<const void *>(&k_stage_m_batch<TY, MAG, MODE>), lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((k_stage_m_batch<TY, MAG, MODE, TXW>), dim3(grid), dim3(TXW * TY), lds, s, boxes, items,
-                       nitems, a);
+    hipLaunchKernelGGL((k_stage_m_batch<TY, MAG, MODE>), dim3(grid), dim3(MTile<TY>::NT), lds, s, boxes, items, nitems,
+                       a);
     return hipGetLastError();
 }
 
-template <int TY, int TXW>
+template <int TY>
 static hipError_t launch_mb_ty(int mode, int lmag, const BoxDev *boxes, const StageItem *items, int nitems,
                                int grid, int a, hipStream_t s) {
     if (lmag) {
-        if (mode == 1) return launch_mb<TY, true, 1, TXW>(boxes, items, nitems, grid, a, s);
-        if (mode == 2) return launch_mb<TY, true, 2, TXW>(boxes, items, nitems, grid, a, s);
-        return launch_mb<TY, true, 3, TXW>(boxes, items, nitems, grid, a, s);
+        if (mode == 1) return launch_mb<TY, true, 1>(boxes, items, nitems, grid, a, s);
+        if (mode == 2) return launch_mb<TY, true, 2>(boxes, items, nitems, grid, a, s);
+        return launch_mb<TY, true, 3>(boxes, items, nitems, grid, a, s);
     }
-    if (mode == 1) return launch_mb<TY, false, 1, TXW>(boxes, items, nitems, grid, a, s);
-    if (mode == 2) return launch_mb<TY, false, 2, TXW>(boxes, items, nitems, grid, a, s);
-    return launch_mb<TY, false, 3, TXW>(boxes, items, nitems, grid, a, s);
+    if (mode == 1) return launch_mb<TY, false, 1>(boxes, items, nitems, grid, a, s);
+    if (mode == 2) return launch_mb<TY, false, 2>(boxes, items, nitems, grid, a, s);
+    return launch_mb<TY, false, 3>(boxes, items, nitems, grid, a, s);
 }
 
-// Tile shapes built for the batched launches: 64x4, 64x8 and 32x8 (the
-// caller validates the shape).
+// 64x8 tiles, or tiles of at most 256 points of the items' own shapes.
 hipError_t launch_stage_batch_mixed(int mode, int tile_x, int tile_y, int lmag, const BoxDev *boxes,
                                     const StageItem *items, int nitems, int grid, int a, hipStream_t s) {
-    if (tile_x == 32) return launch_mb_ty<8, 32>(mode, lmag, boxes, items, nitems, grid, a, s);
-    if (tile_y == 8) return launch_mb_ty<8, MTX>(mode, lmag, boxes, items, nitems, grid, a, s);
-    return launch_mb_ty<4, MTX>(mode, lmag, boxes, items, nitems, grid, a, s);
+    if (tile_x == 64 && tile_y == 8) return launch_mb_ty<8>(mode, lmag, boxes, items, nitems, grid, a, s);
+    return launch_mb_ty<0>(mode, lmag, boxes, items, nitems, grid, a, s);
 }
 
 hipError_t launch_closure_inputs(const Params &p, const Background &bg, const float *h, const unsigned *rr,
