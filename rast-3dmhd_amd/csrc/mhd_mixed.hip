@@ -60,11 +60,17 @@ struct MTile<0> {
     static constexpr int NT = 256, SW = 0, SP = FIT_POINTS_MIXED;
 };
 
-// LDS: raw planes k, k+1 (2 x NF fields) and a three-plane ring of u, v, w,
-// T'.
-template <int TY, bool MAG>
+// LDS: raw planes k, k+1 (2 x NF fields) and a three-plane ring of u, v, w, T'.
+// Lean: T' takes the place of rho', of which only a point's own value is read (it
+// stays in registers, as does T' of plane k-1), 25 instead of 28 values a point.
+// Stage 1, whose registers allow it, so has four workgroups of 64x4 on a CU
+// (512x512x256: 1654 -> 1581 us); the others keep three either way, and stage 3
+// is 1% slower lean (256x256x128).
+template <int MODE>
+constexpr bool lean_lds = MODE == 1;
+template <int TY, bool MAG, int MODE>
 constexpr int mixed_lds_bytes() {
-    return (2 * (MAG ? 8 : 5) + 12) * MTile<TY>::SP * (int)sizeof(float);
+    return (2 * (MAG ? 8 : 5) + (lean_lds<MODE> ? 9 : 12)) * MTile<TY>::SP * (int)sizeof(float);
 }
 
 // P' of temperature perturbation tp at density perturbation rh.  The
@@ -281,6 +287,7 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
     constexpr int SP = T::SP;
     const int W = FIT ? tw : MTX, H = FIT ? th : TY, SW = FIT ? tw + 2 : T::SW;
     constexpr int NF = MAG ? 8 : 5;
+    constexpr bool LEAN = lean_lds<MODE>;
     float *const s_cur = ldsf;
     float *const s_ring = ldsf + 2 * NF * SP;
 
@@ -294,33 +301,35 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
     const int opt = oly * SW + olx;
     const int gi = i0 + olx - 1, gj = j0 + oly - 1;
     const bool valid = (gi < npx) && (gj < npy) && (!FIT || t < W * H);
-    const int gci = wrapc(gi, npx), gcj = wrapc(gj, npy);  // this lane's column
+    const int gci = wrapc(min(gi, npx), npx), gcj = wrapc(gj, npy);  // this lane's column
     const long long ooff = (long long)gcj * npx + gci;
     int hpt = -1;
     long long hoff = 0;
-    if (t < 2 * (SW + H)) {
+    {
+        const int ht = min(t, 2 * (SW + H) - 1);
         int hlx, hly;
-        if (t < SW) { hlx = t; hly = 0; }
-        else if (t < 2 * SW) { hlx = t - SW; hly = H + 1; }
-        else if (t < 2 * SW + H) { hlx = 0; hly = t - 2 * SW + 1; }
-        else { hlx = SW - 1; hly = t - 2 * SW - H + 1; }
+        if (ht < SW) { hlx = ht; hly = 0; }
+        else if (ht < 2 * SW) { hlx = ht - SW; hly = H + 1; }
+        else if (ht < 2 * SW + H) { hlx = 0; hly = ht - 2 * SW + 1; }
+        else { hlx = SW - 1; hly = ht - 2 * SW - H + 1; }
         hpt = hly * SW + hlx;
         hoff = (long long)wrapc(j0 + hly - 1, npy) * npx + wrapc(i0 + hlx - 1, npx);
     }
-    const bool has_h = hpt >= 0;
+    const bool has_h = t < 2 * (SW + H);
 
     auto cur = [&](int k, int f, int pt) -> float & { return s_cur[((k & 1) * NF + f) * SP + pt]; };
-    auto ring = [&](int k, int c, int pt) -> float & { return s_ring[((k % 3) * 4 + c) * SP + pt]; };
+    auto ring = [&](int k, int c, int pt) -> float & { return s_ring[((k % 3) * (LEAN ? 3 : 4) + c) * SP + pt]; };
+    auto tprime = [&](int k, const RawF &r) { return trep(PLB(ro32, k), PLB(tt32, k), r.v[3], r.v[4]); };
     auto put_cur = [&](int k, int pt, const RawF &r) {
 #pragma unroll
-        for (int f = 0; f < NF; ++f) cur(k, f, pt) = r.v[f];
+        for (int f = 0; f < NF; ++f) cur(k, f, pt) = LEAN && f == 3 ? tprime(k, r) : r.v[f];
     };
     auto put_ring = [&](int k, int pt, const RawF &r) {
         const float ri = rcp32(PLB(ro32, k) + r.v[3]);
         ring(k, 0, pt) = r.v[0] * ri;
         ring(k, 1, pt) = r.v[1] * ri;
         ring(k, 2, pt) = r.v[2] * ri;
-        ring(k, 3, pt) = trep(PLB(ro32, k), PLB(tt32, k), r.v[3], r.v[4]);  // temperature perturbation
+        if (!LEAN) ring(k, 3, pt) = tprime(k, r);  // temperature perturbation
     };
 
     // the per-column values are on their way before the warm-up's loads
@@ -346,16 +355,22 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
     }
     // warm-up: planes kbeg-1 .. kbeg+1, every load issued before the first is
     // used (lanes without a halo point re-read their own)
-    RawF rm_, rp_o, rp_h;
+    RawF rm_, rp_o, rp_h;  // planes k-1 (lean: T' in the place of rho'), k+2
+    float rho_k = 0.0f, rho_n = 0.0f;  // lean: own rho' of planes k, k+1
     {
         RawF ro_[2], rh_[3];
-        const long long ho = has_h ? hoff : ooff;
+        const long long ho = hoff;
         load_rawf<MAG>(hin, fs, (long long)(kbeg - 1) * pl + ooff, rm_);
 #pragma unroll
         for (int n = 0; n < 2; ++n) load_rawf<MAG>(hin, fs, (long long)(kbeg + n) * pl + ooff, ro_[n]);
 #pragma unroll
         for (int n = 0; n < 3; ++n) load_rawf<MAG>(hin, fs, (long long)(kbeg - 1 + n) * pl + ho, rh_[n]);
         put_ring(kbeg - 1, opt, rm_);
+        if (LEAN) {
+            rm_.v[3] = tprime(kbeg - 1, rm_);
+            rho_k = ro_[0].v[3];
+            rho_n = ro_[1].v[3];
+        }
 #pragma unroll
         for (int n = 0; n < 2; ++n) {
             put_cur(kbeg + n, opt, ro_[n]);
@@ -400,7 +415,7 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
         {
             const long long kp = (long long)(pre ? k + 2 : k) * pl;
             load_rawf<MAG>(hin, fs, kp + ooff, rp_o);
-            load_rawf<MAG>(hin, fs, kp + (has_h ? hoff : ooff), rp_h);
+            load_rawf<MAG>(hin, fs, kp + hoff, rp_h);
         }
         __syncthreads();
         if (valid) {
@@ -414,14 +429,15 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
 #define CUR(f, d) cur(k, f, opt + (d))
 #define NXT(f) cur(k + 1, f, opt)
 #define RNG(kp, c, d) ring(kp, c, opt + (d))
+#define TP(d) (LEAN ? CUR(3, d) : RNG(k, 3, d))
             float h0[8];
             rhs_t q0[8];
 #pragma unroll
             for (int f = 0; f < NF; ++f) {
-                h0[f] = CUR(f, 0);
+                h0[f] = LEAN && f == 3 ? rho_k : CUR(f, 0);
                 q0[f] = h0[f];
             }
-            const rhs_t rh0 = q0[3], th0 = RNG(k, 3, 0);
+            const rhs_t rh0 = q0[3], th0 = TP(0);
             const rhs_t tf0 = t0 + th0;                    // full temperature
             const rhs_t rinv = rcp32(r0 + rh0);                // 1/rho
             const rhs_t u0 = RNG(k, 0, 0), v0 = RNG(k, 1, 0), w0 = RNG(k, 2, 0);
@@ -432,7 +448,7 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
             const rhs_t wxp = RNG(k, 2, 1), wxm = RNG(k, 2, -1), wyp = RNG(k, 2, SW), wym = RNG(k, 2, -SW);
             const rhs_t ru_m = rm_.v[0], rv_m = rm_.v[1], rw_m = rm_.v[2];
             const rhs_t ru_p = NXT(0), rv_p = NXT(1), rw_p = NXT(2);
-            const rhs_t th_m = RNG(k - 1, 3, 0), th_p = RNG(k + 1, 3, 0);
+            const rhs_t th_m = LEAN ? rm_.v[3] : RNG(k - 1, 3, 0), th_p = LEAN ? NXT(3) : RNG(k + 1, 3, 0);
             // stored pressure perturbation at the six neighbours
             const rhs_t pm = rm_.v[4], pp = NXT(4);
             const rhs_t pxm = CUR(4, -1), pxp = CUR(4, 1), pym = CUR(4, -SW), pyp = CUR(4, SW);
@@ -477,7 +493,7 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
                 fw -= (CUR(2, 1) * uxp - CUR(2, -1) * uxm) * hxdx + (CUR(2, SW) * vyp - CUR(2, -SW) * vym) * hydy
                       + (rw_p * wp - rw_m * wm) * hzdz;
                 // temperature advection, the background gradient included
-                const rhs_t txp = RNG(k, 3, 1), txm = RNG(k, 3, -1), typ = RNG(k, 3, SW), tym = RNG(k, 3, -SW);
+                const rhs_t txp = TP(1), txm = TP(-1), typ = TP(SW), tym = TP(-SW);
                 const rhs_t dtz = (th_p - th_m) * hzdz;
                 ft = -(u0 * (txp - txm) * hxdx + v0 * (typ - tym) * hydy + w0 * (dtz + PLB(dt0dz32, k)));
                 // conduction of T': (1/rho) c [kappa lap T' + kappa' dT'/dz]; plus the
@@ -567,6 +583,7 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
                 }
 #undef CUR
 #undef NXT
+#undef TP
 #undef RNG
             }
             // FP64 accumulation: F = F_bg(z) + F', X = value + D + gamma dt F
@@ -637,7 +654,11 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
                 cfl_acc = c;
             }
 #pragma unroll
-            for (int f = 0; f < NF; ++f) rm_.v[f] = h0[f];
+            for (int f = 0; f < NF; ++f) rm_.v[f] = LEAN && f == 3 ? th0 : h0[f];
+        }
+        if (LEAN) {
+            rho_k = rho_n;
+            rho_n = rp_o.v[3];
         }
         __syncthreads();
         if (pre) {
@@ -855,7 +876,7 @@ __global__ void k_closure_forcing(const Params p, const float *__restrict__ y, c
 template <int TY, bool MAG, int MODE>
 static hipError_t launch_m(const Params &p, const Metrics &m, const Background &bg, const float *hin, float *hout,
                            float *dr, unsigned *rr, DevScalars *sc, CflSlots *cs, hipStream_t s) {
-    constexpr int lds = mixed_lds_bytes<TY, MAG>();
+    constexpr int lds = mixed_lds_bytes<TY, MAG, MODE>();
     static std::atomic<unsigned long long> attr{0};
     {
         hipError_t e = lds_limit_once(attr, reinterpret_cast<const void *>(&k_stage_m<TY, MAG, MODE>), lds);
@@ -926,7 +947,7 @@ hipError_t launch_rebase_mixed(const Params &p, const Background &ob, const Back
 template <int TY, bool MAG, int MODE>
 static hipError_t launch_mb(const BoxDev *boxes, const StageItem *items, int nitems, int grid, int a,
                             hipStream_t s) {
-    constexpr int lds = mixed_lds_bytes<TY, MAG>();
+    constexpr int lds = mixed_lds_bytes<TY, MAG, MODE>();
     static std::atomic<unsigned long long> attr{0};
     {
         hipError_t e = lds_limit_once(attr, reinterpret_cast<const void *>(&k_stage_m_batch<TY, MAG, MODE>), lds);
