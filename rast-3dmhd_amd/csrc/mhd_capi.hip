@@ -59,7 +59,7 @@ struct mhd_ctx {
     DevScalars *report = nullptr;       // pinned: the scalars of the last step of a call (Params::report)
     // closure-corrected step (mixed form)
     mhd_net_t *net = nullptr;
-    float *force = nullptr;    // [7][fsize]
+    float *force = nullptr;    // [npz * plane][8]
     int *force_on = nullptr;
     __bf16 *cx = nullptr;      // network input [npz][npy][npx][8]
     float *nrm = nullptr;      // input plane means [8][npz], 1/std[8]; then nrm_out:
@@ -512,10 +512,9 @@ static hipError_t launches(mhd_t *h, hipEvent_t *ev, bool report = false) {
     }
     if (e == hipSuccess && h->closure) {
         // subgrid forcing from the network on the state at the start of the step
-        const float *y = nullptr;
-        e = launch_closure_inputs(p, h->bg, h->hq[h->cur], h->rr, h->nrm, h->cx, h->stream);
-        if (e == hipSuccess) e = net_forward_device(h->net, h->stream, p.npx, p.npy, p.npz, h->cx, &y);
-        if (e == hipSuccess) e = launch_closure_forcing(p, y, h->nrm_out, h->force, h->force_on, h->stream);
+        e = launch_closure_inputs(p, h->bg, h->hq[h->cur], h->rr, h->nrm, h->cx, h->force_on, h->stream);
+        if (e == hipSuccess)
+            e = net_force(h->net, h->stream, p.npx, p.npy, p.npz, h->cx, h->nrm_out, h->force, h->force_on);
     }
     rec(1);
     int a = h->cur, b = 1 - h->cur;
@@ -731,7 +730,7 @@ extern "C" int mhd_set_closure(mhd_t *h, mhd_net_t *net, const double *in_profil
     if (ndev != h->dev) return fail(h, MHD_ERR_ARG, "mhd_set_closure: network on device %d, box on %d", ndev, h->dev);
     const int nz = p.npz;
     const size_t nin = 8 * (size_t)nz + 8, nout = 7 * (size_t)nz + 7;
-    if (!h->force) HIPCHK(h, hipMalloc(&h->force, (size_t)7 * p.fsize * sizeof(float)));
+    if (!h->force) HIPCHK(h, hipMalloc(&h->force, (size_t)8 * nvox * sizeof(float)));
     if (!h->force_on) HIPCHK(h, hipMalloc(&h->force_on, sizeof(int)));
     if (!h->cx) HIPCHK(h, hipMalloc(&h->cx, (size_t)nvox * 8 * sizeof(__bf16)));
     if (!h->nrm) HIPCHK(h, hipMalloc(&h->nrm, (nin + nout) * sizeof(float)));
@@ -742,8 +741,6 @@ extern "C" int mhd_set_closure(mhd_t *h, mhd_net_t *net, const double *in_profil
     for (int c = 0; c < 7; ++c) nrm[nin + 7 * nz + c] = (float)out_std[c];
     HIPCHK(h, hipMemcpy(h->nrm, nrm.data(), nrm.size() * sizeof(float), hipMemcpyHostToDevice));
     h->nrm_out = h->nrm + nin;
-    // forcing is zero outside the interior planes
-    HIPCHK(h, hipMemset(h->force, 0, (size_t)7 * p.fsize * sizeof(float)));
     h->net = net;
     h->closure = true;
     if (h->have_bg) {

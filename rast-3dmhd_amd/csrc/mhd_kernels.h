@@ -134,8 +134,8 @@ struct Background {
     const double *iddz2, *irk;  // 1/ddz^2 and 1/rkapa per plane (grid only; the CFL of stage 3)
     const PlaneM *planes;       // the same per plane with the metrics, for the stage kernel
     const float *ro32, *tt32, *dt0dz32, *rinv0_32, *s0_32;
-    // optional subgrid forcing of the closure-corrected step: FP32 fields
-    // [RU,RV,RW,TT,BX,BY,BZ][plane][j][i] added to the right-hand side of
+    // optional subgrid forcing of the closure-corrected step: FP32
+    // [plane-1][j][i][RU,RV,RW,TT,BX,BY,BZ,0] added to the right-hand side of
     // every stage while *force_on != 0 (null: none)
     const float *force;
     const int *force_on;
@@ -272,13 +272,9 @@ hipError_t launch_box_filter(const Params &p, const double *q, int nf, int facto
 
 // Closure-corrected mixed step (mhd_mixed.hip): network inputs from the
 // state (rho, u, v, w, s = ln T/(gamma-1) - ln rho, BX, BY, BZ; nrm =
-// per-plane means [8][npz], 1/std[8]) as BF16 [plane-1][j][i][8], and the
-// forcing from the network output (nrm_out = per-plane mean subgrid terms
-// [7][npz], std[7]); force_on is cleared if any output is not finite.
+// per-plane means [8][npz], 1/std[8]) as BF16 [plane-1][j][i][8]; sets *force_on.
 hipError_t launch_closure_inputs(const Params &p, const Background &bg, const float *h, const unsigned *rr,
-                                 const float *nrm, __bf16 *x, hipStream_t s);
-hipError_t launch_closure_forcing(const Params &p, const float *y, const float *nrm_out, float *force, int *force_on,
-                                  hipStream_t s);
+                                 const float *nrm, __bf16 *x, int *force_on, hipStream_t s);
 
 // Horizontal means and mean convective flux per interior plane (mhd_diag.hip):
 // out[3][npz] = TTM, ROM, FCONM.
@@ -313,6 +309,7 @@ hipError_t launch_stage_batch_mixed(int mode, int tile_x, int tile_y, int lmag, 
 // Network entry points used by the closure-corrected step (mhd_net.hip).
 int net_shape(const mhd_net *n, int *cin, int *cout);
 int net_prepare(mhd_net *n, long long nvox, int *dev);
-hipError_t net_forward_device(mhd_net *n, hipStream_t s, int nx, int ny, int nz, const __bf16 *x, const float **y);
+hipError_t net_force(mhd_net *n, hipStream_t s, int nx, int ny, int nz, const __bf16 *x, const float *nrm,
+                     float *force, int *force_on);
 
 }  // namespace rmhd

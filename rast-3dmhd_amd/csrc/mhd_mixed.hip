@@ -597,15 +597,19 @@ __device__ __forceinline__ void stage_tile_m(const Params &p, const Metrics &m, 
             Fd[2] += PLB(fwbg, k);
             Fd[4] += PLB(ftbg, k);
             if (frc) {
-                const float *g = bg.force + o;
-                Fd[0] += (double)g[0];
-                Fd[1] += (double)g[fs];
-                Fd[2] += (double)g[2 * fs];
-                Fd[4] += (double)g[3 * fs];
+                // (two 16-byte loads; the stages took 44, 50 and 54 us with seven of
+                // 4 bytes, 40, 42 and 48 so, 128x128x64)
+                const float4 *g = reinterpret_cast<const float4 *>(bg.force) + 2 * (o - pl);
+                const float4 g0 = g[0];
+                Fd[0] += (double)g0.x;
+                Fd[1] += (double)g0.y;
+                Fd[2] += (double)g0.z;
+                Fd[4] += (double)g0.w;
                 if (MAG) {
-                    Fd[5] += (double)g[4 * fs];
-                    Fd[6] += (double)g[5 * fs];
-                    Fd[7] += (double)g[6 * fs];
+                    const float4 g1 = g[1];
+                    Fd[5] += (double)g1.x;
+                    Fd[6] += (double)g1.y;
+                    Fd[7] += (double)g1.z;
                 }
             }
             const double r0d = PLB(ro, k), t0d = PLB(tt, k);
@@ -823,52 +827,46 @@ __global__ void k_rebase_m(const Params p, const Background ob, const Background
     }
 }
 
-// Network inputs of the closure from the state (h, R) about the background.
-__global__ void k_closure_inputs(const Params p, const Background bg, const float *__restrict__ h,
-                                 const unsigned *__restrict__ rr, const float *__restrict__ nrm,
-                                 __bf16 *__restrict__ x) {
-    const long long fs = p.fsize, n = (long long)p.npz * p.plane;
-    for (long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x; v < n;
-         v += (long long)gridDim.x * blockDim.x) {
-        const int k = (int)(v / p.plane) + 1;
-        const long long o = p.plane + v;
-        auto val = [&](int f) { return (double)h[f * fs + o] + (double)r_get(rr, fs, f, o); };
-        const double ro = bg.ro[k] + val(3);
-        const double tt = bg.tt[k] + (double)trep(bg.ro32[k], bg.tt32[k], h[3 * fs + o], h[4 * fs + o]) +
-                          (double)r_get(rr, fs, 4, o);
-        const double ri = 1.0 / ro;
-        double c[8];
-        c[0] = ro;
-        c[1] = val(0) * ri;
-        c[2] = val(1) * ri;
-        c[3] = val(2) * ri;
-        c[4] = log(tt) / (p.gamma - 1.0) - log(ro);
-        for (int f = 5; f < 8; ++f) c[f] = p.lmag ? val(f) : 0.0;
-        // nrm: per-plane means [8][npz], then 1/std [8]
-        for (int f = 0; f < 8; ++f)
-            x[v * 8 + f] = (__bf16)(float)((c[f] - (double)nrm[f * p.npz + k - 1]) * (double)nrm[8 * p.npz + f]);
-    }
-}
-
-__global__ void k_set_flag(int *flag) { *flag = 1; }
-
-// Forcing fields from the network output y[v][8] (7 channels used).
-__global__ void k_closure_forcing(const Params p, const float *__restrict__ y, const float *__restrict__ nrm,
-                                  float *__restrict__ force, int *__restrict__ force_on) {
-    const long long fs = p.fsize, n = (long long)p.npz * p.plane;
-    for (long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x; v < n;
-         v += (long long)gridDim.x * blockDim.x) {
-        const long long o = p.plane + v;
-        const int k = (int)(v / p.plane);  // plane index 0..npz-1
-        bool ok = true;
-        // nrm: per-plane mean subgrid terms [7][npz], then std [7]
-        for (int c = 0; c < 7; ++c) {
-            const float g = y[v * 8 + c] * nrm[7 * p.npz + c] + nrm[c * p.npz + k];
-            ok = ok && (g - g == 0.0f);
-            force[c * fs + o] = g;
+// Network inputs of the closure from the state (h, R) about the background: a
+// plane per blockIdx.y, one 16-byte store a point.  Bound by the FP64 logarithms
+// and divisions (128x128x64: 18 us; 22 with 64-bit divisions for the plane and
+// eight 2-byte stores).
+template <bool MAG>
+__global__ __launch_bounds__(256) void k_closure_inputs(const Params p, const Background bg, const float *__restrict__ h,
+                                                        const unsigned *__restrict__ rr,
+                                                        const float *__restrict__ nrm, __bf16 *__restrict__ x,
+                                                        int *__restrict__ force_on) {
+    const long long fs = p.fsize;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *force_on = 1;  // (the network's last layer clears it)
+    for (int k = blockIdx.y + 1; k <= p.npz; k += gridDim.y)
+        for (long long c0 = (long long)blockIdx.x * 256 + threadIdx.x; c0 < p.plane; c0 += (long long)gridDim.x * 256) {
+            const long long o = k * p.plane + c0;
+            float hv[8];
+            unsigned w[4];
+#pragma unroll
+            for (int f = 0; f < (MAG ? 8 : 5); ++f) hv[f] = h[f * fs + o];
+#pragma unroll
+            for (int n = 0; n < (MAG ? 4 : 3); ++n) w[n] = rr[n * fs + o];
+            auto val = [&](int f) { return (double)hv[f] + (double)r_half(w[f >> 1], f); };
+            const double ro = bg.ro[k] + val(3);
+            const double tt = bg.tt[k] + (double)trep(bg.ro32[k], bg.tt32[k], hv[3], hv[4]) + (double)r_half(w[2], 4);
+            const double ri = 1.0 / ro;
+            double c[8];
+            c[0] = ro;
+            c[1] = val(0) * ri;
+            c[2] = val(1) * ri;
+            c[3] = val(2) * ri;
+            c[4] = log(tt) / (p.gamma - 1.0) - log(ro);
+#pragma unroll
+            for (int f = 5; f < 8; ++f) c[f] = MAG ? val(f) : 0.0;
+            // nrm: per-plane means [8][npz], then 1/std [8]
+            typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+            bf16x8 v;
+#pragma unroll
+            for (int f = 0; f < 8; ++f)
+                v[f] = (__bf16)(float)((c[f] - (double)nrm[f * p.npz + k - 1]) * (double)nrm[8 * p.npz + f]);
+            *reinterpret_cast<bf16x8 *>(x + (o - p.plane) * 8) = v;
         }
-        if (!ok) *force_on = 0;
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -979,21 +977,11 @@ hipError_t launch_stage_batch_mixed(int mode, int tile_x, int tile_y, int lmag, 
 }
 
 hipError_t launch_closure_inputs(const Params &p, const Background &bg, const float *h, const unsigned *rr,
-                                 const float *nrm, __bf16 *x, hipStream_t s) {
-    long long nb = ((long long)p.npz * p.plane + 255) / 256;
-    if (nb > 8192) nb = 8192;
-    hipLaunchKernelGGL(k_closure_inputs, dim3((unsigned)nb), dim3(256), 0, s, p, bg, h, rr, nrm, x);
-    return hipGetLastError();
-}
-
-hipError_t launch_closure_forcing(const Params &p, const float *y, const float *nrm_out, float *force, int *force_on,
-                                  hipStream_t s) {
-    hipLaunchKernelGGL(k_set_flag, dim3(1), dim3(1), 0, s, force_on);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    long long nb = ((long long)p.npz * p.plane + 255) / 256;
-    if (nb > 8192) nb = 8192;
-    hipLaunchKernelGGL(k_closure_forcing, dim3((unsigned)nb), dim3(256), 0, s, p, y, nrm_out, force, force_on);
+                                 const float *nrm, __bf16 *x, int *force_on, hipStream_t s) {
+    const long long nb = (p.plane + 255) / 256;
+    const dim3 grid((unsigned)(nb > 4096 ? 4096 : nb), (unsigned)(p.npz > 4096 ? 4096 : p.npz));
+    if (p.lmag) hipLaunchKernelGGL(k_closure_inputs<true>, grid, dim3(256), 0, s, p, bg, h, rr, nrm, x, force_on);
+    else hipLaunchKernelGGL(k_closure_inputs<false>, grid, dim3(256), 0, s, p, bg, h, rr, nrm, x, force_on);
     return hipGetLastError();
 }
 
