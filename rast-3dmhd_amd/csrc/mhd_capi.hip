@@ -389,7 +389,7 @@ static int rebase(mhd_t *h) {
         if (!h->bgd2) e = hipMalloc(&h->bgd2, BG_DBL * nzp * sizeof(double));
         if (e == hipSuccess && !h->bgf2) e = hipMalloc(&h->bgf2, BG_FLT * nzp * sizeof(float));
         if (e == hipSuccess && !h->bgp2) e = hipMalloc(&h->bgp2, nzp * sizeof(PlaneM));
-        if (e == hipSuccess && !h->prof) e = hipMalloc(&h->prof, 3 * (size_t)nz * sizeof(double));
+        if (e == hipSuccess && !h->prof) e = hipMalloc(&h->prof, prof_len(nz) * sizeof(double));
         if (e != hipSuccess) return fail(h, MHD_ERR_HIP, "mhd_rebase: allocation: %s", hipGetErrorString(e));
     }
     std::vector<double> prof(3 * (size_t)nz);
@@ -788,7 +788,7 @@ extern "C" int mhd_flux_profiles(mhd_t *h, double *ttm, double *rom, double *fco
     HIPCHK(h, hipSetDevice(h->dev));
     const int nz = p.npz;
     std::vector<double> prof(3 * (size_t)nz);
-    HIPCHK(h, result_buffer(h, prof.size() * sizeof(double)));
+    HIPCHK(h, result_buffer(h, prof_len(nz) * sizeof(double)));
     hipError_t e = h->mixed ? launch_flux_profiles_mixed(p, h->hq[h->cur], h->rr, h->bg, h->out, h->stream)
                             : launch_flux_profiles(p, h->q[h->cur], h->out, h->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(prof.data(), h->out, prof.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream);
