@@ -5,9 +5,13 @@
 // Here the DMA fills the slots of a pinned ring in order, and several threads
 // empty them into the caller's memory at the same time: 512x512x256 (4.3 GB)
 // comes down in 90 ms instead of 250, 64x64x48 (13.6 MB) in 0.48 ms instead of
-// 1.1.  One thread empties 28 GB/s, three 46 GB/s, seven or twelve no more;
-// below 6 MB starting them costs more than they save (4.6 MB: 245 us without,
-// 270 with).  Results up to 256 KB take one ordinary copy.
+// 1.1.  One thread empties 28 GB/s, three 46 GB/s, seven or twelve no more.
+// Starting them costs some 60 us: below 8 MiB this thread empties the ring itself,
+// and all fields that one launch wrote come down as one run, because a copy and an
+// event per field cost 20 us each (eight fields of 16x16x12, 0.3 MB: 180 us with
+// slots per field, 45 as a run; 32x32x24, 1.9 MB: 210, 107; 48x48x28, 4.8 MB: 263,
+// 209).  One array up to 1 MiB takes the runtime's own copy, which needs no second
+// copy here (0.6 MB: 58 us, 65 through the ring; 2.1 MB: 175, 152).
 //
 // Threads live for one call (they start while the first piece is on its way),
 // so nothing runs between calls.  A ring is used by one call at a time; it is
@@ -27,9 +31,10 @@ namespace rmhd {
 
 namespace {
 
-constexpr size_t SMALL = 256 << 10, RING = 32 << 20;
+constexpr size_t SMALL = 1 << 20, RING = 32 << 20;
 constexpr int SLOTS = 8, KEEP = 2, THREADS = 3;
-constexpr size_t THREADS_FROM = 6 << 20;
+constexpr size_t THREADS_FROM = 8 << 20, PIECE = 1 << 20;
+static_assert(THREADS_FROM <= RING && SLOTS >= 4, "a result without threads fits the ring");
 
 struct Ring {
     char *base = nullptr;
@@ -122,8 +127,8 @@ void drain(Job *j) {
     }
 }
 
-// One ordinary copy per contiguous run, for small results.
-hipError_t copy_small(const HostSpan *spans, int n, FillFn fill, void *ctx, hipStream_t s) {
+// One ordinary copy per contiguous run: a small array, or no pinned memory.
+hipError_t copy_plain(const HostSpan *spans, int n, FillFn fill, void *ctx, hipStream_t s) {
     std::vector<char> tmp;
     for (int i = 0; i < n;) {
         const char *src = nullptr;
@@ -150,6 +155,61 @@ hipError_t copy_small(const HostSpan *spans, int n, FillFn fill, void *ctx, hipS
     return hipSuccess;
 }
 
+// Copies n bytes at src into the spans, from byte off of span i on (both moved on).
+void scatter(const HostSpan *spans, int &i, size_t &off, const char *src, size_t n) {
+    while (n) {
+        const size_t m = std::min(n, spans[i].bytes - off);
+        memcpy(static_cast<char *>(spans[i].dst) + off, src, m);
+        src += m;
+        n -= m;
+        off += m;
+        if (off == spans[i].bytes) {
+            ++i;
+            off = 0;
+        }
+    }
+}
+
+// Results that fit the ring, without threads: each contiguous run comes down in
+// one to four pieces whatever its spans, and this thread copies a piece out
+// while the next one is on its way.
+hipError_t copy_mid(const HostSpan *spans, int n, FillFn fill, void *ctx, hipStream_t s) {
+    Ring *ring = nullptr;
+    hipError_t e = ring_get(&ring);
+    if (e != hipSuccess) {  // no pinned memory: the runtime's own copies
+        (void)hipGetLastError();
+        return copy_plain(spans, n, fill, ctx, s);
+    }
+    for (int i = 0; i < n && e == hipSuccess;) {
+        const char *src = nullptr;
+        const int m = fill(ctx, i, &src, &e);
+        if (m < 1) {
+            if (e == hipSuccess) e = hipErrorUnknown;
+            break;
+        }
+        size_t bytes = 0;
+        for (int k = 0; k < m; ++k) bytes += spans[i + k].bytes;
+        const size_t piece = std::max(PIECE, (bytes / 4 + 4095) / 4096 * 4096);
+        int np = 0;
+        for (size_t o = 0; o < bytes && e == hipSuccess; o += piece, ++np) {
+            e = hipMemcpyAsync(ring->base + o, src + o, std::min(piece, bytes - o), hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess && o + piece < bytes) e = hipEventRecord(ring->ev[np], s);
+        }
+        int at = i;
+        size_t off = 0;
+        for (int k = 0; k < np && e == hipSuccess; ++k) {
+            e = k < np - 1 ? hipEventSynchronize(ring->ev[k]) : hipStreamSynchronize(s);
+            const size_t o = (size_t)k * piece;
+            if (e == hipSuccess) scatter(spans, at, off, ring->base + o, std::min(piece, bytes - o));
+        }
+        i += m;
+    }
+    // nothing may still write into the ring when it is used again
+    if (e != hipSuccess) (void)hipStreamSynchronize(s);
+    ring_put(ring);
+    return e;
+}
+
 hipError_t copy_large(const HostSpan *spans, int n, size_t total, FillFn fill, void *ctx, hipStream_t s) {
     // slots small enough that a result makes several of them, so that the
     // copies out of the ring overlap the DMA into it
@@ -162,12 +222,14 @@ hipError_t copy_large(const HostSpan *spans, int n, size_t total, FillFn fill, v
     job.tasks = &tasks;
     job.slot_bytes = slot;
     hipError_t e = ring_get(&job.ring);
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess) {  // no pinned memory: the runtime's own copies
+        (void)hipGetLastError();
+        return copy_plain(spans, n, fill, ctx, s);
+    }
     std::vector<std::thread> th;
-    const int want = total >= THREADS_FROM ? THREADS : 0;
     try {
-        th.reserve((size_t)want);
-        for (int t = 0; t < want; ++t) th.emplace_back(drain, &job);
+        th.reserve((size_t)THREADS);
+        for (int t = 0; t < THREADS; ++t) th.emplace_back(drain, &job);
     } catch (...) {  // fewer threads: this one empties the rest
     }
     const bool alone = th.empty();
@@ -236,7 +298,8 @@ hipError_t copy_out(const HostSpan *spans, int n, FillFn fill, void *ctx, hipStr
     size_t total = 0;
     for (int i = 0; i < n; ++i) total += spans[i].bytes;
     try {
-        if (total <= SMALL) return copy_small(spans, n, fill, ctx, s);
+        if (n == 1 && total <= SMALL) return copy_plain(spans, n, fill, ctx, s);
+        if (total < THREADS_FROM) return copy_mid(spans, n, fill, ctx, s);
         return copy_large(spans, n, total, fill, ctx, s);
     } catch (...) {  // no host memory for the lists
         return hipErrorOutOfMemory;
