@@ -279,7 +279,7 @@ hipError_t launch_closure_inputs(const Params &p, const Background &bg, const fl
 // Horizontal means and mean convective flux per interior plane (mhd_diag.hip):
 // out[3][npz] = TTM, ROM, FCONM, in a buffer of prof_len(npz) doubles.
 constexpr int PROF_SEGS = 8;  // workgroups per plane
-inline size_t prof_len(int npz) { return 3 * (size_t)npz + 3 + 4 * (size_t)PROF_SEGS * npz; }
+inline size_t prof_len(int npz) { return 3 * (size_t)npz + 8 * (size_t)PROF_SEGS * npz; }
 hipError_t launch_flux_profiles(const Params &p, const double *q, double *out, hipStream_t s);
 hipError_t launch_flux_profiles_mixed(const Params &p, const float *h, const unsigned *rr, const Background &bg,
                                       double *out, hipStream_t s);

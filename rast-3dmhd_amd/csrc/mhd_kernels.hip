@@ -889,13 +889,16 @@ __global__ void k_unpack(const Params p, const double *__restrict__ q, const Fie
 // planes within factor/2 of it with trapezoid weights (1/2 at both ends);
 // the two boundary planes are taken as they are.
 //
-// A thread owns a coarse column over `depth` (BF_DEPTH) coarse planes, so that the fine
-// plane that two coarse planes share (zmode 1) is averaged once.  FACTOR 2, 4 and
+// A thread owns a coarse column over `depth` (BF_DEPTH) coarse planes; the fine
+// plane that two of them share (zmode 1) is averaged once.  FACTOR 2, 4 and
 // 8 read their rows in 16-byte pieces, all of a plane (of half a plane: 8) before
 // the first is added; 0 is any other factor.  Bound by the read of the state:
 // 8 fields of 256x256x125 by 4 in 115 us (4.6 TB/s), 156 us with a thread per
-// coarse point and 8-byte loads.
-constexpr int BF_DEPTH = 8;
+// coarse point and 8-byte loads.  More planes a thread save no time on a large box,
+// where the shared plane is found in L2, and leave a small one with too few
+// wavefronts (100x120x49 by 4 with its download: 91 us with 8 planes, 84 with 2;
+// 288x288x145: 758, 742).
+constexpr int BF_DEPTH = 2;
 template <int FACTOR>
 __global__ __launch_bounds__(256) void k_box_filter(const Params p, const double *__restrict__ q, int fct, int zmode,
                                                     int nxc, int nyc, int nzc, int depth, double *__restrict__ out) {
