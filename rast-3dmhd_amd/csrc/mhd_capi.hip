@@ -56,7 +56,7 @@ struct mhd_ctx {
     std::vector<double> dzzdz, d2zzdz2, ddz, rkapa, dkapa;  // host copies for the background
     DevScalars *sc = nullptr;
     CflSlots *cs = nullptr;             // CFL reduction slots (after sc)
-    DevScalars *report = nullptr;       // pinned: the scalars of the last step of a call (Params::report)
+    DevScalars *report = nullptr;       // pinned: the scalars of the last step of a call (Params::report); may be null
     // closure-corrected step (mixed form)
     mhd_net_t *net = nullptr;
     float *force = nullptr;    // [npz * plane][8]
@@ -225,7 +225,11 @@ extern "C" int mhd_create(const mhd_desc *d, mhd_t **out) {
         h->cs = reinterpret_cast<CflSlots *>(reinterpret_cast<char *>(h->sc) + 256);
         h->met = reinterpret_cast<double *>(h->cs + 1);
     }
-    if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void **>(&h->report), sizeof(DevScalars), hipHostMallocCoherent);
+    if (e == hipSuccess &&
+        hipHostMalloc(reinterpret_cast<void **>(&h->report), sizeof(DevScalars), hipHostMallocCoherent) != hipSuccess) {
+        (void)hipGetLastError();
+        h->report = nullptr;  // no pinned memory: the scalars are copied (finish)
+    }
     if (e != hipSuccess) {
         rc = fail(nullptr, MHD_ERR_HIP, "mhd_create: device allocation failed: %s", hipGetErrorString(e));
         free_all(h);
@@ -536,9 +540,10 @@ static hipError_t launches(mhd_t *h, hipEvent_t *ev, bool report = false) {
     return e;
 }
 
-// reported: the last step wrote its scalars to h->report.
+// reported: the last step wrote its scalars to h->report, if there is one.
 static int finish(mhd_t *h, double *dt, double *umach, bool reported) {
     DevScalars s;
+    reported = reported && h->report;
     if (!reported) HIPCHK(h, hipMemcpyAsync(&s, h->sc, sizeof(s), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     if (reported) s = *h->report;
