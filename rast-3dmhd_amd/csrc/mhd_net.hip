@@ -809,8 +809,11 @@ static hipError_t conv(hipStream_t s, const bf16 *x, const bf16 *w, int kp, cons
     return hipGetLastError();
 }
 
+// Buffers for a volume of nvox voxels.  Whoever uses them calls this first: an
+// allocation that failed leaves none (cap 0), also for volumes that fitted.
 static int ensure_workspace(mhd_net_t *n, long long nvox) {
     if (nvox <= n->cap) return MHD_OK;
+    n->cap = 0;
     void **bufs[11] = {(void **)&n->a0, (void **)&n->a1, (void **)&n->a2, (void **)&n->g1, (void **)&n->g2,
                        (void **)&n->g3, (void **)&n->z1, (void **)&n->z2, (void **)&n->y, (void **)&n->tmp32,
                        (void **)&n->dx32};
@@ -1123,6 +1126,8 @@ extern "C" int mhd_net_clear_samples(mhd_net_t *n) {
 static int sample_step(mhd_net_t *n, int s, bool train, float lr, double *loss) {
     const Sample &S = n->samples[s];
     const long long nvox = (long long)S.nx * S.ny * S.nz;
+    const int rc = ensure_workspace(n, nvox);
+    if (rc) return rc;
     NHIP(n, forward_on(n, n->stream, S.x, S.nx, S.ny, S.nz, train));
     const int nb = (int)std::min<long long>(1024, (nvox * 8 + 255) / 256);
     const float gscale = (float)(2.0 / ((double)nvox * n->cout));
@@ -1232,6 +1237,7 @@ int net_prepare(mhd_net_t *n, long long nvox, int *dev) {
 // cleared if a value is not finite.
 hipError_t net_force(mhd_net_t *n, hipStream_t s, int nx, int ny, int nz, const __bf16 *x, const float *nrm,
                      float *force, int *force_on) {
+    if (ensure_workspace(n, (long long)nx * ny * nz) != MHD_OK) return hipErrorOutOfMemory;
     return forward_on(n, s, x, nx, ny, nz, false, nrm, force, force_on);
 }
 
