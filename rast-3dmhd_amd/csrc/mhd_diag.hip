@@ -135,9 +135,12 @@ __global__ __launch_bounds__(64) void k_flux_profiles(const Params p, const Sums
     out[p.npz + k - 1] = a.r.value() / cnt;
     // RW (T - TTM) = RW (T - T0) - RW (TTM - T0), with what the division rounded off TTM
     const double d = 2.5 * ((ttm - t0) + (fma(-ttm, cnt, a.t.s) + a.t.c) / cnt), w = a.w.value();
-    const double x = d * w;
-    a.f.add(x);
-    a.f.c += fma(d, w, -x);
+    // (RW infinite: the flux about any T is; the correction would make it a NaN)
+    if (isfinite(w) || !isfinite(d)) {
+        const double x = d * w;
+        a.f.add(x);
+        a.f.c += fma(d, w, -x);
+    }
     out[2 * p.npz + k - 1] = a.f.value() / cnt;
 }
 
