@@ -127,7 +127,8 @@ void drain(Job *j) {
     }
 }
 
-// One ordinary copy per contiguous run: a small array, or no pinned memory.
+// One ordinary copy per contiguous run: a small array, spans that overlap, or no
+// pinned memory.
 hipError_t copy_plain(const HostSpan *spans, int n, FillFn fill, void *ctx, hipStream_t s) {
     std::vector<char> tmp;
     for (int i = 0; i < n;) {
@@ -208,6 +209,17 @@ hipError_t copy_mid(const HostSpan *spans, int n, FillFn fill, void *ctx, hipStr
     if (e != hipSuccess) (void)hipStreamSynchronize(s);
     ring_put(ring);
     return e;
+}
+
+// Whether two spans share memory (the same array passed twice): they are then
+// copied one after the other, and the later one's bytes stay.
+bool spans_overlap(const HostSpan *spans, int n) {
+    for (int i = 0; i < n; ++i)
+        for (int k = 0; k < i; ++k) {
+            const char *const a = static_cast<const char *>(spans[i].dst), *const b = static_cast<const char *>(spans[k].dst);
+            if (a < b + spans[k].bytes && b < a + spans[i].bytes) return true;
+        }
+    return false;
 }
 
 hipError_t copy_large(const HostSpan *spans, int n, size_t total, FillFn fill, void *ctx, hipStream_t s) {
@@ -300,6 +312,7 @@ hipError_t copy_out(const HostSpan *spans, int n, FillFn fill, void *ctx, hipStr
     try {
         if (n == 1 && total <= SMALL) return copy_plain(spans, n, fill, ctx, s);
         if (total < THREADS_FROM) return copy_mid(spans, n, fill, ctx, s);
+        if (spans_overlap(spans, n)) return copy_plain(spans, n, fill, ctx, s);
         return copy_large(spans, n, total, fill, ctx, s);
     } catch (...) {  // no host memory for the lists
         return hipErrorOutOfMemory;

@@ -1,0 +1,11 @@
+"""Copies of results into the caller's memory, on the CPU (host memory in the
+place of the GPU): the paths that only a failure or odd arguments reach."""
+
+import pytest
+
+import hostbuild
+
+
+@pytest.mark.parametrize("what", ["same_array"])
+def test_copies(what):
+    hostbuild.run("download_copies", what)
