@@ -11,7 +11,8 @@
 // event per field cost 20 us each (eight fields of 16x16x12, 0.3 MB: 180 us with
 // slots per field, 45 as a run; 32x32x24, 1.9 MB: 210, 107; 48x48x28, 4.8 MB: 263,
 // 209).  One array up to 1 MiB takes the runtime's own copy, which needs no second
-// copy here (0.6 MB: 58 us, 65 through the ring; 2.1 MB: 175, 152).
+// copy here (0.6 MB: 58 us, 65 through the ring; 2.1 MB: 175, 152).  Arrays that
+// the caller pinned need no ring (copy_direct).
 //
 // Threads live for one call (they start while the first piece is on its way),
 // so nothing runs between calls.  A ring is used by one call at a time; it is
@@ -33,7 +34,7 @@ namespace {
 
 constexpr size_t SMALL = 1 << 20, RING = 32 << 20;
 constexpr int SLOTS = 8, KEEP = 2, THREADS = 3;
-constexpr size_t THREADS_FROM = 8 << 20, PIECE = 1 << 20;
+constexpr size_t THREADS_FROM = 8 << 20, PIECE = 1 << 20, DIRECT_FROM = 384 << 10;
 static_assert(THREADS_FROM <= RING && SLOTS >= 4, "a result without threads fits the ring");
 
 struct Ring {
@@ -211,6 +212,42 @@ hipError_t copy_mid(const HostSpan *spans, int n, FillFn fill, void *ctx, hipStr
     return e;
 }
 
+// Whether the runtime copies into the spans itself: where the CPU may not write
+// (device memory), and where the caller pinned all of them and they are not short.
+bool spans_direct(const HostSpan *spans, int n, size_t total) {
+    bool known = true;
+    for (int i = 0; i < n; ++i) {
+        hipPointerAttribute_t a;
+        if (hipPointerGetAttributes(&a, spans[i].dst) != hipSuccess) {
+            (void)hipGetLastError();
+            a.type = hipMemoryTypeUnregistered;
+        }
+        if (a.type == hipMemoryTypeDevice) return true;
+        known = known && a.type != hipMemoryTypeUnregistered;
+    }
+    return known && total >= n * DIRECT_FROM;
+}
+
+// Straight into the spans, one wait at the end: the link's rate, without a copy
+// by the CPU (eight pinned fields, us through the ring and so: 4.8 MB 215, 179;
+// 13.9 MB 489, 336; 141 MB 3357, 2674; one of 1.7 MB 101, 53).  Each copy costs
+// 10 us, so that short ones are faster as a run through the ring (eight of 0.1
+// MB: 54, 98; of 0.24 MB: 95, 123; the lines cross at 0.4 MB).
+hipError_t copy_direct(const HostSpan *spans, int n, FillFn fill, void *ctx, hipStream_t s) {
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < n && e == hipSuccess;) {
+        const char *src = nullptr;
+        int m = fill(ctx, i, &src, &e);
+        if (m < 1 && e == hipSuccess) e = hipErrorUnknown;
+        for (; m > 0 && e == hipSuccess; --m, ++i) {
+            e = hipMemcpyAsync(spans[i].dst, src, spans[i].bytes, hipMemcpyDeviceToHost, s);
+            src += spans[i].bytes;
+        }
+    }
+    const hipError_t e2 = hipStreamSynchronize(s);
+    return e != hipSuccess ? e : e2;
+}
+
 // Whether two spans share memory (the same array passed twice): they are then
 // copied one after the other, and the later one's bytes stay.
 bool spans_overlap(const HostSpan *spans, int n) {
@@ -311,6 +348,7 @@ hipError_t copy_out(const HostSpan *spans, int n, FillFn fill, void *ctx, hipStr
     for (int i = 0; i < n; ++i) total += spans[i].bytes;
     try {
         if (n == 1 && total <= SMALL) return copy_plain(spans, n, fill, ctx, s);
+        if (spans_direct(spans, n, total)) return copy_direct(spans, n, fill, ctx, s);
         if (total < THREADS_FROM) return copy_mid(spans, n, fill, ctx, s);
         if (spans_overlap(spans, n)) return copy_plain(spans, n, fill, ctx, s);
         return copy_large(spans, n, total, fill, ctx, s);

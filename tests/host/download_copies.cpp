@@ -56,11 +56,53 @@ static int same_array() {
     return 0;
 }
 
+// Spans in pinned memory of 384 KiB and more on average are copied to directly,
+// without the ring, shorter ones in a run; a pageable one among them is served too.
+static int pinned() {
+    for (const std::vector<size_t> &sizes : {std::vector<size_t>{3 << 20, 100, 9 << 20}, {2 << 20}, {384 << 10, 384 << 10}, {384 << 10, (384 << 10) - 1}}) {
+        for (const size_t room : {(size_t)4 << 20, (size_t)64 << 20})
+            for (int pageable = 0; pageable < 2; ++pageable) {
+                std::vector<HostSpan> spans;
+                std::vector<char> own(sizes.back());
+                for (size_t n : sizes) {
+                    void *p = nullptr;
+                    (void)hipHostMalloc(&p, n, 0);
+                    spans.push_back({p, n});
+                }
+                void *const last = spans.back().dst;
+                size_t total = 0;
+                for (size_t n : sizes) total += n;
+                const bool direct = !pageable && total >= sizes.size() * (384 << 10);
+                if (pageable) spans.back().dst = own.data();
+                hh::copies.clear();
+                HH_CHECK(copy_all(spans, room) == hipSuccess);
+                for (size_t i = 0; i < spans.size(); ++i) {
+                    for (size_t b = 0; b < spans[i].bytes; ++b)
+                        HH_CHECK(static_cast<char *>(spans[i].dst)[b] == Source::value((int)i, b));
+                    HH_CHECK(direct == (hh::copies[0].dst == spans[0].dst));
+                    if (direct) HH_CHECK(hh::copies.size() == spans.size() && hh::copies[i].dst == spans[i].dst);
+                }
+                spans.back().dst = last;
+                for (const HostSpan &s : spans) (void)hipHostFree(s.dst);
+            }
+    }
+    // memory the CPU may not write, however short
+    void *dev = nullptr;
+    (void)hipMalloc(&dev, 6000);
+    std::vector<char> own(4000);
+    const std::vector<HostSpan> spans = {{own.data(), own.size()}, {dev, 6000}};
+    hh::copies.clear();
+    HH_CHECK(copy_all(spans, 1 << 20) == hipSuccess && hh::copies.size() == 2 && hh::copies[1].dst == dev);
+    (void)hipFree(dev);
+    return 0;
+}
+
 int main(int argc, char **argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     copy_retain();
     int rc = 1;
     if (what == "same_array") rc = same_array();
+    else if (what == "pinned") rc = pinned();
     else printf("unknown check\n");
     copy_release();
     HH_CHECK(hh::ranges.empty());

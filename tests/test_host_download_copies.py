@@ -6,6 +6,6 @@ import pytest
 import hostbuild
 
 
-@pytest.mark.parametrize("what", ["same_array"])
+@pytest.mark.parametrize("what", ["same_array", "pinned"])
 def test_copies(what):
     hostbuild.run("download_copies", what)
