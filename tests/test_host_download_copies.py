@@ -6,6 +6,6 @@ import pytest
 import hostbuild
 
 
-@pytest.mark.parametrize("what", ["same_array", "pinned"])
+@pytest.mark.parametrize("what", ["sizes", "no_pinned_memory", "no_threads", "one_thread", "same_array", "pinned"])
 def test_copies(what):
     hostbuild.run("download_copies", what)
