@@ -15,8 +15,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "--offload-host-only", "-fuse-cuid=none", "-O1", "-std=c++17", "-fPIC", "-pthread"]
 
 
-def _run(cmd):
-    r = subprocess.run(cmd, capture_output=True, text=True, timeout=300)
+def _run(cmd, stdin=None):
+    r = subprocess.run(cmd, input=stdin, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, " ".join(cmd) + "\n" + r.stdout + r.stderr
     return r.stdout
 
@@ -42,6 +42,6 @@ def _program(name):
     return exe
 
 
-def run(name, *args):
+def run(name, *args, stdin=None):
     """Builds tests/host/<name>.cpp and runs it; its output, or the test fails with it."""
-    return _run([_program(name), *args])
+    return _run([_program(name), *args], stdin)
