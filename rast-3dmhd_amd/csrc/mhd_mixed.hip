@@ -710,8 +710,11 @@ __global__ __launch_bounds__(MTile<TY>::NT, 3) void k_stage_m(const BoxArgs b,
 
 // Ensemble: persistent grid over the work items of all boxes (static stride);
 // each item carries its tile's shape.
+// Stage 1 of 64x8 tiles, 512 threads: at most 128 registers a lane, so that two
+// workgroups fit a CU (a step of 8 boxes of 128x128x64 with 8 planes a chunk: 912
+// us with 129 registers, 881 so; 16 of 64x64x64: 439, 418).
 template <int TY, bool MAG, int MODE>
-__global__ __launch_bounds__(MTile<TY>::NT, 3) void k_stage_m_batch(const BoxDev *__restrict__ boxes,
+__global__ __launch_bounds__(MTile<TY>::NT, TY == 8 && MODE == 1 ? 4 : 3) void k_stage_m_batch(const BoxDev *__restrict__ boxes,
                                                            const StageItem *__restrict__ items, int nitems, int a) {
     extern __shared__ float ldsf[];
     const int slot = xcd_remap(blockIdx.x, gridDim.x);
