@@ -57,15 +57,18 @@ int mhd_ens_set_fixed_dt(mhd_ens_t *e, int box, double dt);
 int mhd_ens_steps(mhd_ens_t *e, int n, int use_graph, double *dt, double *umach);
 
 /* Tiling of the batched launches: tile_y (4: tiles of up to 256 points, 64x4 or
- * of a shape fitted to each box's width; 8: 64x8), kdepth (planes per z chunk; 0 = whole column) and grid (persistent
- * workgroups; 0 = one workgroup per work item).  get_tiling reports the
- * rows of the current tile whatever its width. */
+ * of a shape fitted to each box's width; 8: 64x8), kdepth (planes per z chunk,
+ * at least three in the first and the last; 0 = whole column) and grid
+ * (persistent workgroups; 0 = one workgroup per work item).  get_tiling reports the tiling as it was set or tuned, rows whatever the
+ * width: 4 also where boxes have fitted tiles of other shapes. */
 int mhd_ens_set_tiling(mhd_ens_t *e, int tile_y, int kdepth, int grid);
 int mhd_ens_get_tiling(const mhd_ens_t *e, int *tile_y, int *kdepth, int *grid);
 
 /* The same with the tile width: tile_x x tile_y is 64x4, 64x8, or (mixed
  * form only) 32x8; 64x4 is fitted to each box (see mhd_ens_set_tiling), 32x8
- * is that shape for all.  The results do not depend on the tiling. */
+ * is that shape for all.  get_tile reports what was set or tuned, so that a
+ * tiling can be set again: 64x4 stands for the fitted shapes too.  The results do
+ * not depend on the tiling. */
 int mhd_ens_set_tile(mhd_ens_t *e, int tile_x, int tile_y, int kdepth, int grid);
 int mhd_ens_get_tile(const mhd_ens_t *e, int *tile_x, int *tile_y, int *kdepth, int *grid);
 
@@ -73,9 +76,9 @@ int mhd_ens_get_tile(const mhd_ens_t *e, int *tile_x, int *tile_y, int *kdepth, 
  * launches), keeps the fastest, and restores the state and clocks of every
  * box to what they were before the call.  report (may be NULL) receives a
  * JSON list of {tile_x, tile_y, kdepth, grid, ms_step} for the candidates
- * (tile shapes as in mhd_ens_set_tile; 7 chunk depths x 4 grids per shape,
- * about 80 bytes each: 8 KiB holds the list, a shorter report_len cuts it
- * at report_len - 1 bytes). */
+ * (tile shapes as in mhd_ens_set_tile, 64x4 fitted to each box; 7 chunk
+ * depths x 4 grids per shape, about 80 bytes each: 8 KiB holds the list, a
+ * shorter report_len cuts it at report_len - 1 bytes). */
 int mhd_ens_autotune(mhd_ens_t *e, int nsteps, char *report, int report_len);
 
 /* Mean milliseconds per ensemble step over n steps (HIP events on the

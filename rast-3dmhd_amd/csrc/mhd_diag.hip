@@ -83,8 +83,8 @@ struct StateMixed {
     }
 };
 
-// part[k-1][segment] = sums of T, RO, RW and of the flux about T0 over the points of segment blockIdx.y of plane k = blockIdx.x + 1.
-// T0 goes to out's place of FCONM.
+// part[k-1][segment] = sums of T, RO, RW and of the flux about T0 over the points
+// of segment blockIdx.y of plane k = blockIdx.x + 1.  T0 goes to out's place of FCONM.
 template <class S>
 __global__ __launch_bounds__(PROF_THREADS) void k_flux_sums(const Params p, const S st, Sums *__restrict__ part,
                                                             double *__restrict__ out) {

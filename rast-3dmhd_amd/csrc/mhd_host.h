@@ -79,8 +79,8 @@ inline int check_desc(const mhd_desc *d, char *msg, size_t len) {
 // time of a plane, which grows with the workgroups that share the CU (FP64:
 // 3.3 us alone, 5.7 us with two; mixed: 2.6, 3.5, 4.4 us).  The count with
 // the least sum wins: small boxes split until the chip is about full (64x64x32
-// FP64: 11 chunks of up to 3 planes, a stage of 18 us against 38 with 4 chunks on 64
-// of 256 CUs), larger ones take whole rounds (256x256x128 mixed: 6 chunks, two
+// FP64: 11 chunks of up to 3 planes, stages of 16, 17 and 22 us against 38 with 4
+// chunks on 64 of 256 CUs), larger ones take whole rounds (256x256x128 mixed: 6 chunks, two
 // full rounds, 230 us against 254 with 16 chunks of 5.3 rounds).  Chunks are
 // at most 32 planes: over a longer march the tiles that share halo rows drift
 // apart and re-read them from HBM (512x512x256 FP64, 128 planes: 14% more

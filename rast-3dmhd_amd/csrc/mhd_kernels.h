@@ -176,7 +176,8 @@ struct StageItem {
 // chunk_depth(npz, nc) of them.  The first and the last chunk hold a boundary
 // plane and apply the boundary conditions there, which read the two planes
 // next to it, so they have at least three planes (as many as the deepest); the
-// others share the rest evenly, down to one plane each.
+// others share the rest evenly, down to one plane each (an ensemble's table asks
+// for that; z_chunks mostly stops at three, the depth of the two).
 __host__ __device__ inline int max_chunks(int npz) { return npz < 6 ? 1 : npz - 4; }
 __host__ __device__ inline int chunk_depth(int npz, int nc) {
     const int d = (npz + nc - 1) / nc;

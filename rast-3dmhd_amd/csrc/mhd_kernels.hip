@@ -18,10 +18,10 @@
 // no x/y ghost cells: neighbours wrap periodically.
 //
 // Stage kernel organisation.  A workgroup owns a 64 x TY column tile, or one of
-// up to 256 points fitted to the box (TY = 0, see fit_tile), and marches down a chunk of planes.  LDS holds the raw fields of planes k and
-// k+1 with a one-point halo (double buffer) and a three-plane ring of the
-// velocities u,v,w (needed at (i+-1,k+-1) and (j+-1,k+-1) by the cross terms
-// of the viscous stress).  Plane k+2 is loaded into registers while plane k
+// up to 256 points fitted to the box (TY = 0, see fit_tile), and marches down a
+// chunk of planes.  LDS holds the raw fields of planes k and k+1 with a one-point
+// halo (double buffer) and a three-plane ring of the velocities u,v,w (needed at
+// (i+-1,k+-1) and (j+-1,k+-1) by the cross terms of the viscous stress).  Plane k+2 is loaded into registers while plane k
 // is computed, and the Z register of the RK3 scheme is prefetched the same
 // way, so each global load has a whole plane of arithmetic to hide behind.
 // Outputs are written with non-temporal stores so that L2 keeps the halo
@@ -30,7 +30,7 @@
 // small boxes the latency of a plane's march (3.3 us with one workgroup on a
 // CU) and of the launch, hence few planes per chunk (z_chunks) and three
 // launches per step (64x64x32: 56 us per step, 132 with boundary, CFL and
-// 8-plane launches of their own; 16x16x12 by single steps: 73 against 210).
+// 8-plane launches of their own; 16x16x12 by single steps: 67 against 207).
 //
 // Arithmetic: every expression keeps the reference's left-to-right
 // association and the file is compiled with -ffp-contract=off, so results
@@ -244,7 +244,8 @@ constexpr int stage_lds_bytes() {
 // diffusion, Rempel conduction, shear boundaries, flux relaxation and embedded
 // heat loss; the main path has none of their code.  Form 2 spills 60-90
 // registers of each lane, form 1 none (96x96x48 with density diffusion, stages
-// 1 to 3: 53, 81, 85 us as form 2, 35, 40, 44 us as form 1).
+// 1 to 3 in 64x4 tiles: 53, 81, 85 us as form 2, 35, 40, 44 us as form 1; 32, 35,
+// 41 us in the fitted 48x5).
 template <int TY, bool MAG, int MODE, int OPT = 0>
 __device__ __forceinline__ void stage_tile(const Params &p, const Metrics &m, ArgPtr args,
                                            const double *__restrict__ qin,

@@ -64,7 +64,7 @@ struct MTile<0> {
 // Lean: T' takes the place of rho', of which only a point's own value is read (it
 // stays in registers, as does T' of plane k-1), 25 instead of 28 values a point.
 // Stage 1, whose registers allow it, so has four workgroups of 64x4 on a CU
-// (512x512x256: 1654 -> 1581 us); the others keep three either way, and stage 3
+// (512x512x256: 1634 -> 1573 us); the others keep three either way, and stage 3
 // is 1% slower lean (256x256x128).
 template <int MODE>
 constexpr bool lean_lds = MODE == 1;
