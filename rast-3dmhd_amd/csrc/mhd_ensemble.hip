@@ -655,8 +655,9 @@ extern "C" int mhd_ens_autotune(mhd_ens_t *e, int nsteps, char *report, int repo
                 r = copy_state(false);
                 e->cur = cur0;
                 char line[160];
+                // (every digit of the time: the least in the report is the one kept)
                 snprintf(line, sizeof line,
-                         "%s{\"tile_x\": %d, \"tile_y\": %d, \"kdepth\": %d, \"grid\": %d, \"ms_step\": %.5f}",
+                         "%s{\"tile_x\": %d, \"tile_y\": %d, \"kdepth\": %d, \"grid\": %d, \"ms_step\": %.9g}",
                          rep.size() > 1 ? ", " : "", txs[a], tys[a], kds[k], grid, ms);
                 rep += line;
                 if (ms < best) {

@@ -24,6 +24,7 @@ inline bool no_pinned = false;            // hipHostMalloc fails
 inline long malloc_until = -1;            // hipMalloc fails once this many have succeeded (-1: never)
 inline std::function<void(const char *, void **)> on_launch;
 inline std::function<void(hipEvent_t)> on_event_wait;
+inline std::function<float()> elapsed_ms; // between any two events
 // what it reads
 struct Copy {
     const void *dst, *src;
@@ -201,7 +202,7 @@ hipError_t hipEventSynchronize(hipEvent_t e) {
     return hipSuccess;
 }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
-    *ms = 1.0f;
+    *ms = hh::elapsed_ms ? hh::elapsed_ms() : 1.0f;
     return hipSuccess;
 }
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorInvalidValue; }
