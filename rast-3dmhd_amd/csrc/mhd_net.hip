@@ -492,8 +492,12 @@ __global__ __launch_bounds__(768, 3) void k_dw(const bf16 *__restrict__ x, int c
         if (t < gtasks) {
             const int c8 = t % ng, pr = t / ng % 32, r = t / (32 * ng);
             bf16 *const row = tg + (buf * 2 + r) * 3 * CO * DS;
+            // (zero where X is past the row's end: 0 times an infinite G is a NaN)
+            const uint4 none = make_uint4(0, 0, 0, 0);
+            const bool in0 = sx0 + 2 * pr < nx, in1 = sx0 + 2 * pr + 1 < nx;
 #pragma unroll
-            for (int dx = 0; dx < 3; ++dx) put_pair(row + dx * CO * DS, c8, pr, q.v[2 - dx], q.v[3 - dx]);
+            for (int dx = 0; dx < 3; ++dx)
+                put_pair(row + dx * CO * DS, c8, pr, in0 ? q.v[2 - dx] : none, in1 ? q.v[3 - dx] : none);
             if (row0 + r < ny) {
 #pragma unroll
                 for (int n = 0; n < 2; ++n)
