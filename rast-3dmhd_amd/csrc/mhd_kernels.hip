@@ -102,14 +102,16 @@ __device__ __forceinline__ void cfl_point(const Params &p, const double *q, doub
 
 // Workgroup reduction of the CFL accumulators, published as order-preserving
 // keys (min/max are exact, so the order is irrelevant); workgroup seq of
-// total.  NaN keys sort above +Inf: they win the max and, through the key of
-// -NaN (below -Inf), the min, so a non-finite state cannot go unnoticed.
+// total.  The key of +NaN sorts above +Inf and wins the max, that of -NaN sorts
+// below -Inf and wins the min, so a non-finite state cannot go unnoticed.
 __device__ void cfl_reduce(double mach, double w1, double w2, double w3, double w4, double sf, int lmag,
                            int clock, DevScalars *__restrict__ sc, CflSlots *__restrict__ cs, int seq, int total,
                            DevScalars *report = nullptr) {
     __shared__ unsigned long long red[16][5];
     unsigned long long km = dkey(mach), k1 = dkey(w1), k2 = dkey(w2), k3 = dkey(w3), k4 = dkey(w4);
-    // a NaN limit becomes -NaN for the min reduction
+    // a NaN, of either sign, wins: the Mach number's as +NaN of the max, a limit's
+    // as -NaN of the min reduction
+    if (!(mach == mach)) km = ~0ull;
     if (!(w1 == w1)) k1 = 0;
     if (!(w2 == w2)) k2 = 0;
     if (!(w3 == w3)) k3 = 0;

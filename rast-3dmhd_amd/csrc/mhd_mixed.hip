@@ -153,8 +153,8 @@ __device__ void cflf_reduce(const Params &p, CflFast c, int clock, DevScalars *_
         c.d2 = nmin(c.d2, d2extra);
         const double w[4] = {1.0 / sqrt(c.q1), 0.5 * p.repr * p.cv * c.s2, 0.375 * p.re * c.s3, 0.5 * p.rm * c.d2};
         unsigned long long k[CFL_KEYS];
-        k[0] = ~dkey(c.mach);
-        // a NaN limit becomes -NaN for the min reduction
+        // a NaN, of either sign, wins: as in cfl_reduce
+        k[0] = c.mach == c.mach ? ~dkey(c.mach) : 0ull;
         for (int n = 0; n < 4; ++n) k[n + 1] = (w[n] == w[n]) ? dkey(w[n]) : 0ull;
         cfl_publish(k, sc, cs, p.sf, p.lmag, clock, seq, total, clock ? p.report : nullptr);
     }
